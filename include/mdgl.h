@@ -58,6 +58,12 @@ extern "C" {
  * block of neighbouring rows stays in cache. Results are the same bit for
  * bit; only the lane layout changes. */
 #define MDGL_NARROW_SLABS 32
+/* mdgl_gspmm: lanes of 16 bytes at any alignment and width. A row's columns
+ * are cut into runs over which each operand is consecutive or one value, and
+ * each run's last lane ends with the run (sharing columns with the lane
+ * before it), so odd widths and heads load and store whole vectors. Results
+ * are the same bit for bit; only the lane layout changes. */
+#define MDGL_ANY_ALIGNMENT 64
 /* mdgl_segment_reduce(_arg): the caller knows that no segment has more than
  * MDGL_SEGMENT_SPLIT_ROWS rows, so the pass that splits longer segments is
  * not launched (a longer segment is then still reduced whole, in row order) */
@@ -186,6 +192,13 @@ int mdgl_gspmm_rows(const int32_t* indptr, const int32_t* indices, const int32_t
 int mdgl_gspmm_lanes(int op, int64_t dl, int64_t dr, int64_t dout, int nd,
                      const int64_t* lhs_shape, const int64_t* rhs_shape, const void* lhs,
                      const void* rhs, int flags, int dtype, int64_t* vec, int64_t* group);
+
+/* The same query with, through `lanes` (optional), the lanes a row takes:
+ * it is cut into ceil(lanes / group) column slabs, whatever the flags. */
+int mdgl_gspmm_layout(int op, int64_t dl, int64_t dr, int64_t dout, int nd,
+                      const int64_t* lhs_shape, const int64_t* rhs_shape, const void* lhs,
+                      const void* rhs, int flags, int dtype, int64_t* vec, int64_t* group,
+                      int64_t* lanes);
 
 /* Locality of a graph for mdgl_gspmm's MDGL_NARROW_SLABS: partial[b]
  * (device int64, MDGL_COO_LOCALITY_BLOCKS of them) receives workgroup b's
@@ -486,6 +499,18 @@ int mdgl_gspmm_mul_sum_dot(const int32_t* indptr, const int32_t* indices, const 
                            int64_t num_chunks, int32_t chunk_len, const int32_t* heavy_rows,
                            const int32_t* heavy_ptr, int64_t num_heavy, void* workspace,
                            int64_t workspace_bytes, int dtype, void* stream);
+
+/* The same with mdgl_gspmm's `flags`: MDGL_ANY_ALIGNMENT takes runs of any
+ * dout / dr of at least 16 bytes (and at most 64 16-byte lanes, rounded up to
+ * a power of two) at any alignment, instead of whole aligned 16-byte lanes. */
+int mdgl_gspmm_mul_sum_dot_any(const int32_t* indptr, const int32_t* indices, const int32_t* eid,
+                           const void* lhs, const void* rhs, const void* rowop, void* dst,
+                           void* dot, int64_t num_dst, int64_t dl, int64_t dr, int64_t dout,
+                           int nd, const int64_t* lhs_shape, const int64_t* rhs_shape,
+                           const int32_t* chunk_row, const int32_t* chunk_start,
+                           int64_t num_chunks, int32_t chunk_len, const int32_t* heavy_rows,
+                           const int32_t* heavy_ptr, int64_t num_heavy, void* workspace,
+                           int64_t workspace_bytes, int flags, int dtype, void* stream);
 
 /* dst[r, k] = src[r, k] / max(indptr[r+1] - indptr[r], 1): the mean's divisor on a
  * node-shaped gradient. */

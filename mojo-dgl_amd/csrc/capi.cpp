@@ -499,26 +499,45 @@ int64_t mdgl_gspmm_workspace_bytes(int64_t num_chunks, int64_t dout, int reduce_
 
 namespace {
 
-// Lane width and operand load modes of a gspmm (p.bc and p.lstride set):
-// 16-byte lanes when the width allows (or the node rows are padded to
-// lines, so the last lane may read a whole vector of them), else 8-byte
-// lanes for even float32 widths, else one element per lane; a lane whose
-// columns straddle broadcast groups (heads of 2, 3, 6 columns ...) would
-// gather element by element through the any-layout kernel, so narrower
-// lanes keep compile-time layouts (per-element offsets at one element per
-// lane: on a 60M-edge graph, 48 columns as 8 heads of 6 with one weight per
-// head, 12.0 -> 3.8 ms; 12 columns as 4 heads of 3, 7.4 -> 2.7 ms).
+// Lane width, columns per run and operand load modes of a gspmm (p.bc and
+// p.lstride set). With MDGL_ANY_ALIGNMENT a row is cut into runs of L columns
+// (the innermost axis after collapsing the broadcast: each operand is
+// consecutive or one value over it), each covered by lanes of 16 bytes (8 for
+// float32 runs of 2 or 3 columns) whose last one ends with the run, at any
+// alignment (47 columns as 12 lanes of 16 bytes instead of 47 of 4; 8 heads of
+// 25 as 56 lanes in one slab instead of 200 in four).
+// Without it: 16-byte lanes when the width allows (or the node rows are padded
+// to lines), else 8-byte lanes for even float32 widths, else one element per
+// lane; a lane whose columns straddle broadcast groups (heads of 2, 3, 6
+// columns ...) would gather element by element through the any-layout kernel,
+// so narrower lanes keep compile-time layouts.
 void choose_gspmm_lanes(GspmmParams& p, int op, int64_t dl, int64_t dr, int64_t dout,
-                        const void* lhs, const void* rhs, int64_t es, int dtype, bool dot) {
+                        const void* lhs, const void* rhs, int64_t es, int dtype, int flags) {
   const int vw = vec_width(dtype);
+  if (flags & MDGL_ANY_ALIGNMENT) {
+    const int64_t L = p.bc.shape[p.bc.nd - 1];
+    const bool lc = op == OP_COPY_RHS || p.bc.lstride[p.bc.nd - 1] == 1;
+    const bool rc = op == OP_COPY_LHS || p.bc.rstride[p.bc.nd - 1] == 1;
+    p.run_len = L;
+    p.vec = L >= vw ? vw : (L >= 2 && dtype == MDGL_FLOAT32 ? 2 : 1);
+    // float64 rows of more than one slab and at most two: 32-byte lanes, so
+    // the row's edges are walked once instead of twice
+    const int64_t runs = L > 0 ? dout / L : 0;
+    if (dtype == MDGL_FLOAT64 && L >= 2 * vw && runs * ((L + vw - 1) / vw) > WAVE &&
+        runs * ((L + 2 * vw - 1) / (2 * vw)) <= WAVE)
+      p.vec = 2 * vw;
+    p.lpg = (int)((L + p.vec - 1) / p.vec);
+    p.lmode = p.vec == 1 || lc ? M_CONTIG : M_SPLAT;
+    p.rmode = p.vec == 1 || rc ? M_CONTIG : M_SPLAT;
+    return;
+  }
   const bool lined = p.lstride != dl;  // node rows on 128-byte lines
-  p.vec = (dout % vw == 0 || (lined && !dot)) ? vw
-          : (dtype == MDGL_FLOAT32 && dout % 2 == 0 ? 2 : 1);
+  p.vec = (dout % vw == 0 || lined) ? vw : (dtype == MDGL_FLOAT32 && dout % 2 == 0 ? 2 : 1);
   p.lmode = op == OP_COPY_RHS ? M_CONTIG : pick_mode(p.bc, true, dout, p.vec, dl, lhs, es, lined);
   p.rmode = op == OP_COPY_LHS ? M_CONTIG : pick_mode(p.bc, false, dout, p.vec, dr, rhs, es);
   // float64 rows of 129-256 columns: 32-byte lanes (two 16-byte loads each)
   // make one 64-lane slab, so the row's edges are walked once instead of twice
-  if (dtype == MDGL_FLOAT64 && !dot && p.vec == vw && dout > WAVE * vw && dout <= 2 * WAVE * vw &&
+  if (dtype == MDGL_FLOAT64 && p.vec == vw && dout > WAVE * vw && dout <= 2 * WAVE * vw &&
       dout % (2 * vw) == 0 && p.lmode != M_GATHER && p.rmode != M_GATHER) {
     const int lm = op == OP_COPY_RHS ? M_CONTIG : pick_mode(p.bc, true, dout, 2 * vw, dl, lhs, es, lined);
     const int rm = op == OP_COPY_LHS ? M_CONTIG : pick_mode(p.bc, false, dout, 2 * vw, dr, rhs, es);
@@ -528,7 +547,7 @@ void choose_gspmm_lanes(GspmmParams& p, int op, int64_t dl, int64_t dr, int64_t 
       p.rmode = rm;
     }
   }
-  if (!dot && !lined && p.vec > 1 && (p.lmode == M_GATHER || p.rmode == M_GATHER)) {
+  if (!lined && p.vec > 1 && (p.lmode == M_GATHER || p.rmode == M_GATHER)) {
     for (int nv = p.vec / 2; nv >= 1; nv /= 2) {
       if (nv > 1 && dout % nv != 0) continue;
       const int lm = op == OP_COPY_RHS ? M_CONTIG : pick_mode(p.bc, true, dout, nv, dl, lhs, es);
@@ -541,10 +560,24 @@ void choose_gspmm_lanes(GspmmParams& p, int op, int64_t dl, int64_t dr, int64_t 
       }
     }
   }
+  if (dout < p.vec) p.vec = 1;  // padded rows of fewer columns than a lane
+  p.run_len = dout;
+  p.lpg = (int)((dout + p.vec - 1) / p.vec);
+  if (dout % p.vec != 0) {
+    // padded rows: the last lane's columns end with the row, so it is no
+    // longer on the vec-aligned groups the modes were found for
+    if (p.lmode == M_SPLAT && dl != 1) p.lmode = M_GATHER;
+    if (p.rmode == M_SPLAT && dr != 1) p.rmode = M_GATHER;
+  }
 }
 
-// Lanes per row slab: the power of two covering the row's vectors, at most
-// 64. With MDGL_NARROW_SLABS, rows wider than 64 vectors take 32-lane slabs
+// Lanes a row takes with the layout chosen above.
+int64_t gspmm_row_lanes(const GspmmParams& p, int64_t dout) {
+  return p.run_len > 0 ? dout / p.run_len * p.lpg : 0;
+}
+
+// Lanes per row slab: the power of two covering the row's lanes, at least 16
+// (gspmm_impl.h says why) and at most 64. With MDGL_NARROW_SLABS, rows wider than 64 vectors take 32-lane slabs
 // (two rows per wavefront) when that makes at most GSPMM_NARROW_MAX_SLABS of
 // them: each slab walks all of a row's edges again, and on a graph whose
 // sources lie near their destinations the 512-byte slabs of a block of
@@ -552,13 +585,12 @@ void choose_gspmm_lanes(GspmmParams& p, int op, int64_t dl, int64_t dr, int64_t 
 // (float32 602-column rows: 3 -> 5 walks, 10-14 % faster on a 50-block
 // community graph; float64 ones: 5 -> 10 walks, 1-4 % slower, so excluded).
 constexpr int GSPMM_NARROW_MAX_SLABS = 5;
-int gspmm_group(int64_t dout, int vec, int flags, bool dot) {
-  const int64_t nvec = (dout + vec - 1) / vec;
+int gspmm_group(int64_t nvec, int flags, bool dot) {
   int gmax = WAVE;
   if ((flags & MDGL_NARROW_SLABS) && !dot && nvec > WAVE &&
       (nvec + WAVE / 2 - 1) / (WAVE / 2) <= GSPMM_NARROW_MAX_SLABS)
     gmax = WAVE / 2;
-  int g = 1;
+  int g = 16;
   while (g < nvec && g < gmax) g <<= 1;
   return g;
 }
@@ -687,14 +719,13 @@ int gspmm_common(const int32_t* indptr, const int32_t* indices, const int32_t* e
       return fail(MDGL_EINVAL, "gspmm: MDGL_LHS_LINE_ROWS needs lhs on a 128-byte boundary");
     p.lstride = (dl * es + 127) / 128 * 128 / es;
   }
-  const int vw = vec_width(dtype);
-  choose_gspmm_lanes(p, op, dl, dr, dout, lhs, rhs, es, dtype, dot_out != nullptr);
-  p.group = gspmm_group(dout, p.vec, flags, dot_out != nullptr);
-  if (p.vec > 1 && dout % p.vec == 0 && aligned(dst, p.vec * es)) p.flags |= F_OUT_VEC;
   if (dot_out) {
-    // the fused dot: mul / sum, 16-byte lanes, lhs rows contiguous, the edge
-    // operand constant over groups of D = dout / dr consecutive columns
-    // (D / vec lanes, a power of two up to 64), the row operand aligned
+    // the fused dot: mul / sum, lhs rows contiguous, the edge operand constant
+    // over runs of D = dout / dr consecutive columns, each on a power of two of
+    // 16-byte lanes (at most 64). Without MDGL_ANY_ALIGNMENT the runs are whole
+    // aligned lanes; with it any run of at least 16 bytes, the lanes past the
+    // run repeating its last columns and adding nothing
+    const int vw = vec_width(dtype);
     if (op != OP_MUL || reduce_op != RED_SUM)
       return fail(MDGL_EINVAL, "gspmm dot: mul with sum only");
     if (!rowop) return fail(MDGL_EINVAL, "gspmm dot: null row operand");
@@ -702,19 +733,28 @@ int gspmm_common(const int32_t* indptr, const int32_t* indices, const int32_t* e
       return fail(MDGL_EINVAL, "gspmm dot: dout %lld is not a multiple of dr %lld",
                   (long long)dout, (long long)dr);
     const int64_t D = dout / dr;
-    const int64_t lanes = D / vw;
-    bool ok = p.vec == vw && D % vw == 0 && lanes <= WAVE && (lanes & (lanes - 1)) == 0 &&
-              p.lmode == M_CONTIG && aligned(rowop, vw * es);
+    int64_t lanes = 1;
+    while (lanes * vw < D) lanes <<= 1;
+    bool ok = D >= vw && lanes <= WAVE;
+    if (!(flags & MDGL_ANY_ALIGNMENT))
+      ok = ok && D == lanes * vw && aligned(lhs, vw * es) && aligned(rowop, vw * es);
     for (int64_t k = 0; ok && k < dout; ++k)
       ok = bcast_off(p.bc, k, false) == k / D && bcast_off(p.bc, k, true) == k;
     if (!ok)
-      return fail(MDGL_ENOTSUP, "gspmm dot: needs contiguous aligned rows and the edge operand "
-                  "splat over power-of-two groups of 16-byte lanes");
+      return fail(MDGL_ENOTSUP, "gspmm dot: needs contiguous rows and the edge operand splat "
+                  "over groups of one 16-byte lane to 64 of them");
     p.rowop = rowop;
     p.dot_out = dot_out;
     p.dot_lanes = (int)lanes;
+    p.vec = vw;
+    p.run_len = D;
+    p.lpg = (int)lanes;
+    p.lmode = M_CONTIG;
     p.rmode = M_SPLAT;
+  } else {
+    choose_gspmm_lanes(p, op, dl, dr, dout, lhs, rhs, es, dtype, flags);
   }
+  p.group = gspmm_group(gspmm_row_lanes(p, dout), flags, dot_out != nullptr);
   hipError_t e;
   if (dtype == MDGL_FLOAT32) {
     e = p.red == RED_MAX ? launch_gspmm_red<float, RED_MAX>(p)
@@ -762,9 +802,10 @@ int mdgl_gspmm_rows(const int32_t* indptr, const int32_t* indices, const int32_t
                       rows, num_rows);
 }
 
-int mdgl_gspmm_lanes(int op, int64_t dl, int64_t dr, int64_t dout, int nd,
-                     const int64_t* lhs_shape, const int64_t* rhs_shape, const void* lhs,
-                     const void* rhs, int flags, int dtype, int64_t* vec, int64_t* group) {
+int mdgl_gspmm_layout(int op, int64_t dl, int64_t dr, int64_t dout, int nd,
+                      const int64_t* lhs_shape, const int64_t* rhs_shape, const void* lhs,
+                      const void* rhs, int flags, int dtype, int64_t* vec, int64_t* group,
+                      int64_t* lanes) {
   MDGL_RANGE();
   if (!dtype_ok(dtype)) return fail(MDGL_EINVAL, "gspmm_lanes: bad dtype %d", dtype);
   if (op < OP_ADD || op > OP_COPY_RHS || op == OP_DOT)
@@ -779,10 +820,18 @@ int mdgl_gspmm_lanes(int op, int64_t dl, int64_t dr, int64_t dout, int nd,
       return fail(MDGL_EINVAL, "gspmm_lanes: MDGL_LHS_LINE_ROWS needs lhs on a 128-byte boundary");
     p.lstride = (dl * es + 127) / 128 * 128 / es;
   }
-  choose_gspmm_lanes(p, op, dl, dr, dout, lhs, rhs, es, dtype, false);
+  choose_gspmm_lanes(p, op, dl, dr, dout, lhs, rhs, es, dtype, flags);
   *vec = p.vec;
-  if (group) *group = gspmm_group(dout, p.vec, flags, false);
+  if (group) *group = gspmm_group(gspmm_row_lanes(p, dout), flags, false);
+  if (lanes) *lanes = gspmm_row_lanes(p, dout);
   return MDGL_OK;
+}
+
+int mdgl_gspmm_lanes(int op, int64_t dl, int64_t dr, int64_t dout, int nd,
+                     const int64_t* lhs_shape, const int64_t* rhs_shape, const void* lhs,
+                     const void* rhs, int flags, int dtype, int64_t* vec, int64_t* group) {
+  return mdgl_gspmm_layout(op, dl, dr, dout, nd, lhs_shape, rhs_shape, lhs, rhs, flags, dtype,
+                           vec, group, nullptr);
 }
 
 static_assert(MDGL_COO_LOCALITY_BLOCKS == COO_LOCALITY_BLOCKS, "one count per workgroup");
@@ -797,6 +846,22 @@ int mdgl_coo_locality(const int32_t* u, const int32_t* v, int64_t num_edges, int
                     "coo_locality");
 }
 
+int mdgl_gspmm_mul_sum_dot_any(const int32_t* indptr, const int32_t* indices, const int32_t* eid,
+                           const void* lhs, const void* rhs, const void* rowop, void* dst,
+                           void* dot, int64_t num_dst, int64_t dl, int64_t dr, int64_t dout,
+                           int nd, const int64_t* lhs_shape, const int64_t* rhs_shape,
+                           const int32_t* chunk_row, const int32_t* chunk_start,
+                           int64_t num_chunks, int32_t chunk_len, const int32_t* heavy_rows,
+                           const int32_t* heavy_ptr, int64_t num_heavy, void* workspace,
+                           int64_t workspace_bytes, int flags, int dtype, void* stream) {
+  MDGL_RANGE();
+  if (num_dst > 0 && dout > 0 && !dot) return fail(MDGL_EINVAL, "gspmm dot: null dot output");
+  return gspmm_common(indptr, indices, eid, lhs, rhs, dst, num_dst, OP_MUL, dl, dr, dout, RED_SUM,
+                      nullptr, nd, lhs_shape, rhs_shape, nullptr, nullptr, chunk_row, chunk_start,
+                      num_chunks, chunk_len, heavy_rows, heavy_ptr, num_heavy, workspace,
+                      workspace_bytes, flags, dtype, stream, rowop, dot);
+}
+
 int mdgl_gspmm_mul_sum_dot(const int32_t* indptr, const int32_t* indices, const int32_t* eid,
                            const void* lhs, const void* rhs, const void* rowop, void* dst,
                            void* dot, int64_t num_dst, int64_t dl, int64_t dr, int64_t dout,
@@ -805,12 +870,10 @@ int mdgl_gspmm_mul_sum_dot(const int32_t* indptr, const int32_t* indices, const 
                            int64_t num_chunks, int32_t chunk_len, const int32_t* heavy_rows,
                            const int32_t* heavy_ptr, int64_t num_heavy, void* workspace,
                            int64_t workspace_bytes, int dtype, void* stream) {
-  MDGL_RANGE();
-  if (num_dst > 0 && dout > 0 && !dot) return fail(MDGL_EINVAL, "gspmm dot: null dot output");
-  return gspmm_common(indptr, indices, eid, lhs, rhs, dst, num_dst, OP_MUL, dl, dr, dout, RED_SUM,
-                      nullptr, nd, lhs_shape, rhs_shape, nullptr, nullptr, chunk_row, chunk_start,
-                      num_chunks, chunk_len, heavy_rows, heavy_ptr, num_heavy, workspace,
-                      workspace_bytes, 0, dtype, stream, rowop, dot);
+  return mdgl_gspmm_mul_sum_dot_any(indptr, indices, eid, lhs, rhs, rowop, dst, dot, num_dst, dl,
+                                    dr, dout, nd, lhs_shape, rhs_shape, chunk_row, chunk_start,
+                                    num_chunks, chunk_len, heavy_rows, heavy_ptr, num_heavy,
+                                    workspace, workspace_bytes, 0, dtype, stream);
 }
 
 namespace {

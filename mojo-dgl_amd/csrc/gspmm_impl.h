@@ -8,9 +8,18 @@
 // so each XCD serves a contiguous run of units and the rows of a block of
 // neighbouring destinations share its L2 (a community graph's chunks dealt
 // round-robin over the XCDs held its L2 hit rate at 70 %). A unit is processed
-// by G consecutive lanes (G = the power of two covering the row's vectors,
-// at most 64), so a wavefront packs 64 / G units; output rows wider than
-// 64 * VEC are cut into S slabs, one wavefront per slab.
+// by G consecutive lanes (G = the power of two covering the row's lanes, at
+// least 16 and at most 64), so a wavefront packs 64 / G units; output rows wider than
+// 64 lanes are cut into S slabs, one wavefront per slab.
+//
+// Lane columns. A row is made of dout / L runs of L columns over which each
+// operand is either consecutive or one value (run_len, from the broadcast;
+// one run when nothing broadcasts). Each run takes `lpg` lanes of VEC columns;
+// when VEC does not divide L the run's last lane starts VEC columns before its
+// end and so shares some with its neighbour (both compute and store the same
+// values). Every load and store is then a whole vector, at element alignment:
+// one float per lane made 47-column rows (47 lanes, 4 bytes each) move a
+// quarter of the bytes per instruction.
 //
 // Fold order. Each lane owns VEC output columns and folds its unit's CSR
 // slots one after the other, in CSR order: for a row that is not split this
@@ -21,20 +30,34 @@
 // the earlier chunk wins ties, so the arg is still the first edge in CSR
 // order reaching the value).
 //
-// Memory. Per 64 CSR slots a lane group issues one coalesced load of the
-// neighbour ids and one of the edge ids; the ids are then broadcast with
-// v_readlane (whole-wavefront units, scalar registers, so the row address is
-// formed on the scalar unit) or ds_bpermute (packed units). Each edge costs
-// one 16-byte (float32 rows of odd multiples of 2 columns: 8-byte) gather per
-// lane of the source row and one of the edge row, with U edges in flight per
-// lane.
+// Memory. U edges are in flight per lane, their ids loaded a batch ahead.
+// How the ids reach a unit's lanes depends on G:
+//   G = 64      64 ids per load, one per lane, broadcast by v_readlane into
+//               scalar registers;
+//   G = 16, 32  16 ids per load, the same 16 in each DPP row of the unit, row
+//               offsets formed once by the lane that loaded the id and
+//               broadcast by DPP (row_newbcast, one VALU operation per word;
+//               ds_bpermute with a 64-bit multiply per lane and edge took 45
+//               instructions per two edges).
+// Rows of fewer than 16 lanes take 16 all the same, the lanes past the row
+// repeating its last columns: with only the lanes they need, 1 to 8, a row had
+// as few edges in flight as lanes (one id per lane), and a wavefront of 8 to
+// 64 rows waited for the longest of them (4 columns on 4.9M edges of a
+// power-law graph: 1,121 us that way, 398 with 8 ids per lane instead, 192 at
+// 16 lanes; 16 columns on 89M edges, forward and backward: 7.7, 7.1, 6.6 ms).
+// Ids past a row repeat its last one, so id loads need no branch; operand rows
+// are requested and folded without one except in the batch that ends a row.
 #pragma once
+
+#include <type_traits>
+#include <utility>
 
 #include "mdgl_kernels.h"
 
 namespace mdgl {
 
 constexpr int M_DYN = 3;
+constexpr int M_SCALAR = 4;  // edge operand of one value per edge (dr == 1)
 
 template <class T>
 struct GspmmArgs {
@@ -50,7 +73,8 @@ struct GspmmArgs {
   int64_t num_rows, dl, dr, dout;
   int64_t lstride;  // elements between lhs rows
   Bcast bc;
-  int lmode, rmode, flags, G, S, vec;
+  int lmode, rmode, flags, gshift, S;
+  int run_len, lpg, nvec;  // columns per run, lanes per run, lanes per row
   int64_t num_chunks;
   const int32_t* chunk_row;
   const int32_t* chunk_start;
@@ -59,10 +83,9 @@ struct GspmmArgs {
   int32_t* part_u;
   int32_t* part_e;
   int64_t chunk_waves, row_waves, chunk_blocks, num_blocks;
-  // waves per slab (slab-major order: every unit's slab s before slab s + 1,
+  // waves per slab (with several, every unit's slab s comes before slab s + 1,
   // so the rows of neighbouring units share cache lines across wavefronts)
   int64_t chunk_uwaves, row_uwaves;
-  int slab_major;
   const T* rowop;  // dot output (see GspmmParams), else null
   T* dot_out;
   int dot_lanes;
@@ -70,52 +93,141 @@ struct GspmmArgs {
   int64_t row_limit;
 };
 
-template <class T, int VEC, int M>
+// N consecutive elements at element alignment (one 4- to 32-byte access).
+template <class T, int N>
+__device__ __forceinline__ void load_any(const T* p, T (&out)[N], bool stream) {
+  if constexpr (N == 1) {
+    out[0] = stream ? __builtin_nontemporal_load(p) : *p;
+  } else {
+    typedef T V __attribute__((ext_vector_type(N), aligned(sizeof(T))));
+    const V v = stream ? __builtin_nontemporal_load(reinterpret_cast<const V*>(p))
+                       : *reinterpret_cast<const V*>(p);
+#pragma unroll
+    for (int i = 0; i < N; ++i) out[i] = v[i];
+  }
+}
+
+template <class T, int N>
+__device__ __forceinline__ void store_any_stream(T* p, const T (&in)[N]) {
+  if constexpr (N == 1) {
+    *p = in[0];
+  } else {
+    typedef T V __attribute__((ext_vector_type(N), aligned(sizeof(T))));
+    V v;
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = in[i];
+    __builtin_nontemporal_store(v, reinterpret_cast<V*>(p));
+  }
+}
+
+// The VEC columns a lane reads from an operand row (off: their offsets; only
+// off[0] unless the mode is gather). Edge rows are read once per edge and
+// stream past the caches, so they do not displace source rows that other
+// edges will gather.
+template <class T, int VEC, int M, bool STREAM>
 __device__ __forceinline__ void fetch(const T* __restrict__ row, int mode_rt, const int (&off)[VEC],
                                       T (&x)[VEC]) {
   const int m = (M == M_DYN) ? mode_rt : M;
-  if (VEC > 1 && m == M_CONTIG) {
-    if constexpr (VEC > 1) load_n<T, VEC>(row + off[0], x);
+  if (m == M_CONTIG) {
+    load_any<T, VEC>(row + off[0], x, STREAM);
   } else if (m == M_SPLAT) {
-    const T s = row[off[0]];
+    const T s = STREAM ? __builtin_nontemporal_load(row + off[0]) : row[off[0]];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) x[v] = s;
   } else {
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) x[v] = row[off[v]];
+    for (int v = 0; v < VEC; ++v)
+      x[v] = STREAM ? __builtin_nontemporal_load(row + off[v]) : row[off[v]];
   }
 }
 
-// The same for the edge operand, read once per edge: non-temporal, so it
-// does not displace source rows that other edges will gather.
-template <class T, int VEC, int M>
-__device__ __forceinline__ void fetch_stream(const T* __restrict__ row, int mode_rt,
-                                             const int (&off)[VEC], T (&x)[VEC]) {
-  const int m = (M == M_DYN) ? mode_rt : M;
-  if (VEC > 1 && m == M_CONTIG) {
-    if constexpr (VEC > 1) load_n_stream<T, VEC>(row + off[0], x);
-  } else if (m == M_SPLAT) {
-    const T s = __builtin_nontemporal_load(row + off[0]);
-#pragma unroll
-    for (int v = 0; v < VEC; ++v) x[v] = s;
+// Lane N of each DPP row of 16 lanes, to all 16 of them.
+template <int N>
+__device__ __forceinline__ int row_bcast(int v) {
+  return __builtin_amdgcn_mov_dpp(v, 0x150 + N, 0xF, 0xF, false);
+}
+template <int N>
+__device__ __forceinline__ float row_bcast(float v) {
+  return __int_as_float(row_bcast<N>(__float_as_int(v)));
+}
+typedef int32_t int_pair __attribute__((ext_vector_type(2)));
+template <int N>
+__device__ __forceinline__ int64_t row_bcast(int64_t v) {
+  const int_pair p = __builtin_bit_cast(int_pair, v);  // a register pair, no shifts
+  const int_pair q = {row_bcast<N>(p[0]), row_bcast<N>(p[1])};
+  return __builtin_bit_cast(int64_t, q);
+}
+template <int N>
+__device__ __forceinline__ double row_bcast(double v) {
+  return __longlong_as_double(row_bcast<N>((int64_t)__double_as_longlong(v)));
+}
+
+template <class V>
+__device__ __forceinline__ V lane_xor_dpp(V v, int step) {
+  auto mov = [&](int w) {
+    return step == 0   ? __builtin_amdgcn_mov_dpp(w, 0xB1, 0xF, 0xF, false)    // quad [1,0,3,2]
+           : step == 1 ? __builtin_amdgcn_mov_dpp(w, 0x4E, 0xF, 0xF, false)    // quad [2,3,0,1]
+           : step == 2 ? __builtin_amdgcn_mov_dpp(w, 0x141, 0xF, 0xF, false)   // row_half_mirror
+                       : __builtin_amdgcn_mov_dpp(w, 0x140, 0xF, 0xF, false);  // row_mirror
+  };
+  if constexpr (sizeof(V) == 4) {
+    return __builtin_bit_cast(V, mov(__builtin_bit_cast(int, v)));
   } else {
-#pragma unroll
-    for (int v = 0; v < VEC; ++v) x[v] = __builtin_nontemporal_load(row + off[v]);
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)mov((int)(uint32_t)b), hi = (uint32_t)mov((int)(b >> 32));
+    return __builtin_bit_cast(V, ((uint64_t)hi << 32) | lo);
   }
 }
 
-template <class T, int OP, int RED, int VEC, int LM, int RM, bool WIDE, bool NT,
-          bool DOT = false>
+// Sum over groups of `lanes` (a power of two) consecutive lanes, in every
+// lane of the group: the butterfly's partners 1, 2, 4, 8 lanes away by DPP (a
+// mirror stands in for 4 and 8, whose partners already hold equal sums).
+template <class T>
+__device__ __forceinline__ T group_sum(T v, int lanes) {
+  if (lanes > 1) v = v + lane_xor_dpp(v, 0);
+  if (lanes > 2) v = v + lane_xor_dpp(v, 1);
+  if (lanes > 4) v = v + lane_xor_dpp(v, 2);
+  if (lanes > 8) v = v + lane_xor_dpp(v, 3);
+  if (lanes > 16) v = v + __shfl_xor(v, 16);
+  if (lanes > 32) v = v + __shfl_xor(v, 32);
+  return v;
+}
+
+// A lambda kept out of line would put the arrays it captures in memory.
+#define MDGL_INLINE __attribute__((always_inline))
+
+// f(0), ..., f(N - 1) with the number known to the compiler.
+template <int... I, class F>
+__device__ __forceinline__ void for_each_of(std::integer_sequence<int, I...>, F f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void for_each(F f) {
+  for_each_of(std::make_integer_sequence<int, N>{}, f);
+}
+
+// How ids reach the lanes of a unit (see the top): by G.
+enum { LAY_ROW = 0, LAY_WIDE = 1 };
+
+template <class T, int OP, int RED, int VEC, int LM, int RM, int LAY, bool DOT = false>
 __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, int64_t wave,
                                            int lane) {
   // edges in flight per lane: 8 (4 in the dot pass, whose per-edge
   // butterflies already hide the loads; 8 there cost 14 %)
   constexpr int U = DOT ? 4 : 8;
-  const int G = WIDE ? WAVE : a.G;
-  const int grp = lane / G, gl = lane % G, gbase = grp * G;
-  const int64_t uw = chunk ? a.chunk_uwaves : a.row_uwaves;
-  const int64_t slab = a.slab_major ? wave / uw : wave % a.S;
-  const int64_t unit = (a.slab_major ? wave % uw : wave / a.S) * (WAVE / G) + grp;
+  constexpr bool ARG = (RED == RED_MAX || RED == RED_MIN);
+  constexpr bool HAS_L = OP != OP_COPY_RHS, HAS_R = OP != OP_COPY_LHS;
+  const int G = LAY == LAY_WIDE ? WAVE : 1 << a.gshift;
+  const int grp = LAY == LAY_WIDE ? 0 : lane >> a.gshift, gl = lane & (G - 1);
+  // (a 64-bit divide is about a hundred instructions, and rows of a few
+  // edges run few more: none where one slab or one run makes it 1)
+  int slab = 0;
+  if (a.S > 1) {
+    const int64_t uw = chunk ? a.chunk_uwaves : a.row_uwaves;
+    slab = (int)(wave / uw);
+    wave -= slab * uw;
+  }
+  const int64_t unit = LAY == LAY_WIDE ? wave : (wave << (6 - a.gshift)) + grp;
 
   // ---- resolve the unit to a CSR slot range
   bool ok = unit < (chunk ? a.num_chunks : a.num_rows);
@@ -142,14 +254,29 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
   }
 
   // ---- this lane's output columns and operand offsets
-  const int64_t k0 = (slab * G + gl) * VEC;
-  const bool feat_ok = k0 < a.dout;
+  int li = slab * G + gl;
+  const bool feat_ok = li < a.nvec;
+  if (!feat_ok) li = a.nvec - 1;  // a lane past the row repeats its last one, unwritten
+  int64_t k0 = 0;
+  int dup = 0;  // leading columns that the run's previous lane also holds
+  {
+    const int run = a.lpg == a.nvec ? 0 : li / a.lpg, j = li - run * a.lpg;
+    const int c = j * VEC < a.run_len - VEC ? j * VEC : a.run_len - VEC;
+    k0 = (int64_t)run * a.run_len + c;
+    dup = j * VEC - c < VEC ? j * VEC - c : VEC;
+  }
   int loff[VEC], roff[VEC];
 #pragma unroll
   for (int v = 0; v < VEC; ++v) {
-    const int64_t k = (feat_ok && k0 + v < a.dout) ? k0 + v : (feat_ok ? k0 : 0);
-    loff[v] = (int)bcast_off(a.bc, k, true);
-    roff[v] = (int)bcast_off(a.bc, k, false);
+    const bool each = (LM == M_DYN && RM == M_DYN);
+    loff[v] = roff[v] = 0;
+    if (a.bc.nd == 1) {
+      loff[v] = (int)((k0 + v) * a.bc.lstride[0]);
+      roff[v] = (int)((k0 + v) * a.bc.rstride[0]);
+    } else if (v == 0 || each) {
+      loff[v] = (int)bcast_off(a.bc, k0 + v, true);
+      roff[v] = (int)bcast_off(a.bc, k0 + v, false);
+    }
   }
 
   // DOT: this row's own feature columns, dotted with every gathered lhs row
@@ -157,142 +284,183 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
   if constexpr (DOT) {
 #pragma unroll
     for (int v = 0; v < VEC; ++v) rowv[v] = T(0);
-    if (ok && feat_ok) load_n<T, VEC>(a.rowop + row * a.dout + k0, rowv);
+    if (ok) load_any<T, VEC>(a.rowop + row * a.dout + k0, rowv, false);
   }
 
   T acc[VEC];
-  int au[VEC], ae[VEC];
+  int at[VEC];  // max / min: the CSR slot selected (-1: none yet)
 #pragma unroll
   for (int v = 0; v < VEC; ++v) {
     acc[v] = seed<T>(RED);
-    au[v] = -1;  // nothing selected yet
-    ae[v] = -1;
+    at[v] = -1;
   }
 
   const bool ident = a.flags & F_EID_IDENTITY;
-  constexpr bool ARG_OUT = (RED == RED_MAX || RED == RED_MIN);
   const int n = ok ? stop - start : 0;
-  const int nmax = WIDE ? n : wave_max_int(n);
   // a scalar edge operand (one value per edge, splatted over the columns) is
   // loaded with the ids, one edge per lane, and broadcast like them
-  constexpr bool SCALAR_E = RM == M_SPLAT && OP != OP_COPY_LHS;
-  const bool scalar_e = SCALAR_E && a.dr == 1;
+  constexpr bool SCALAR = RM == M_SCALAR && HAS_R;
+  constexpr bool ROW_R = HAS_R && !SCALAR;
   // the edge operand may come in CSR slot order (row i of rhs for slot i)
   const bool rhs_csr = a.flags & F_RHS_CSR;
-  // edge ids are read only for an arg or an edge operand in edge-id order
-  // (fixed at compile time where it can be: the dot pass, whose edge operand
-  // is always in edge-id order, ran 11 % slower with the load made
-  // conditional at run time)
-  constexpr bool E_ALWAYS = ARG_OUT || DOT;
-  constexpr bool E_NEVER = !ARG_OUT && OP == OP_COPY_LHS;
-  const bool need_e = E_ALWAYS || (!E_NEVER && !rhs_csr);
-  for (int base = 0; base < nmax; base += G) {
-    int my_s = 0, my_e = 0;
-    T my_w = T(0);
-    if (base + gl < n) {
-      const int i = start + base + gl;
-      if (a.indices) my_s = __builtin_nontemporal_load(a.indices + i);
-      my_e = ident ? i : (need_e ? __builtin_nontemporal_load(a.eid + i) : 0);
-      if (SCALAR_E && scalar_e) my_w = a.rhs[rhs_csr ? (int64_t)i : (int64_t)my_e];
-    }
-    const int cnt = n - base < G ? n - base : G;  // may be <= 0 on finished groups
-    const int jmax = WIDE ? cnt : (nmax - base < G ? nmax - base : G);
-    for (int j = 0; j < jmax; j += U) {
-      T x[U][VEC], y[U][VEC];
-      int su[U], se[U];
+  const bool need_e = HAS_R && !rhs_csr && !ident;
+
+  const char* const lbase = reinterpret_cast<const char*>(a.lhs + loff[0]);
+  const char* const rbase = reinterpret_cast<const char*>(a.rhs + roff[0]);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int jj = (j + u < G) ? j + u : G - 1;
-        // copy_rhs needs the source only for an arg
-        constexpr bool NEED_S = OP != OP_COPY_RHS || ARG_OUT;
-        int s = 0, e;
-        if constexpr (WIDE) {
-          e = readlane_int(my_e, jj);
+  for (int v = VEC - 1; v >= 0; --v) {  // from here on relative to the lane's first column
+    loff[v] -= loff[0];
+    roff[v] -= roff[0];
+  }
+
+  // One batch is the edges of U slots, of which the first `rem` are the
+  // unit's (all U with FULL: no branch per edge). `lo_of` / `ro_of` give the
+  // byte offset of edge u's operand rows, `w_of` its value of a scalar edge
+  // operand, `after` runs between the requests and the folds. A broadcast right
+  // before its request keeps one offset live instead of U of them (32
+  // registers, and with them two wavefronts per SIMD).
+  auto batch = [&](auto full, int slot0, int rem, auto lo_of, auto ro_of, auto w_of,
+                   auto after) MDGL_INLINE {
+    constexpr bool FULL = decltype(full)::value;
+    T x[U][VEC], y[U][VEC], w[U];
+    auto request = [&](auto iu) MDGL_INLINE {
+      constexpr int u = decltype(iu)::value;
+      if constexpr (HAS_L)
+        fetch<T, VEC, LM, false>(reinterpret_cast<const T*>(lbase + lo_of(iu)), a.lmode, loff,
+                                 x[u]);
+      if constexpr (ROW_R)
+        fetch<T, VEC, RM, true>(reinterpret_cast<const T*>(rbase + ro_of(iu)), a.rmode, roff,
+                                y[u]);
+    };
+    auto fold = [&](auto iu) MDGL_INLINE {
+      constexpr int u = decltype(iu)::value;
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        T xv = T(0), yv = T(0);
+        if constexpr (HAS_L) xv = x[u][v];
+        if constexpr (SCALAR) yv = w[u];
+        else if constexpr (HAS_R) yv = y[u][v];
+        const T m = message<OP>(xv, yv);
+        if constexpr (RED == RED_MAX) {
+          if (m > acc[v]) { acc[v] = m; at[v] = slot0 + u; }
+        } else if constexpr (RED == RED_MIN) {
+          if (m < acc[v]) { acc[v] = m; at[v] = slot0 + u; }
         } else {
-          e = __shfl(my_e, gbase + jj);
-        }
-        if constexpr (NEED_S) {
-          if constexpr (WIDE) s = readlane_int(my_s, jj);
-          else s = __shfl(my_s, gbase + jj);
-        }
-        su[u] = s;
-        se[u] = e;
-        if constexpr (SCALAR_E) {
-          if (scalar_e) {
-            T w;
-            if constexpr (WIDE) w = readlane_val(my_w, jj);
-            else w = __shfl(my_w, gbase + jj);
-#pragma unroll
-            for (int v = 0; v < VEC; ++v) y[u][v] = w;
-          }
-        }
-        if (j + u < cnt && feat_ok) {
-          if constexpr (OP != OP_COPY_RHS)
-            fetch<T, VEC, LM>(a.lhs + (int64_t)s * a.lstride, a.lmode, loff, x[u]);
-          if constexpr (OP != OP_COPY_LHS) {
-            if (!(SCALAR_E && scalar_e)) {
-              const int64_t rrow = rhs_csr ? (int64_t)(start + base + j + u) : (int64_t)e;
-              // a row gathered by a random edge id is read once: stream it
-              if constexpr (NT)
-                fetch_stream<T, VEC, RM>(a.rhs + rrow * a.dr, a.rmode, roff, y[u]);
-              else
-                fetch<T, VEC, RM>(a.rhs + rrow * a.dr, a.rmode, roff, y[u]);
-            }
-          }
+          acc[v] = acc[v] + m;
         }
       }
-      if constexpr (DOT) {
-        // per slot and column group: the lanes' partial dots, then a
-        // butterfly over the group's lanes; the group's first lane writes
+    };
+    // DOT: the lanes' partial dots per edge and column group, then the sum
+    // over the group's lanes; the group's first lane writes
+    auto dot = [&](auto iu) MDGL_INLINE {
+      constexpr int u = decltype(iu)::value;
+      T pd = T(0);
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          if (j + u >= jmax) break;  // uniform in the wavefront
-          T pd = T(0);
-          if (j + u < cnt && feat_ok) {
-#pragma unroll
-            for (int v = 0; v < VEC; ++v) pd = pd + x[u][v] * rowv[v];
-          }
-          for (int off = 1; off < a.dot_lanes; off <<= 1) pd = pd + __shfl_xor(pd, off);
-          if (j + u < cnt && feat_ok && (gl % a.dot_lanes) == 0) {
-            const int64_t slot = start + base + j + u;
-            a.dot_out[slot * a.dr + k0 / ((int64_t)a.dot_lanes * VEC)] = pd;
-          }
-        }
+      for (int v = 0; v < VEC; ++v) pd = v < dup ? pd : pd + x[u][v] * rowv[v];
+      pd = group_sum(pd, a.dot_lanes);
+      if (feat_ok && (gl & (a.dot_lanes - 1)) == 0)
+        a.dot_out[(int64_t)(slot0 + u) * a.dr + li / a.dot_lanes] = pd;
+    };
+    for_each<U>([&](auto iu) MDGL_INLINE {
+      if (FULL || decltype(iu)::value < rem) request(iu);
+    });
+    after();
+    if constexpr (SCALAR)
+      for_each<U>([&](auto iu) MDGL_INLINE { w[decltype(iu)::value] = w_of(iu); });
+    if constexpr (DOT)
+      for_each<U>([&](auto iu) MDGL_INLINE {
+        if (FULL || decltype(iu)::value < rem) dot(iu);
+      });
+    for_each<U>([&](auto iu) MDGL_INLINE {
+      if (FULL || decltype(iu)::value < rem) fold(iu);
+    });
+  };
+  const int64_t lbytes = a.lstride * (int64_t)sizeof(T), rbytes = a.dr * (int64_t)sizeof(T);
+
+  if constexpr (LAY == LAY_ROW) {
+    // ---- 16 ids per load, broadcast by DPP: a unit's lanes (whole DPP rows)
+    // take every branch together, so the lane that holds an id is active
+    const int nmax = wave_max_int(n);
+    int my_s = 0, my_e = 0;
+    // past the unit's slots its last one; slot 0 for a unit without any
+    auto fill = [&](int base) MDGL_INLINE {
+      const int p = base + (lane & 15);
+      const int i = n > 0 ? start + (p < n ? p : n - 1) : 0;
+      if constexpr (HAS_L) my_s = a.indices[i];
+      if constexpr (HAS_R) {
+        my_e = i;
+        if (need_e) my_e = a.eid[i];
       }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (j + u < cnt && feat_ok) {
-#pragma unroll
-          for (int v = 0; v < VEC; ++v) {
-            T xv = T(0), yv = T(0);
-            if constexpr (OP != OP_COPY_RHS) xv = x[u][v];
-            if constexpr (OP != OP_COPY_LHS) yv = y[u][v];
-            const T m = message<OP>(xv, yv);
-            if constexpr (RED == RED_MAX) {
-              if (m > acc[v]) { acc[v] = m; au[v] = su[u]; ae[v] = se[u]; }
-            } else if constexpr (RED == RED_MIN) {
-              if (m < acc[v]) { acc[v] = m; au[v] = su[u]; ae[v] = se[u]; }
-            } else {
-              acc[v] = acc[v] + m;
-            }
-          }
-        }
+    };
+    if (nmax > 0) fill(0);
+    for (int base = 0; base < nmax; base += 16) {
+      int64_t my_lo = 0, my_ro = 0;
+      T my_w = T(0);
+      if constexpr (HAS_L) my_lo = (int64_t)my_s * lbytes;
+      if constexpr (SCALAR) my_w = a.rhs[my_e];
+      else if constexpr (HAS_R) my_ro = (int64_t)my_e * rbytes;
+      if (base + 16 < nmax) fill(base + 16);
+      for_each<16 / U>([&](auto part) MDGL_INLINE {
+        constexpr int F = decltype(part)::value * U;
+        const int rem = n - base - F;
+        if (rem <= 0) return;
+        auto lo_of = [&](auto iu) MDGL_INLINE { return row_bcast<F + decltype(iu)::value>(my_lo); };
+        auto ro_of = [&](auto iu) MDGL_INLINE { return row_bcast<F + decltype(iu)::value>(my_ro); };
+        auto w_of = [&](auto iu) MDGL_INLINE { return row_bcast<F + decltype(iu)::value>(my_w); };
+        if (rem >= U)
+          batch(std::true_type{}, start + base + F, U, lo_of, ro_of, w_of, [] {});
+        else
+          batch(std::false_type{}, start + base + F, rem, lo_of, ro_of, w_of, [] {});
+      });
+    }
+  } else {
+    // ---- 64 ids per load, broadcast by v_readlane (n is uniform here)
+    const int un = __builtin_amdgcn_readfirstlane(n);
+    const int ustart = __builtin_amdgcn_readfirstlane(start);
+    int my_s = 0, my_e = 0;
+    auto fill = [&](int base) MDGL_INLINE {
+      const int p = base + lane;
+      const int i = ustart + (p < un ? p : un - 1);
+      if constexpr (HAS_L) my_s = __builtin_nontemporal_load(a.indices + i);
+      if constexpr (HAS_R) {
+        my_e = i;
+        if (need_e) my_e = __builtin_nontemporal_load(a.eid + i);
+      }
+    };
+    if (un > 0) fill(0);
+    for (int base = 0; base < un; base += WAVE) {
+      const int cs = my_s, ce = my_e;
+      T my_w = T(0);
+      if constexpr (SCALAR) my_w = a.rhs[ce];
+      if (base + WAVE < un) fill(base + WAVE);
+      const int cnt = un - base < WAVE ? un - base : WAVE;
+      for (int j = 0; j < cnt; j += U) {
+        auto lo_of = [&](auto iu) MDGL_INLINE {
+          return (int64_t)readlane_int(cs, j + decltype(iu)::value) * lbytes;
+        };
+        auto ro_of = [&](auto iu) MDGL_INLINE {
+          return (int64_t)readlane_int(ce, j + decltype(iu)::value) * rbytes;
+        };
+        auto w_of = [&](auto iu) MDGL_INLINE {
+          return readlane_val(my_w, (j + decltype(iu)::value) & (WAVE - 1));
+        };
+        if (cnt - j >= U)
+          batch(std::true_type{}, ustart + base + j, U, lo_of, ro_of, w_of, [] {});
+        else
+          batch(std::false_type{}, ustart + base + j, cnt - j, lo_of, ro_of, w_of, [] {});
       }
     }
   }
 
   if (!ok || !feat_ok) return;
-  constexpr bool ARG = (RED == RED_MAX || RED == RED_MIN);
   if (chunk) {
     const int64_t o = unit * a.dout + k0;
 #pragma unroll
     for (int v = 0; v < VEC; ++v) {
-      if (k0 + v < a.dout) {
-        a.part_val[o + v] = acc[v];
-        if constexpr (ARG) {
-          a.part_u[o + v] = au[v];
-          a.part_e[o + v] = ae[v];
-        }
+      a.part_val[o + v] = acc[v];
+      if constexpr (ARG) {
+        a.part_u[o + v] = at[v] >= 0 && a.indices ? a.indices[at[v]] : -1;
+        a.part_e[o + v] = at[v] >= 0 && a.eid ? a.eid[at[v]] : -1;
       }
     }
     return;
@@ -308,67 +476,65 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
     for (int v = 0; v < VEC; ++v)
       if (is_inf(acc[v])) {
         acc[v] = T(0);  // a replaced value has no message behind it
-        au[v] = -1;
-        ae[v] = -1;
+        at[v] = -1;
       }
   }
   const int64_t o = row * a.dout + k0;
-  if (VEC > 1 && (a.flags & F_OUT_VEC)) {
-    if constexpr (VEC > 1) store_n_stream<T, VEC>(a.out + o, acc);
-  } else {
-#pragma unroll
-    for (int v = 0; v < VEC; ++v)
-      if (k0 + v < a.dout) a.out[o + v] = acc[v];
-  }
+  store_any_stream<T, VEC>(a.out + o, acc);
   if constexpr (ARG) {
+    auto put = [&](int32_t* dst, const int32_t* id) {
+      int32_t x[VEC];
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) {
-      if (k0 + v < a.dout) {
-        if (a.arg_u) a.arg_u[o + v] = au[v];
-        if (a.arg_e) a.arg_e[o + v] = ae[v];
-      }
-    }
+      for (int v = 0; v < VEC; ++v) x[v] = at[v] >= 0 ? id[at[v]] : -1;
+      store_any_stream<int32_t, VEC>(dst + o, x);
+    };
+    if (a.arg_u) put(a.arg_u, a.indices);
+    if (a.arg_e) put(a.arg_e, a.eid);
   }
 }
 
 // Kernel variants, one body each so that every launch only carries the
-// registers of its own path: whole-wavefront units (G = 64) with both
-// operands contiguous, with a splatted edge operand, or any modes; packed
-// units likewise. A scalar edge operand (one value per edge) is loaded with
-// the ids and broadcast by v_readlane or ds_bpermute in both layouts: read
-// per lane and edge through the any-modes path it cost a GCN aggregation over
-// 128 columns 4x the time of the same gather without the weight.
-enum { P_WIDE_CC = 0, P_WIDE_CS = 1, P_WIDE_DYN = 2, P_PACK_CC = 3, P_PACK_DYN = 4,
-       P_WIDE_CS_DOT = 5, P_PACK_DYN_DOT = 6, P_PACK_CS = 7 };
+// registers of its own path: per id layout, with both operands contiguous,
+// with a splatted edge operand, with a scalar edge operand (one value per
+// edge), or any modes. The scalar one is loaded with the ids and broadcast like
+// them: read per lane and edge through the any-modes path it cost a GCN
+// aggregation over 128 columns 4x the time of the same gather without it.
+enum { P_CC = 0, P_CS = 1, P_DYN = 2, P_CS_DOT = 3, P_CW = 4 };
 
-template <class T, int OP, int RED, int VEC, int PATH, bool NT>
-__global__ __launch_bounds__(BLOCK) void gspmm_kernel(GspmmArgs<T> a) {
+// Wavefronts per SIMD asked of the register allocation: what each path needs
+// plus a few registers would otherwise round down to one wavefront less (98
+// registers for both operands contiguous: 4 instead of 5, and 9 % of the time
+// on rows of 5 edges of two 256-byte rows).
+// Sums only: the other reducers' selected slots and a divide's temporaries
+// would spill.
+constexpr int gspmm_waves(int op, int red, int path, int lay, int vec, int size) {
+  if (red != RED_SUM || op == OP_DIV || path == P_DYN || vec * size > 16) return 1;
+  if (path == P_CC && op != OP_COPY_LHS && op != OP_COPY_RHS) return lay == LAY_WIDE ? 6 : 5;
+  return size == 8 ? 6 : 7;
+}
+
+template <class T, int OP, int RED, int VEC, int PATH, int LAY>
+__global__ __launch_bounds__(BLOCK, gspmm_waves(OP, RED, PATH, LAY, VEC, sizeof(T))) void
+gspmm_kernel(GspmmArgs<T> a) {
   const int64_t b = blockIdx.x;
   const bool chunk = b < a.chunk_blocks;
   const int64_t blk =
       chunk ? xcd_remap(b, a.chunk_blocks) : xcd_remap(b - a.chunk_blocks, a.num_blocks - a.chunk_blocks);
   const int lane = threadIdx.x & (WAVE - 1);
-  // every lane of a wavefront takes the same path below, so shuffles and
+  // every lane of a wavefront takes the same path below, so DPP moves and
   // readlanes always see a full wavefront
   const int64_t wave = blk * WAVES_PER_BLOCK + (threadIdx.x >> 6);
   if (wave >= (chunk ? a.chunk_waves : a.row_waves)) return;
-  if constexpr (PATH == P_WIDE_CC)
-    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_CONTIG, true, NT>(a, chunk, wave, lane);
-  else if constexpr (PATH == P_WIDE_CS)
-    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SPLAT, true, NT>(a, chunk, wave, lane);
-  else if constexpr (PATH == P_WIDE_DYN)
-    gspmm_body<T, OP, RED, VEC, M_DYN, M_DYN, true, NT>(a, chunk, wave, lane);
-  else if constexpr (PATH == P_PACK_CC)
-    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_CONTIG, false, NT>(a, chunk, wave, lane);
-  else if constexpr (PATH == P_PACK_CS)
-    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SPLAT, false, NT>(a, chunk, wave, lane);
-  else if constexpr (PATH == P_WIDE_CS_DOT)
-    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SPLAT, true, NT, true>(a, chunk, wave, lane);
-  else if constexpr (PATH == P_PACK_DYN_DOT)
-    gspmm_body<T, OP, RED, VEC, M_DYN, M_DYN, false, NT, true>(a, chunk, wave, lane);
-
+  if constexpr (PATH == P_CC)
+    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_CONTIG, LAY>(a, chunk, wave, lane);
+  else if constexpr (PATH == P_CS)
+    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SPLAT, LAY>(a, chunk, wave, lane);
+  else if constexpr (PATH == P_CW)
+    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SCALAR, LAY>(a, chunk, wave, lane);
+  else if constexpr (PATH == P_CS_DOT)
+    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SPLAT, LAY, true>(a, chunk, wave, lane);
   else
-    gspmm_body<T, OP, RED, VEC, M_DYN, M_DYN, false, NT>(a, chunk, wave, lane);
+    gspmm_body<T, OP, RED, VEC, M_DYN, M_DYN, LAY>(a, chunk, wave, lane);
 }
 
 // Folds the chunk partials of each heavy row in chunk (= CSR) order.
@@ -385,14 +551,35 @@ __global__ __launch_bounds__(BLOCK) void gspmm_combine_kernel(
   const int64_t row = heavy_rows[h];
   T acc = seed<T>(RED);
   int au = -1, ae = -1;
-  for (int c = heavy_ptr[h]; c < heavy_ptr[h + 1]; ++c) {
-    const T v = part_val[(int64_t)c * dout + k];
-    if constexpr (RED == RED_MAX) {
-      if (v > acc) { acc = v; au = part_u[(int64_t)c * dout + k]; ae = part_e[(int64_t)c * dout + k]; }
-    } else if constexpr (RED == RED_MIN) {
-      if (v < acc) { acc = v; au = part_u[(int64_t)c * dout + k]; ae = part_e[(int64_t)c * dout + k]; }
-    } else {
-      acc = acc + v;
+  // C partials requested at once (a chain of single loads made a hub of
+  // hundreds of chunks wait for each of them in turn); past the end the last
+  // one again, not folded
+  constexpr int C = 16;
+  const int c1 = heavy_ptr[h + 1];
+  int sel = -1;  // max / min: the chunk selected
+  for (int c = heavy_ptr[h]; c < c1; c += C) {
+    T v[C];
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const int cc = c + j < c1 ? c + j : c1 - 1;
+      v[j] = part_val[(int64_t)cc * dout + k];
+    }
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const bool in = c + j < c1;
+      if constexpr (RED == RED_MAX) {
+        if (in && v[j] > acc) { acc = v[j]; sel = c + j; }
+      } else if constexpr (RED == RED_MIN) {
+        if (in && v[j] < acc) { acc = v[j]; sel = c + j; }
+      } else {
+        acc = in ? acc + v[j] : acc;
+      }
+    }
+  }
+  if constexpr (RED == RED_MAX || RED == RED_MIN) {
+    if (sel >= 0) {
+      au = part_u[(int64_t)sel * dout + k];
+      ae = part_e[(int64_t)sel * dout + k];
     }
   }
   if (flags & F_MEAN) {
@@ -411,23 +598,18 @@ __global__ __launch_bounds__(BLOCK) void gspmm_combine_kernel(
   }
 }
 
-template <class T, int OP, int RED, int VEC, bool NT>
+template <class T, int OP, int RED, int VEC, int LAY>
 void launch_path(const GspmmArgs<T>& a, dim3 grid, dim3 block, int lm, int rm, hipStream_t st) {
-  if (a.G == WAVE) {
-    if (lm == M_CONTIG && rm == M_CONTIG)
-      hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_WIDE_CC, NT>), grid, block, 0, st, a);
-    else if (lm == M_CONTIG && rm == M_SPLAT)
-      hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_WIDE_CS, NT>), grid, block, 0, st, a);
-    else
-      hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_WIDE_DYN, NT>), grid, block, 0, st, a);
-  } else {
-    if (lm == M_CONTIG && rm == M_CONTIG)
-      hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_PACK_CC, NT>), grid, block, 0, st, a);
-    else if (lm == M_CONTIG && rm == M_SPLAT)
-      hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_PACK_CS, NT>), grid, block, 0, st, a);
-    else
-      hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_PACK_DYN, NT>), grid, block, 0, st, a);
-  }
+  if constexpr (OP == OP_COPY_LHS || OP == OP_COPY_RHS)
+    hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CC, LAY>), grid, block, 0, st, a);
+  else if (lm == M_CONTIG && rm == M_CONTIG)
+    hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CC, LAY>), grid, block, 0, st, a);
+  else if (lm == M_CONTIG && rm == M_SCALAR)
+    hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CW, LAY>), grid, block, 0, st, a);
+  else if (lm == M_CONTIG && rm == M_SPLAT)
+    hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CS, LAY>), grid, block, 0, st, a);
+  else
+    hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_DYN, LAY>), grid, block, 0, st, a);
 }
 
 template <class T, int OP, int RED, int VEC>
@@ -451,10 +633,13 @@ hipError_t launch_gspmm_op(const GspmmParams& p) {
   a.lmode = p.lmode;
   a.rmode = p.rmode;
   a.flags = p.flags;
-  a.vec = VEC;
-  const int64_t nvec = (p.dout + VEC - 1) / VEC;
+  a.run_len = (int)p.run_len;
+  a.lpg = p.lpg;
+  const int64_t nvec = p.dout / p.run_len * p.lpg;
+  a.nvec = (int)nvec;
   const int G = p.group;  // chosen by the host (gspmm_group)
-  a.G = G;
+  a.gshift = 0;
+  while ((1 << a.gshift) < G) ++a.gshift;
   a.S = (int)((nvec + G - 1) / G);
   a.num_chunks = p.num_chunks;
   a.chunk_row = p.chunk_row;
@@ -468,7 +653,6 @@ hipError_t launch_gspmm_op(const GspmmParams& p) {
   a.row_uwaves = (p.num_rows + per_wave - 1) / per_wave;
   a.chunk_waves = a.chunk_uwaves * a.S;
   a.row_waves = a.row_uwaves * a.S;
-  a.slab_major = a.S > 1;
   a.chunk_blocks = (a.chunk_waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
   a.num_blocks = a.chunk_blocks + (a.row_waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
   a.rowop = static_cast<const T*>(p.rowop);
@@ -479,24 +663,27 @@ hipError_t launch_gspmm_op(const GspmmParams& p) {
   if (a.num_blocks > 0) {
     const bool copy_l = OP == OP_COPY_LHS, copy_r = OP == OP_COPY_RHS;
     const int lm = copy_r ? a.rmode : a.lmode;
-    const int rm = copy_l ? a.lmode : a.rmode;
+    const int rm = copy_l ? a.lmode : (!copy_r && a.rmode == M_SPLAT && a.dr == 1 ? M_SCALAR : a.rmode);
     const dim3 grid((unsigned)a.num_blocks), block(BLOCK);
-    // edge rows are streamed (NT = true: every caller gathers them by edge
-    // id or reads each once in CSR order)
     bool launched = false;
-    if constexpr (OP == OP_MUL && RED == RED_SUM) {
+    if constexpr (OP == OP_MUL && RED == RED_SUM && VEC == VecOf<T>::n) {
       if (p.dot_out) {
         // the caller checked: contiguous lhs rows, rhs splat over the groups
-        if (a.G == WAVE)
-          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_WIDE_CS_DOT, true>), grid, block, 0,
+        if (G == WAVE)
+          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CS_DOT, LAY_WIDE>), grid, block, 0,
                              p.stream, a);
         else
-          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_PACK_DYN_DOT, true>), grid, block,
-                             0, p.stream, a);
+          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CS_DOT, LAY_ROW>), grid, block, 0,
+                             p.stream, a);
         launched = true;
       }
     }
-    if (!launched) launch_path<T, OP, RED, VEC, true>(a, grid, block, lm, rm, p.stream);
+    if (!launched) {
+      if (G == WAVE)
+        launch_path<T, OP, RED, VEC, LAY_WIDE>(a, grid, block, lm, rm, p.stream);
+      else
+        launch_path<T, OP, RED, VEC, LAY_ROW>(a, grid, block, lm, rm, p.stream);
+    }
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
   }

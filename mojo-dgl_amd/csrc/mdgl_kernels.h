@@ -11,7 +11,6 @@ namespace mdgl {
 enum {
   F_MEAN = 1,          // divide the sum by max(degree, 1)
   F_REPLACE_INF = 2,   // +-inf -> 0 on the final value (update_all max/min)
-  F_OUT_VEC = 4,       // output rows allow 16-byte stores
   F_EID_IDENTITY = 8,  // edge id of CSR slot i is i (copy_lhs given no edge ids)
   F_RHS_CSR = 16,      // the edge operand is in CSR slot order (rhs row i for slot i)
 };
@@ -37,7 +36,9 @@ struct GspmmParams {
   int op, red;  // red in {SUM, MAX, MIN}; mean is F_MEAN
   int flags;
   int vec;      // elements per lane (1 or 16 / sizeof(T))
-  int group;    // lanes per row slab (a power of two, at most 64)
+  int64_t run_len;  // columns per run of consecutive operand columns (>= vec)
+  int lpg;      // lanes per run
+  int group;    // lanes per row slab (16, 32 or 64)
   int64_t num_chunks;
   const int32_t* chunk_row;
   const int32_t* chunk_start;

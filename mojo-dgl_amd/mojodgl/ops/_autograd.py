@@ -197,7 +197,7 @@ class GSpMM(torch.autograd.Function):
                 # operand is constant over trailing groups of x (attention)
                 from .spmm import _mul_sum_dot
 
-                fused = _mul_sum_dot(g, G, y, x) if _trailing_groups(x, y) else None
+                fused = _mul_sum_dot(g, G, y, x, min_run=1) if _trailing_groups(x, y) else None
                 if fused is not None:
                     return None, None, None, _back(fused[0], x0), _back(fused[1], y0), None
             if need_x:

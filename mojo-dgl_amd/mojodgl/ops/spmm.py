@@ -36,7 +36,7 @@ _LANES = {}
 
 def _lanes(code, dl, dr, dout, sp, lhs, rhs, flags, dtype):
     """(packed, slabs) of the lane layout mdgl_gspmm picks for these operands
-    and flags (mdgl_gspmm_lanes): whether several rows share a wavefront
+    and flags (mdgl_gspmm_layout): whether several rows share a wavefront
     (slabs of 32 lanes or fewer) and how many column slabs a row is cut
     into. `sp` is shape_ptrs' entry for the operands' feature shapes (None
     for the copy ops). The answer depends only on the sizes, shapes, flags,
@@ -54,13 +54,13 @@ def _lanes(code, dl, dr, dout, sp, lhs, rhs, flags, dtype):
 
 
 def _lanes_query(code, dl, dr, dout, sp, lhs, rhs, flags, dtype):
-    vec, group = ctypes.c_int64(), ctypes.c_int64()
+    vec, group, lanes = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64()
     nd, lsp, rsp = (0, None, None) if sp is None else (sp[0], sp[3], sp[4])
-    _lib.check(_lib.lib().mdgl_gspmm_lanes(
+    _lib.check(_lib.lib().mdgl_gspmm_layout(
         code, dl, dr, dout, nd, lsp, rsp, _lib.ptr(lhs), _lib.ptr(rhs), flags,
-        _lib.dtype_code(dtype), ctypes.byref(vec), ctypes.byref(group)), "gspmm_lanes")
-    lanes = -(-dout // vec.value)
-    return group.value <= 32, -(-lanes // group.value)
+        _lib.dtype_code(dtype), ctypes.byref(vec), ctypes.byref(group), ctypes.byref(lanes)),
+        "gspmm_layout")
+    return group.value <= 32, -(-lanes.value // group.value)
 
 
 def _line_rows_pay(rows, dl, num_edges, dtype):
@@ -245,7 +245,7 @@ def _run(g, op, reduce_op, lhs_data, rhs_data, replace_inf=False, want_arg=False
         lhs = _lib.on_device(L, dtype) if L is not None else None
         rhs = _lib.on_device(R, dtype) if R is not None else None
         csr = g._device_csr(kind)
-        flags = _lib.REPLACE_INF if replace_inf else 0
+        flags = _lib.ANY_ALIGNMENT | (_lib.REPLACE_INF if replace_inf else 0)
         replay = key is not None
         if rows is not None:
             # the layout choices below pay over whole graphs, not a few rows
@@ -344,12 +344,15 @@ def _run_rows(csr, rows, code, reduce_op, lhs, rhs, out, arg_u, arg_e, dl, dr, d
     return out, arg_u, arg_e, as_torch, dev
 
 
-def _mul_sum_dot(g, grad, y, x, kind="out"):
+def _mul_sum_dot(g, grad, y, x, kind="out", min_run=7):
     """Both gradients of a u_mul_e_sum whose edge operand `y` is constant
     over trailing groups of the node operand `x`, in one pass over the `kind`
     CSR (mdgl_gspmm_mul_sum_dot): returns (dx, dy) as GPU tensors shaped like
     x and y, or None when the shapes do not fit the fused kernel (the caller
-    then runs gspmm and gsddmm)."""
+    then runs gspmm and gsddmm). `min_run`: other runs (columns per value of
+    `y`) than 2 and 4 of fewer columns are left to those too; the backward
+    passes take every run the kernel does (on 6M edges, 4 heads of 5, 9 or 12
+    columns: 448, 461, 470 us against 1,078, 1,971, 775 us separately)."""
     G = grad.contiguous()
     X = x.contiguous()
     # y as (E, *x's leading feature axes, 1): the same rank as the node rows
@@ -367,6 +370,8 @@ def _mul_sum_dot(g, grad, y, x, kind="out"):
         return None
     if E == 0:  # no messages: both gradients are zero
         return torch.zeros_like(x), torch.zeros_like(y)
+    if dout // dr < min_run and dout // dr not in (2, 4):
+        return None
     csr = g._device_csr(kind)
     sched = csr.chunks
     gdev = _lib.device()
@@ -375,12 +380,13 @@ def _mul_sum_dot(g, grad, y, x, kind="out"):
     nbytes = _lib.lib().mdgl_gspmm_workspace_bytes(sched.num_chunks, dout, REDUCERS["sum"],
                                                      _lib.dtype_code(dtype))
     ws = torch.empty(nbytes, dtype=torch.uint8, device=gdev) if nbytes else None
-    rc = _lib.lib().mdgl_gspmm_mul_sum_dot(
+    rc = _lib.lib().mdgl_gspmm_mul_sum_dot_any(
         csr.indptr.data_ptr(), csr.indices.data_ptr(), csr.eid.data_ptr(), G.data_ptr(),
         Y.data_ptr(), X.data_ptr(), dx.data_ptr(), dot.data_ptr(), num_rows, dout, dr, dout, nd,
         lsp, rsp, _lib.ptr(sched.chunk_row), _lib.ptr(sched.chunk_start),
         sched.num_chunks, sched.chunk_len, _lib.ptr(sched.heavy_rows), _lib.ptr(sched.heavy_ptr),
-        sched.num_heavy, _lib.ptr(ws), nbytes, _lib.dtype_code(dtype), _lib.stream())
+        sched.num_heavy, _lib.ptr(ws), nbytes, _lib.ANY_ALIGNMENT, _lib.dtype_code(dtype),
+        _lib.stream())
     if rc == _lib.ENOTSUP:
         return None
     _lib.check(rc, "gspmm_mul_sum_dot")

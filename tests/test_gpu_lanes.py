@@ -1,0 +1,137 @@
+"""gspmm's lane layouts at the widths where they can go wrong: runs of columns
+that no lane width divides (their last lane shares columns with the one before
+it), one to 64 lanes per row and several slabs, rows that end inside, at and
+just past a batch of ids, misaligned operands and results; and the fused
+backward pass of attention over runs of any length. Sums fold in the oracle's
+order, so whole rows are equal bit for bit."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import mojodgl as dgl
+import mojodgl.ops as ops
+import oracle
+from mojodgl import _lib
+
+# 1 to 64 lanes of 4, 2 or 1 columns, remainders on both sides, 2 to 5 slabs
+WIDTHS = [1, 2, 3, 4, 5, 7, 9, 15, 16, 17, 31, 33, 47, 63, 66, 97, 127, 130, 255, 257, 258, 515]
+
+
+def ragged_graph(seed, n=160, most=40):
+    """In-degrees 0, 1, 2, ... `most`, then random, and a hub of 700."""
+    rng = np.random.default_rng(seed)
+    deg = np.concatenate([np.arange(most + 1), rng.integers(0, most, n - most - 2), [700]])
+    v = np.repeat(np.arange(n), deg)
+    v = v[rng.permutation(v.size)]
+    return rng.integers(0, n, v.size), v, n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("d", WIDTHS)
+def test_any_width(dtype, d, monkeypatch):
+    """copy, a weight per edge and an edge row per edge, sum / mean / max /
+    min with args, operands one element off a 16-byte boundary, against the
+    oracle bit for bit (no row split)."""
+    from mojodgl import heterograph
+
+    monkeypatch.setattr(heterograph, "CHUNK_LEN", 1 << 20)
+    u, v, n = ragged_graph(d)
+    rng = np.random.default_rng(d + 1)
+    g = dgl.graph((u, v), num_nodes=n)
+
+    def off(a):  # a GPU copy that starts one element into its buffer
+        buf = torch.empty(a.size + 1, dtype=torch.from_numpy(a).dtype, device="cuda")
+        view = buf[1:].view(a.shape)
+        view.copy_(torch.from_numpy(a))
+        return view
+
+    x = rng.normal(size=(n, d)).astype(dtype)
+    for op, y in (("copy_lhs", None), ("mul", (rng.random((u.size, 1)) + 0.5).astype(dtype)),
+                  ("add", rng.normal(size=(u.size, d)).astype(dtype))):
+        for red in ("sum", "mean", "max", "min"):
+            got, (au, ae) = ops.spmm._gspmm(g, op, red, off(x), None if y is None else off(y))
+            what = "{} {} d={}".format(op, red, d)
+            if red in ("max", "min"):
+                want, ru, re_ = oracle.gspmm(u, v, n, op, red, x, y, dtype, with_arg=True)
+                np.testing.assert_array_equal(au.cpu().numpy(), ru, err_msg=what)
+                np.testing.assert_array_equal(ae.cpu().numpy(), re_, err_msg=what)
+            else:
+                want = oracle.gspmm(u, v, n, op, red, x, y, dtype)
+            np.testing.assert_array_equal(got.cpu().numpy(), want, err_msg=what)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("heads,d", [(1, 7), (2, 5), (8, 25), (3, 10), (6, 7), (4, 3), (5, 2),
+                                     (3, 33), (2, 130)])
+def test_heads_of_any_width(dtype, heads, d):
+    """One weight per head: no lane straddles two heads. The same graph split
+    into chunks of 16 slots folds in another order (within tolerance)."""
+    u, v, n = ragged_graph(heads * 100 + d)
+    rng = np.random.default_rng(d)
+    x = rng.normal(size=(n, heads, d)).astype(dtype)
+    y = rng.normal(size=(u.size, heads, 1)).astype(dtype)
+    keep = v != n - 1  # without the hub no row is split
+    g = dgl.graph((u[keep], v[keep]), num_nodes=n)
+    np.testing.assert_array_equal(
+        ops.u_mul_e_sum(g, x, y[keep]),
+        oracle.gspmm(u[keep], v[keep], n, "mul", "sum", x, y[keep], dtype))
+    g = dgl.graph((u, v), num_nodes=n)
+    from mojodgl.ops import spmm
+
+    got = spmm._run(g, "mul", "sum", torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda(),
+                    narrow_split=16)[0].cpu().numpy()
+    ref = oracle.gspmm(u, v, n, "mul", "sum", x, y, np.float64)
+    bound = oracle.gspmm(u, v, n, "mul", "sum", np.abs(x), np.abs(y), np.float64)
+    # a sum of k terms in another order: at most k * eps of the terms' magnitudes
+    assert (np.abs(got - ref) <= 700 * np.finfo(dtype).eps * bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("heads,d", [(1, 7), (8, 7), (4, 25), (3, 10), (2, 100), (1, 126),
+                                     (8, 33)])
+def test_fused_dot_over_any_run(dtype, heads, d):
+    """Both gradients of u_mul_e_sum in one pass, runs that no power of two of
+    lanes covers exactly: dX equals the separate gspmm bit for bit, dY the
+    separate dot to rounding (a sum of d products: d * eps of their
+    magnitudes)."""
+    from mojodgl.ops import spmm
+
+    u, v, n = ragged_graph(7 * heads + d)
+    g = dgl.graph((u, v), num_nodes=n)
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    G = torch.randn(n, heads, d, device="cuda", generator=gen, dtype=torch.float64).to(dtype)
+    X = torch.randn(n, heads, d, device="cuda", generator=gen, dtype=torch.float64).to(dtype)
+    Y = torch.randn(u.size, heads, 1, device="cuda", generator=gen, dtype=torch.float64).to(dtype)
+    fused = spmm._mul_sum_dot(g, G, Y, X)
+    assert fused is not None
+    dx = spmm._run(g, "mul", "sum", G, Y, kind="out")[0]
+    assert torch.equal(fused[0], dx.reshape(X.shape))
+    ud, vd = torch.from_numpy(u).cuda(), torch.from_numpy(v).cuda()
+    t = X.double()[ud] * G.double()[vd]
+    off = (fused[1].double() - t.sum(-1, keepdim=True)).abs()
+    assert bool((off <= 2 * d * torch.finfo(dtype).eps * t.abs().sum(-1, keepdim=True)).all())
+
+
+def test_layout_covers_every_column():
+    """mdgl_gspmm_layout with any alignment allowed: lanes of `vec` columns,
+    enough of them for every run, at most 64 to a slab (no launch)."""
+    lib = _lib.lib()
+    for dt in (0, 1):
+        for heads, d in [(1, w) for w in WIDTHS] + [(8, 25), (4, 3), (6, 7), (3, 130)]:
+            vec, group, lanes = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64()
+            ls, rs = (ctypes.c_int64 * 2)(heads, d), (ctypes.c_int64 * 2)(heads, 1)
+            rc = lib.mdgl_gspmm_layout(_lib.BINARY_OPS["mul"], heads * d, heads, heads * d, 2, ls,
+                                       rs, 4, 4, _lib.ANY_ALIGNMENT, dt, ctypes.byref(vec),
+                                       ctypes.byref(group), ctypes.byref(lanes))
+            assert rc == 0
+            run = d if heads > 1 or d > 1 else 1
+            assert vec.value <= max(run, 1) and lanes.value * vec.value >= heads * d
+            assert lanes.value == heads * -(-run // vec.value)
+            assert group.value in (16, 32, 64)
+            assert group.value >= min(lanes.value, 64)
