@@ -209,6 +209,19 @@ int mdgl_gspmm_layout(int op, int64_t dl, int64_t dr, int64_t dout, int nd,
 int mdgl_coo_locality(const int32_t* u, const int32_t* v, int64_t num_edges, int64_t window,
                       int64_t* partial, void* stream);
 
+/* dst[r] = sum over r's CSR slots i, in order, of lhs[indices[i]][k] where
+ * sel[indices[i]][k] == eid[i] (0 elsewhere): over the out-CSR, with sel the
+ * arg_e of a max or min gspmm and lhs the gradient of its result, the gradient
+ * of its node operand (copy_lhs, add, sub). sel: int32, one per element of
+ * lhs. Schedule, workspace and flags (MDGL_ANY_ALIGNMENT) as for mdgl_gspmm
+ * with sum. No counterpart in the reference (it has no backward). */
+int mdgl_gspmm_selected_sum(const int32_t* indptr, const int32_t* indices, const int32_t* eid,
+                            const void* lhs, const int32_t* sel, void* dst, int64_t num_dst,
+                            int64_t d, const int32_t* chunk_row, const int32_t* chunk_start,
+                            int64_t num_chunks, int32_t chunk_len, const int32_t* heavy_rows,
+                            const int32_t* heavy_ptr, int64_t num_heavy, void* workspace,
+                            int64_t workspace_bytes, int flags, int dtype, void* stream);
+
 /* Workspace mdgl_gspmm needs for `num_chunks` chunk partials. */
 int64_t mdgl_gspmm_workspace_bytes(int64_t num_chunks, int64_t dout, int reduce_op, int dtype);
 

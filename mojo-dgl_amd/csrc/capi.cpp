@@ -631,7 +631,8 @@ int gspmm_common(const int32_t* indptr, const int32_t* indices, const int32_t* e
                  const int32_t* heavy_ptr, int64_t num_heavy, void* workspace,
                  int64_t workspace_bytes, int flags, int dtype, void* stream,
                  const void* rowop = nullptr, void* dot_out = nullptr,
-                 const int32_t* rows = nullptr, int64_t num_listed = -1) {
+                 const int32_t* rows = nullptr, int64_t num_listed = -1,
+                 const int32_t* sel = nullptr) {
   if (!dtype_ok(dtype)) return fail(MDGL_EINVAL, "gspmm: bad dtype %d", dtype);
   if (op < OP_ADD || op > OP_COPY_RHS || op == OP_DOT)
     return fail(MDGL_EINVAL, "gspmm: bad op %d (dot is a gsddmm operator)", op);
@@ -661,6 +662,7 @@ int gspmm_common(const int32_t* indptr, const int32_t* indices, const int32_t* e
   p.rhs = rhs;
   p.out = dst;
   p.num_rows = num_dst;
+  p.sel = sel;
   p.dl = dl;
   p.lstride = dl;
   p.dr = dr;
@@ -785,6 +787,23 @@ int mdgl_gspmm(const int32_t* indptr, const int32_t* indices, const int32_t* eid
                       deg, nd, lhs_shape, rhs_shape, arg_u, arg_e, chunk_row, chunk_start,
                       num_chunks, chunk_len, heavy_rows, heavy_ptr, num_heavy, workspace,
                       workspace_bytes, flags, dtype, stream);
+}
+
+int mdgl_gspmm_selected_sum(const int32_t* indptr, const int32_t* indices, const int32_t* eid,
+                            const void* lhs, const int32_t* sel, void* dst, int64_t num_dst,
+                            int64_t d, const int32_t* chunk_row, const int32_t* chunk_start,
+                            int64_t num_chunks, int32_t chunk_len, const int32_t* heavy_rows,
+                            const int32_t* heavy_ptr, int64_t num_heavy, void* workspace,
+                            int64_t workspace_bytes, int flags, int dtype, void* stream) {
+  MDGL_RANGE();
+  if (num_dst > 0 && d > 0 && (!sel || !eid))
+    return fail(MDGL_EINVAL, "gspmm_selected_sum: null selection or eid");
+  if (flags & ~MDGL_ANY_ALIGNMENT) return fail(MDGL_EINVAL, "gspmm_selected_sum: bad flags");
+  return gspmm_common(indptr, indices, eid, lhs, nullptr, dst, num_dst, OP_COPY_LHS, d, d, d,
+                      RED_SUM, nullptr, 0, nullptr, nullptr, nullptr, nullptr, chunk_row,
+                      chunk_start, num_chunks, chunk_len, heavy_rows, heavy_ptr, num_heavy,
+                      workspace, workspace_bytes, flags, dtype, stream, nullptr, nullptr, nullptr,
+                      -1, sel);
 }
 
 int mdgl_gspmm_rows(const int32_t* indptr, const int32_t* indices, const int32_t* eid,

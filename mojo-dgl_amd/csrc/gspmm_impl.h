@@ -86,6 +86,7 @@ struct GspmmArgs {
   // waves per slab (with several, every unit's slab s comes before slab s + 1,
   // so the rows of neighbouring units share cache lines across wavefronts)
   int64_t chunk_uwaves, row_uwaves;
+  const int32_t* sel;  // selected sum (see GspmmParams), else null
   const T* rowop;  // dot output (see GspmmParams), else null
   T* dot_out;
   int dot_lanes;
@@ -209,7 +210,8 @@ __device__ __forceinline__ void for_each(F f) {
 // How ids reach the lanes of a unit (see the top): by G.
 enum { LAY_ROW = 0, LAY_WIDE = 1 };
 
-template <class T, int OP, int RED, int VEC, int LM, int RM, int LAY, bool DOT = false>
+template <class T, int OP, int RED, int VEC, int LM, int RM, int LAY, bool DOT = false,
+          bool SEL = false>
 __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, int64_t wave,
                                            int lane) {
   // edges in flight per lane: 8 (4 in the dot pass, whose per-edge
@@ -303,10 +305,12 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
   constexpr bool ROW_R = HAS_R && !SCALAR;
   // the edge operand may come in CSR slot order (row i of rhs for slot i)
   const bool rhs_csr = a.flags & F_RHS_CSR;
-  const bool need_e = HAS_R && !rhs_csr && !ident;
+  const bool need_e = SEL || (HAS_R && !rhs_csr && !ident);
 
   const char* const lbase = reinterpret_cast<const char*>(a.lhs + loff[0]);
   const char* const rbase = reinterpret_cast<const char*>(a.rhs + roff[0]);
+  // SEL: the selection's rows lie as the lhs rows do (int32, dl == dout)
+  const char* const sbase = reinterpret_cast<const char*>(a.sel + (SEL ? k0 : 0));
 #pragma unroll
   for (int v = VEC - 1; v >= 0; --v) {  // from here on relative to the lane's first column
     loff[v] -= loff[0];
@@ -316,31 +320,40 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
   // One batch is the edges of U slots, of which the first `rem` are the
   // unit's (all U with FULL: no branch per edge). `lo_of` / `ro_of` give the
   // byte offset of edge u's operand rows, `w_of` its value of a scalar edge
-  // operand, `after` runs between the requests and the folds. A broadcast right
+  // operand, `e_of` its edge id (SEL only). A broadcast right
   // before its request keeps one offset live instead of U of them (32
   // registers, and with them two wavefronts per SIMD).
   auto batch = [&](auto full, int slot0, int rem, auto lo_of, auto ro_of, auto w_of,
-                   auto after) MDGL_INLINE {
+                   auto e_of) MDGL_INLINE {
     constexpr bool FULL = decltype(full)::value;
     T x[U][VEC], y[U][VEC], w[U];
+    int32_t sel[U][VEC];
     auto request = [&](auto iu) MDGL_INLINE {
       constexpr int u = decltype(iu)::value;
-      if constexpr (HAS_L)
-        fetch<T, VEC, LM, false>(reinterpret_cast<const T*>(lbase + lo_of(iu)), a.lmode, loff,
-                                 x[u]);
+      if constexpr (HAS_L) {
+        const int64_t lo = lo_of(iu);
+        fetch<T, VEC, LM, false>(reinterpret_cast<const T*>(lbase + lo), a.lmode, loff, x[u]);
+        if constexpr (SEL)
+          load_any<int32_t, VEC>(
+              reinterpret_cast<const int32_t*>(sbase + lo / (int64_t)(sizeof(T) / 4)), sel[u],
+              false);
+      }
       if constexpr (ROW_R)
         fetch<T, VEC, RM, true>(reinterpret_cast<const T*>(rbase + ro_of(iu)), a.rmode, roff,
                                 y[u]);
     };
     auto fold = [&](auto iu) MDGL_INLINE {
       constexpr int u = decltype(iu)::value;
+      int eid = 0;
+      if constexpr (SEL) eid = e_of(iu);
 #pragma unroll
       for (int v = 0; v < VEC; ++v) {
         T xv = T(0), yv = T(0);
         if constexpr (HAS_L) xv = x[u][v];
         if constexpr (SCALAR) yv = w[u];
         else if constexpr (HAS_R) yv = y[u][v];
-        const T m = message<OP>(xv, yv);
+        T m = message<OP>(xv, yv);
+        if constexpr (SEL) m = sel[u][v] == eid ? m : T(0);
         if constexpr (RED == RED_MAX) {
           if (m > acc[v]) { acc[v] = m; at[v] = slot0 + u; }
         } else if constexpr (RED == RED_MIN) {
@@ -364,7 +377,6 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
     for_each<U>([&](auto iu) MDGL_INLINE {
       if (FULL || decltype(iu)::value < rem) request(iu);
     });
-    after();
     if constexpr (SCALAR)
       for_each<U>([&](auto iu) MDGL_INLINE { w[decltype(iu)::value] = w_of(iu); });
     if constexpr (DOT)
@@ -387,7 +399,7 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
       const int p = base + (lane & 15);
       const int i = n > 0 ? start + (p < n ? p : n - 1) : 0;
       if constexpr (HAS_L) my_s = a.indices[i];
-      if constexpr (HAS_R) {
+      if constexpr (HAS_R || SEL) {
         my_e = i;
         if (need_e) my_e = a.eid[i];
       }
@@ -396,6 +408,7 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
     for (int base = 0; base < nmax; base += 16) {
       int64_t my_lo = 0, my_ro = 0;
       T my_w = T(0);
+      const int cur_e = my_e;
       if constexpr (HAS_L) my_lo = (int64_t)my_s * lbytes;
       if constexpr (SCALAR) my_w = a.rhs[my_e];
       else if constexpr (HAS_R) my_ro = (int64_t)my_e * rbytes;
@@ -407,10 +420,11 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
         auto lo_of = [&](auto iu) MDGL_INLINE { return row_bcast<F + decltype(iu)::value>(my_lo); };
         auto ro_of = [&](auto iu) MDGL_INLINE { return row_bcast<F + decltype(iu)::value>(my_ro); };
         auto w_of = [&](auto iu) MDGL_INLINE { return row_bcast<F + decltype(iu)::value>(my_w); };
+        auto e_of = [&](auto iu) MDGL_INLINE { return row_bcast<F + decltype(iu)::value>(cur_e); };
         if (rem >= U)
-          batch(std::true_type{}, start + base + F, U, lo_of, ro_of, w_of, [] {});
+          batch(std::true_type{}, start + base + F, U, lo_of, ro_of, w_of, e_of);
         else
-          batch(std::false_type{}, start + base + F, rem, lo_of, ro_of, w_of, [] {});
+          batch(std::false_type{}, start + base + F, rem, lo_of, ro_of, w_of, e_of);
       });
     }
   } else {
@@ -422,7 +436,7 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
       const int p = base + lane;
       const int i = ustart + (p < un ? p : un - 1);
       if constexpr (HAS_L) my_s = __builtin_nontemporal_load(a.indices + i);
-      if constexpr (HAS_R) {
+      if constexpr (HAS_R || SEL) {
         my_e = i;
         if (need_e) my_e = __builtin_nontemporal_load(a.eid + i);
       }
@@ -444,10 +458,11 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
         auto w_of = [&](auto iu) MDGL_INLINE {
           return readlane_val(my_w, (j + decltype(iu)::value) & (WAVE - 1));
         };
+        auto e_of = [&](auto iu) MDGL_INLINE { return readlane_int(ce, j + decltype(iu)::value); };
         if (cnt - j >= U)
-          batch(std::true_type{}, ustart + base + j, U, lo_of, ro_of, w_of, [] {});
+          batch(std::true_type{}, ustart + base + j, U, lo_of, ro_of, w_of, e_of);
         else
-          batch(std::false_type{}, ustart + base + j, cnt - j, lo_of, ro_of, w_of, [] {});
+          batch(std::false_type{}, ustart + base + j, cnt - j, lo_of, ro_of, w_of, e_of);
       }
     }
   }
@@ -499,7 +514,10 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
 // edge), or any modes. The scalar one is loaded with the ids and broadcast like
 // them: read per lane and edge through the any-modes path it cost a GCN
 // aggregation over 128 columns 4x the time of the same gather without it.
-enum { P_CC = 0, P_CS = 1, P_DYN = 2, P_CS_DOT = 3, P_CW = 4 };
+// P_SEL (copy / sum) adds a gathered value only where the selection's entry is
+// the edge itself: the gradient of a max or min without a tensor of per-edge
+// gradients in between.
+enum { P_CC = 0, P_CS = 1, P_DYN = 2, P_CS_DOT = 3, P_CW = 4, P_SEL = 5 };
 
 // Wavefronts per SIMD asked of the register allocation: what each path needs
 // plus a few registers would otherwise round down to one wavefront less (98
@@ -509,6 +527,7 @@ enum { P_CC = 0, P_CS = 1, P_DYN = 2, P_CS_DOT = 3, P_CW = 4 };
 // would spill.
 constexpr int gspmm_waves(int op, int red, int path, int lay, int vec, int size) {
   if (red != RED_SUM || op == OP_DIV || path == P_DYN || vec * size > 16) return 1;
+  if (path == P_SEL) return size == 8 ? 4 : 5;
   if (path == P_CC && op != OP_COPY_LHS && op != OP_COPY_RHS) return lay == LAY_WIDE ? 6 : 5;
   return size == 8 ? 6 : 7;
 }
@@ -531,6 +550,8 @@ gspmm_kernel(GspmmArgs<T> a) {
     gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SPLAT, LAY>(a, chunk, wave, lane);
   else if constexpr (PATH == P_CW)
     gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SCALAR, LAY>(a, chunk, wave, lane);
+  else if constexpr (PATH == P_SEL)
+    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_CONTIG, LAY, false, true>(a, chunk, wave, lane);
   else if constexpr (PATH == P_CS_DOT)
     gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SPLAT, LAY, true>(a, chunk, wave, lane);
   else
@@ -600,6 +621,12 @@ __global__ __launch_bounds__(BLOCK) void gspmm_combine_kernel(
 
 template <class T, int OP, int RED, int VEC, int LAY>
 void launch_path(const GspmmArgs<T>& a, dim3 grid, dim3 block, int lm, int rm, hipStream_t st) {
+  if constexpr (OP == OP_COPY_LHS && RED == RED_SUM) {
+    if (a.sel) {
+      hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_SEL, LAY>), grid, block, 0, st, a);
+      return;
+    }
+  }
   if constexpr (OP == OP_COPY_LHS || OP == OP_COPY_RHS)
     hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CC, LAY>), grid, block, 0, st, a);
   else if (lm == M_CONTIG && rm == M_CONTIG)
@@ -655,6 +682,7 @@ hipError_t launch_gspmm_op(const GspmmParams& p) {
   a.row_waves = a.row_uwaves * a.S;
   a.chunk_blocks = (a.chunk_waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
   a.num_blocks = a.chunk_blocks + (a.row_waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+  a.sel = p.sel;
   a.rowop = static_cast<const T*>(p.rowop);
   a.dot_out = static_cast<T*>(p.dot_out);
   a.dot_lanes = p.dot_lanes;

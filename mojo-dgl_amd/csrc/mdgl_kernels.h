@@ -56,6 +56,9 @@ struct GspmmParams {
   const void* rowop;
   void* dot_out;
   int dot_lanes;
+  // optional (copy_lhs / sum): an int32 per element of lhs; a value is added
+  // for slot i only where sel[indices[i]][k] == eid[i]
+  const int32_t* sel;
   // optional: the rows to reduce (num_rows of them, each in [0, row_limit));
   // null: rows 0 .. num_rows - 1
   const int32_t* rows;

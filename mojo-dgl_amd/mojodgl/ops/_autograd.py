@@ -16,8 +16,10 @@ these follow the calculus of the forward ops and run on the same kernels:
     its negation for sub, X[u] * G[v] for mul -- a per-head dot when Y
     broadcasts over X's trailing axes --, -X[u] G[v] / Y[e]^2 for div);
   - max / min: only the arg edge of an output element receives its
-    gradient: ``mdgl_gspmm_edge_grad`` writes the masked per-edge gradient M,
-    then dX is a gspmm over the out-CSR of M (times d msg / dX) and dY is M
+    gradient: when only dX of copy_lhs / add / sub is asked for,
+    ``mdgl_gspmm_selected_sum`` sums G[v] over u's out-edges where they are
+    the arg edge; otherwise ``mdgl_gspmm_edge_grad`` writes the masked per-edge
+    gradient M, then dX is a gspmm over the out-CSR of M (times d msg / dX) and dY is M
     times d msg / dY, per edge;
 * gsddmm(op, X at target tx, Y at target ty): the per-edge gradient times
   d op / dX (dY) is reduced over the edges of each node of the operand's
@@ -172,7 +174,7 @@ class GSpMM(torch.autograd.Function):
         from .spmm import _run
 
         out, _, arg_e, _, dev = _run(g, op, red, x, y, replace_inf=replace_inf,
-                                     want_arg=red in ("max", "min"), arg_dtype=torch.int32)
+                                     want_arg="e", arg_dtype=torch.int32)
         ctx.g, ctx.op, ctx.red = g, op, red
         ctx.save_for_backward(x if isinstance(x, torch.Tensor) else None,
                               y if isinstance(y, torch.Tensor) else None, arg_e)
@@ -223,7 +225,19 @@ class GSpMM(torch.autograd.Function):
             # gradient (none where nothing was selected or update_all replaced
             # an infinite value: the kernel's arg is -1 there); the terms of
             # the other edges are exactly zero, not 0 times their operand
-            M = _edge_grad(g, G, arg_e, False, 1.0)
+            M = None
+            if need_x and not need_y and op in ("copy_lhs", "add", "sub") \
+                    and arg_e.is_contiguous():
+                # only the node operand: the selected gradients summed over the
+                # out-CSR without the per-edge tensor (two rows read per edge
+                # instead of three and one written)
+                from .spmm import _selected_sum
+
+                dx = _reduce_to(_selected_sum(g, G, arg_e, NARROW_SPLIT),
+                                _padded(x.shape, G.shape))
+                need_x = False
+            elif need_x or need_y:
+                M = _edge_grad(g, G, arg_e, False, 1.0)
             if need_x:
                 if op in ("copy_lhs", "add", "sub"):
                     p = M

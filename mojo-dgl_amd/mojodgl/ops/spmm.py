@@ -120,10 +120,11 @@ class _Launch:
         args[_A_OUT] = out.data_ptr()
         arg_u = arg_e = None
         if self.arg:
-            arg_u = torch.empty(self.shape, dtype=torch.int32, device=gdev)
             arg_e = torch.empty(self.shape, dtype=torch.int32, device=gdev)
-            args[_A_ARG_U] = arg_u.data_ptr()
             args[_A_ARG_E] = arg_e.data_ptr()
+            if self.arg != "e":
+                arg_u = torch.empty(self.shape, dtype=torch.int32, device=gdev)
+                args[_A_ARG_U] = arg_u.data_ptr()
         ws = None
         if self.nbytes:
             ws = torch.empty(self.nbytes, dtype=torch.uint8, device=gdev)
@@ -131,7 +132,7 @@ class _Launch:
         args[_A_STREAM] = _lib.stream()
         _lib.check(_lib.lib().mdgl_gspmm(*args), "gspmm")
         if self.arg:
-            arg_u = arg_u.to(self.arg_dtype)
+            arg_u = None if arg_u is None else arg_u.to(self.arg_dtype)
             arg_e = arg_e.to(self.arg_dtype)
         return out, arg_u, arg_e, True, self.dev
 
@@ -170,7 +171,7 @@ def _launch_key(op, reduce_op, lhs, rhs, replace_inf, want_arg, arg_dtype, kind,
 def _run(g, op, reduce_op, lhs_data, rhs_data, replace_inf=False, want_arg=False,
          arg_dtype=torch.int64, kind="in", narrow_split=None, rows=None):
     """Validate, launch, and return device tensors (out, arg_u, arg_e) plus
-    the caller-container info. `kind` "out" reduces over the out-CSR instead
+    the caller-container info. `want_arg` "e" leaves arg_u out (None). `kind` "out" reduces over the out-CSR instead
     (the reversed graph: rows are sources, the node operand is read at the
     destinations), which the backward passes use. `narrow_split`: when
     several rows share a wavefront, split rows longer than this (instead of
@@ -226,10 +227,10 @@ def _run(g, op, reduce_op, lhs_data, rhs_data, replace_inf=False, want_arg=False
     tdt = _lib.torch_dtype(dtype)
     dcode = _lib.dtype_code(dtype)
     gdev = _lib.device()
-    arg = want_arg and reduce_op in ("max", "min")
+    arg = want_arg if reduce_op in ("max", "min") else False
     if rows is None:
         out = torch.empty(shape, dtype=tdt, device=gdev)
-        arg_u = torch.empty(shape, dtype=torch.int32, device=gdev) if arg else None
+        arg_u = torch.empty(shape, dtype=torch.int32, device=gdev) if arg is True else None
         arg_e = torch.empty(shape, dtype=torch.int32, device=gdev) if arg else None
     else:  # the rows that are not listed stay zero (no message: arg -1)
         out = torch.zeros(shape, dtype=tdt, device=gdev)
@@ -313,7 +314,7 @@ def _run(g, op, reduce_op, lhs_data, rhs_data, replace_inf=False, want_arg=False
                 g._launches.clear()
             g._launches[key] = launch
     if arg:
-        arg_u = arg_u.to(arg_dtype)
+        arg_u = None if arg_u is None else arg_u.to(arg_dtype)
         arg_e = arg_e.to(arg_dtype)
     return out, arg_u, arg_e, as_torch, dev
 
@@ -397,6 +398,36 @@ def _mul_sum_dot(g, grad, y, x, kind="out", min_run=7):
                                                dy.data_ptr(), E, dr, _lib.dtype_code(dtype),
                                                _lib.stream()), "gather_rows")
     return dx.reshape(x.shape), dy.reshape(y.shape)
+
+
+def _selected_sum(g, grad, arg_e, chunk_len):
+    """Sum over each node's out-edges e = (u, v) of grad[v] where arg_e[v] == e
+    (mdgl_gspmm_selected_sum), shaped like `grad`; rows of more than
+    `chunk_len` edges fold in chunks when several share a wavefront, like the
+    other reductions of the backward passes."""
+    num_rows, d = grad.shape[0], width(grad.shape)
+    E = g.number_of_edges()
+    out = torch.empty_like(grad)
+    if num_rows == 0 or d == 0:
+        return out
+    if E == 0:  # no messages: nothing was selected
+        return out.zero_()
+    csr = g._device_csr("out")
+    dtype = np.dtype(np.float32 if grad.dtype == torch.float32 else np.float64)
+    code = _lib.dtype_code(dtype)
+    packed, _ = _lanes(OP_COPY_LHS, d, d, d, None, grad, None, _lib.ANY_ALIGNMENT, dtype)
+    sched = csr.chunks
+    if packed and chunk_len < sched.chunk_len:
+        sched = csr.chunks_for(chunk_len)
+    nbytes = _lib.lib().mdgl_gspmm_workspace_bytes(sched.num_chunks, d, REDUCERS["sum"], code)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=grad.device) if nbytes else None
+    _lib.check(_lib.lib().mdgl_gspmm_selected_sum(
+        csr.indptr.data_ptr(), csr.indices.data_ptr(), csr.eid.data_ptr(), grad.data_ptr(),
+        arg_e.data_ptr(), out.data_ptr(), num_rows, d, _lib.ptr(sched.chunk_row),
+        _lib.ptr(sched.chunk_start), sched.num_chunks, sched.chunk_len,
+        _lib.ptr(sched.heavy_rows), _lib.ptr(sched.heavy_ptr), sched.num_heavy, _lib.ptr(ws),
+        nbytes, _lib.ANY_ALIGNMENT, code, _lib.stream()), "gspmm_selected_sum")
+    return out
 
 
 def gspmm(g, op, reduce_op, lhs_data, rhs_data):

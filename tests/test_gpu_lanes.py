@@ -135,3 +135,38 @@ def test_layout_covers_every_column():
             assert lanes.value == heads * -(-run // vec.value)
             assert group.value in (16, 32, 64)
             assert group.value >= min(lanes.value, 64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("d", [1, 3, 16, 47, 100, 130, 258])
+@pytest.mark.parametrize("op", ["copy_lhs", "add", "sub"])
+def test_selected_sum_is_the_max_gradient(dtype, d, op):
+    """The gradient of max / min in the node operand alone, without the
+    per-edge gradients: equal bit for bit to the path through them (taken when
+    the edge operand's gradient is asked for too), duplicate edges, equal
+    messages and nodes without edges among the inputs."""
+    u, v, n = ragged_graph(d + 5)
+    u = np.concatenate([u, u[:200]])  # the same edge twice: the first one wins
+    v = np.concatenate([v, v[:200]])
+    g = dgl.graph((u, v), num_nodes=n)
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    x = torch.randn(n, d, device="cuda", generator=gen, dtype=torch.float64).to(dtype)
+    x[:, 0] = torch.round(x[:, 0])  # equal messages
+    y = torch.randn(u.size, d, device="cuda", generator=gen, dtype=torch.float64).to(dtype)
+    G = torch.randn(n, d, device="cuda", generator=gen, dtype=torch.float64).to(dtype)
+    x.requires_grad_(True)
+    for red in ("max", "min"):
+        if op == "copy_lhs":
+            dx, = torch.autograd.grad(ops.gspmm(g, op, red, x, None), x, G)
+            with torch.no_grad():
+                _, (_, ae) = ops.spmm._gspmm(g, op, red, x.detach(), None)
+            from mojodgl.ops import _autograd
+
+            M = _autograd._edge_grad(g, G, ae, False, 1.0)
+            want = _autograd._node_reduce(g, M, "u")
+        else:
+            dx, = torch.autograd.grad(ops.gspmm(g, op, red, x, y), x, G)
+            yy = y.clone().requires_grad_(True)
+            want, _ = torch.autograd.grad(ops.gspmm(g, op, red, x, yy), (x, yy), G)
+        assert torch.equal(dx, want)
