@@ -7,10 +7,17 @@
 // gather_mm's are the rows with idx_b == g, found by a stable counting sort
 // on the GPU (count per block, scan, ballot-ranked scatter) into `perm`.
 //
-// Two forward kernels: float32 with K a multiple of 32 up to 128 and rows of
-// a on a 16-byte boundary runs on the bf16 matrix cores through exact
-// three-way splits (grouped_gemm_split_kernel, described where it is
-// defined); every other shape, and float64, takes grouped_gemm_kernel:
+// Forward kernels, each described where it is defined:
+//  * grouped_gemm_split_kernel: float32, K a multiple of 32 up to 128, rows of a
+//    on a 16-byte boundary, more than 64 columns: bf16 matrix cores through exact
+//    three-way splits, one b block of 128 columns per CU;
+//  * grouped_gemm_any_kernel: the same products for other float32 shapes with K
+//    of 4 to 256, in one, two or four blocks of 32 columns;
+//  * grouped_gemm_f64_kernel: float64, K a multiple of 16 up to 128, in two,
+//    four or eight blocks of 16 columns;
+//  * grouped_gemm_kernel: what is left.
+//
+// grouped_gemm_kernel:
 //
 // Tiles. A workgroup (4 wavefronts, 2 x 2) computes a 128 x 128 output tile
 // of one group: 128 rows of the group x 128 columns. Wavefront (wm, wn) owns
@@ -332,8 +339,24 @@ __device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& q0, uin
   q2 = bf16_pair(r0 - bf16_lo(q1), r1 - bf16_hi(q1));
 }
 
-// bt3[g][q][n][k] (bf16 bit patterns): part q of b[g][k][n] (of b[g][n][k]
-// with `given_t`), zero for k in [K, Kp). Workgroup (g, s) splits slice s of
+// The row element behind place kv of the 16-deep chunks, -1 for none: element
+// kv itself, except that the last 4-float piece of a row whose K is no multiple
+// of 4 is read from K - 4 on and gives only the elements no other piece does.
+__device__ __forceinline__ int64_t k_of(int64_t kv, int64_t K) {
+  const int64_t p4 = kv & ~int64_t(3);
+  if (p4 + 4 <= K) return kv;
+  if (p4 >= K) return -1;
+  const int64_t k = K - 4 + (kv & 3);
+  return k >= p4 ? k : -1;
+}
+
+// Wavefronts per SIMD that the registers of an instance allow.
+constexpr int any_waves(int nb, int km) {
+  return nb == 4 || nb * km > 256 ? 2 : (nb == 2 || km == 256 ? 3 : 5);
+}
+
+// bt3[g][q][n][k] (bf16 bit patterns): part q of b[g][k_of(k)][n] (of
+// b[g][n][k_of(k)] with `given_t`), zero where k_of gives none. Workgroup (g, s) splits slice s of
 // group g's N x Kp values and sets flags[g * slices + s] when the slice holds
 // a value off the fast path (its parts are left zero: the group's chunks all
 // take the float32 path).
@@ -350,8 +373,9 @@ static __global__ __launch_bounds__(BLOCK) void split_b_kernel(const float* __re
   int bad = 0;
   for (int64_t i = lo + threadIdx.x; i < hi; i += BLOCK) {
     const int64_t k = i % Kp, n = i / Kp;
+    const int64_t kr = k_of(k, K);
     float x = 0.f;
-    if (k < K) x = given_t ? b[(g * N + n) * K + k] : b[(g * K + k) * N + n];
+    if (kr >= 0) x = given_t ? b[(g * N + n) * K + kr] : b[(g * K + kr) * N + n];
     uint32_t q0 = 0, q1 = 0, q2 = 0;
     if (splits(x))
       split_pair(x, 0.f, q0, q1, q2);  // x's parts in the low halves
@@ -596,6 +620,222 @@ __global__ __launch_bounds__(SB_THREADS, 1) void grouped_gemm_split_kernel(
   }
 }
 
+// ---------------------------------------------------------------- float32, any K and N
+// The products of the split kernel (three bf16 parts per operand, the same six
+// part products, the same float32 fallback) for the shapes it does not take: K
+// of 4 to 256 at any alignment, and 64 columns or fewer, where its four column
+// blocks of 32 would multiply zeros.
+//
+// What bounds it is memory: a row is read and written once, and 100 x 47
+// products of 2.5M rows take 85 us of MFMA against 0.3 ms of traffic. The
+// general kernel moved the same rows through LDS a float at a time with
+// float32 MFMAs on 128-column tiles. Before and after, us: 100 x 47 (2.5M rows)
+// with both gradients 3,168 -> 1,576; 16 x 16 over 29.5M rows 4,969 -> 856;
+// 128 -> 64 over 1.7M rows (the split kernel before) 422 -> 386.
+//
+// Work mapping. A workgroup of NW wavefronts holds the group's b block (NB
+// blocks of 32 columns x KMAX) in LDS as three bf16 planes and walks a
+// contiguous range of 32 NW-row tiles; wavefront w owns 32 rows of a tile and
+// all NB blocks. The block is small (14 to 104 KB), so up to eight workgroups
+// share a CU and their wavefronts cover each other's waits: the loads of a row
+// run only two 16-deep chunks ahead, without the split kernel's exact wait
+// counts.
+//
+// K axis. Lane (lr, hf) reads chunk c of its row as two 4-float pieces at
+// 16c + 8hf and 4 floats on, at the row's own alignment. A piece that would
+// pass the row's end is read 4 floats before it instead and its elements that
+// an earlier piece covers, like every element past K, count as zero (k_of: the
+// row element behind a place in the chunks); b's planes are laid out in the
+// same places.
+template <int NB, int KMAX, int NW, bool GATHER>
+__global__ __launch_bounds__(64 * NW, any_waves(NB, KMAX)) void grouped_gemm_any_kernel(
+    GemmArgs<float> p, const uint16_t* __restrict__ bt3, const int32_t* __restrict__ bflags,
+    int slices, const float* __restrict__ b, int given_t, int64_t tiles_per_wg,
+    const int32_t* __restrict__ tile_ptr, const int32_t* __restrict__ group_off) {
+  typedef float f32x16 __attribute__((ext_vector_type(16)));
+  constexpr int LD = KMAX + 8;  // bf16 per LDS row: an odd number of 16-byte pieces
+  constexpr int NC = 32 * NB, NT = 64 * NW, TM = 32 * NW;
+  __shared__ __align__(16) uint16_t Bs[3][NC][LD];
+  const int t = threadIdx.x;
+  const int lane = t & 63, w = t >> 6;
+  const int lr = lane & 31, hf = lane >> 5;
+  const int s4 = lane & 3, k4 = lr >> 2;
+  const int64_t total = tile_ptr[p.R];
+  const int64_t first = (int64_t)blockIdx.x * tiles_per_wg;
+  const int64_t last = first + tiles_per_wg < total ? first + tiles_per_wg : total;
+  if (first >= last) return;  // uniform per workgroup
+  const int64_t n0 = (int64_t)blockIdx.y * NC;
+  const int nch = (int)((p.K + 15) / 16);
+  const int full = (int)(p.K / 16);  // chunks wholly inside a row
+  const int K = (int)p.K;
+
+  // the row of a behind tile row 32w + lr of tile tl in group gg (-1: none)
+  auto row_of = [&](int64_t tl, int64_t gg) -> int32_t {
+    const int64_t pos = group_off[gg] + (tl - tile_ptr[gg]) * TM + w * 32 + lr;
+    if (pos >= group_off[gg + 1]) return -1;
+    if constexpr (GATHER) return p.perm[pos];
+    return (int32_t)pos;
+  };
+  auto load4 = [&](const float* q, float* d) {
+    typedef float V __attribute__((ext_vector_type(4), aligned(4)));
+    typedef const __attribute__((address_space(1))) V GV;
+    const V v = *(GV*)q;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = v[i];
+  };
+  // chunk c of a row; pieces past its end are read inside it (K >= 4)
+  auto load_chunk = [&](const float* row, int c, float (&d)[8]) {
+    int k0 = 16 * c + 8 * hf, k1 = k0 + 4;
+    k0 = k0 < K - 4 ? k0 : K - 4;
+    k1 = k1 < K - 4 ? k1 : K - 4;
+    load4(row + k0, d);
+    load4(row + k1, d + 4);
+  };
+  auto group_at = [&](int64_t tl, int64_t g) {
+    while (tile_ptr[g + 1] <= tl) ++g;
+    return g;
+  };
+  int64_t tile = first, g = 0;
+  {
+    int64_t lo = 0, hi = p.R - 1;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi + 1) / 2;
+      if (tile_ptr[mid] <= tile) lo = mid; else hi = mid - 1;
+    }
+    g = lo;
+  }
+  int32_t rid = row_of(tile, g);
+  const float* row = p.a + (int64_t)(rid < 0 ? 0 : rid) * p.K;
+  float af[2][8];
+  load_chunk(row, 0, af[0]);
+  if (nch > 1) load_chunk(row, 1, af[1]);
+
+  int64_t cur_g = -1;
+  bool b_whole = false;  // the group's b block has a value that does not split
+  while (true) {
+    if (g != cur_g) {
+      __syncthreads();  // every wavefront is done with the previous block
+      const int64_t per = p.N * p.Kp;
+      const uint16_t* src = bt3 + g * 3 * per;
+      const int cpr = 2 * nch;  // 16-byte pieces per column of a part
+      for (int c = t; c < 3 * NC * cpr; c += NT) {
+        const int q = c / (NC * cpr), rem = c - q * NC * cpr;
+        const int r = rem / cpr, k = (rem - r * cpr) * 8;
+        u32x4 v = {0u, 0u, 0u, 0u};
+        if (n0 + r < p.N)
+          v = *(const __attribute__((address_space(1))) u32x4*)(src + q * per + (n0 + r) * p.Kp + k);
+        *reinterpret_cast<u32x4*>(&Bs[q][r][k]) = v;
+      }
+      int bad = 0;
+      for (int s = 0; s < slices; ++s) bad |= bflags[g * slices + s];
+      b_whole = bad != 0;
+      __syncthreads();
+      cur_g = g;
+    }
+    const bool has_next = tile + 1 < last;
+    int64_t g1 = g;
+    int32_t rid1 = -1;
+    if (has_next) {
+      g1 = group_at(tile + 1, g);
+      rid1 = row_of(tile + 1, g1);
+    }
+    const float* row1 = p.a + (int64_t)(rid1 < 0 ? 0 : rid1) * p.K;
+
+    f32x16 acc[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
+    auto step = [&](float (&x)[8], int c, int slot) __attribute__((always_inline)) {
+      if (c >= full) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (k_of(16 * c + 8 * hf + i, p.K) < 0) x[i] = 0.f;
+      }
+      int ok = 1;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) ok &= splits(x[s]) ? 1 : 0;
+      if (!b_whole && __builtin_amdgcn_ballot_w64(!ok) == 0) {
+        u32x4 A[3];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          uint32_t q0, q1, q2;
+          split_pair(x[2 * i], x[2 * i + 1], q0, q1, q2);
+          A[0][i] = q0;
+          A[1][i] = q1;
+          A[2][i] = q2;
+        }
+        constexpr int ORD[6][2] = {{0, 2}, {2, 0}, {1, 1}, {0, 1}, {1, 0}, {0, 0}};
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          u32x4 B[3];
+#pragma unroll
+          for (int q = 0; q < 3; ++q)
+            B[q] = *reinterpret_cast<const u32x4*>(&Bs[q][32 * j + lr][16 * c + 8 * hf]);
+#pragma unroll
+          for (int o = 0; o < 6; ++o)
+            acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                __builtin_bit_cast(bf16x8, A[ORD[o][0]]),
+                __builtin_bit_cast(bf16x8, B[ORD[o][1]]), acc[j], 0, 0, 0);
+        }
+      } else {
+        // float32 MFMAs on b from the caller's array (0 past K and past N)
+        const int64_t ks = given_t ? 1 : p.N, ns = given_t ? p.K : 1;
+        const float* bg = b + g * p.K * p.N;
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const int64_t n = n0 + 32 * j + lr;
+#pragma unroll
+          for (int s = 0; s < 8; ++s) {
+            const int64_t k = k_of(16 * c + 8 * hf + s, p.K);
+            const float y = n < p.N && k >= 0 ? load_global(bg + n * ns + k * ks) : 0.f;
+            acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[s], y, acc[j], 0, 0, 0);
+          }
+        }
+      }
+      // the chunk's values are used: request the one two on, or the next
+      // tile's first ones
+      if (c + 2 < nch) load_chunk(row, c + 2, x);
+      else if (slot < nch) load_chunk(row1, slot, x);
+    };
+    for (int c = 0; c < nch; c += 2) {
+      step(af[0], c, 0);
+      if (c + 1 < nch) step(af[1], c + 1, 1);
+    }
+    // lane (lr, hf) holds column lr of rows 8q + 4hf + r in acc[j][4q + r];
+    // the quad transpose gives lane 4 k4 + s4 row 8q + 4hf + s4 at columns
+    // 4 k4 .. 4 k4 + 3
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int32_t orow = __shfl(rid, 8 * q + 4 * hf + s4);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        float x[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x[v] = acc[j][4 * q + v];
+        quad_transpose(x, s4);
+        const int64_t n = n0 + 32 * j + 4 * k4;
+        if (orow >= 0 && n < p.N) {
+          float* o = p.out + (int64_t)orow * p.N + n;
+          if (n + 4 <= p.N) {
+            typedef float V __attribute__((ext_vector_type(4), aligned(4)));
+            *reinterpret_cast<V*>(o) = V{x[0], x[1], x[2], x[3]};
+          } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+              if (n + v < p.N) o[v] = x[v];
+          }
+        }
+      }
+    }
+    if (!has_next) return;
+    ++tile;
+    g = g1;
+    rid = rid1;
+    row = row1;
+  }
+}
+
 // ---------------------------------------------------------------- float64
 // float64 shapes with K a multiple of 16 up to 128 and a on a 16-byte
 // boundary (the host checks; others take grouped_gemm_kernel).
@@ -626,14 +866,15 @@ constexpr int F64_LD = F64_KMAX + 4;  // doubles per LDS row
 constexpr int F64_RB = 1, F64_NW = 8;  // the library's shape: 128-row tiles
 constexpr int F64_TM = 16 * F64_RB * F64_NW;
 
-template <int NCH, int RB, int NW, bool GATHER>
+template <int NCH, int RB, int NW, int CB, bool GATHER>
 __global__ __launch_bounds__(64 * NW, 1) void grouped_gemm_f64_kernel(
     GemmArgs<double> p, int64_t tiles_per_wg, const int32_t* __restrict__ tile_ptr,
     const int32_t* __restrict__ group_off, double* __restrict__ sink) {
   constexpr int TM = 16 * RB * NW;
   constexpr int NT = 64 * NW;
-  constexpr int CB = GBN / 16;  // column blocks
-  __shared__ __align__(16) double Bs[GBN][F64_LD];
+  constexpr int NC = 16 * CB;  // columns
+  constexpr int JG = CB < 4 ? CB : 4;
+  __shared__ __align__(16) double Bs[NC][F64_LD];
   const int t = threadIdx.x;
   const int lane = t & 63, w = t >> 6;
   const int li = lane & 15, q = lane >> 4;
@@ -641,7 +882,7 @@ __global__ __launch_bounds__(64 * NW, 1) void grouped_gemm_f64_kernel(
   const int64_t first = (int64_t)blockIdx.x * tiles_per_wg;
   const int64_t last = first + tiles_per_wg < total ? first + tiles_per_wg : total;
   if (first >= last) return;  // uniform per workgroup
-  const int64_t n0 = (int64_t)blockIdx.y * GBN;
+  const int64_t n0 = (int64_t)blockIdx.y * NC;
 
   // group metadata through scalar loads (uniform index, read-only arguments)
   auto uget = [](const int32_t* __restrict__ arr, int64_t i) -> int64_t {
@@ -728,7 +969,7 @@ __global__ __launch_bounds__(64 * NW, 1) void grouped_gemm_f64_kernel(
       __syncthreads();  // every wavefront is done with the previous block
       const double* src = p.bt + g * p.N * p.Kp;
       constexpr int CPR = NCH * 8;  // 16-byte pieces per LDS row
-      for (int c = t; c < GBN * CPR; c += NT) {
+      for (int c = t; c < NC * CPR; c += NT) {
         const int r = c / CPR, k = (c % CPR) * 2;
         double v[2] = {0.0, 0.0};
         if (n0 + r < p.N) load_global_n<double, 2>(src + (n0 + r) * p.Kp + k, v);
@@ -767,10 +1008,10 @@ __global__ __launch_bounds__(64 * NW, 1) void grouped_gemm_f64_kernel(
       // over them (four or more independent accumulators between two MFMAs
       // that share one)
 #pragma unroll
-      for (int jg = 0; jg < CB; jg += 4) {
-        double bv[4][4];
+      for (int jg = 0; jg < CB; jg += JG) {
+        double bv[JG][4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < JG; ++j) {
           const double* bp = &Bs[16 * (jg + j) + li][16 * c + 2 * q];
           double x[2], y[2];
           load_n<double, 2>(bp, x);
@@ -783,7 +1024,7 @@ __global__ __launch_bounds__(64 * NW, 1) void grouped_gemm_f64_kernel(
 #pragma unroll
         for (int s = 0; s < 4; ++s)
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
+          for (int j = 0; j < JG; ++j)
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)
               acc[rb][jg + j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
@@ -1075,6 +1316,28 @@ int64_t grouped_workspace_bytes(int64_t n, int64_t K, int64_t N, int64_t R, bool
   return b_region_bytes<T>(K, N, R) + plan_workspace_bytes(n, R, gather);
 }
 
+// grouped_gemm_any_kernel's instance for a shape: column blocks, LDS depth,
+// wavefronts, and workgroups per CU (what 160 KB of LDS and the registers
+// allow). Four column blocks only for K of 65 to 128: beyond, they would need
+// more LDS than a CU has, and below, two blocks twice (a is then the smaller
+// side, read again from L2) leave more wavefronts to a SIMD.
+struct AnyShape {
+  int nb, km, nw, per_cu;
+};
+constexpr int64_t ANY_KMAX = 256;
+inline AnyShape any_shape(int64_t K, int64_t N) {
+  AnyShape s;
+  const int64_t k16 = (K + 15) / 16 * 16;
+  s.km = k16 <= 64 ? 64 : (k16 <= 128 ? 128 : 256);
+  s.nb = N <= 32 ? 1 : (N <= 64 || s.km != 128 ? 2 : 4);
+  const int lds = 3 * 32 * s.nb * (s.km + 8) * 2;
+  s.nw = lds > (54 << 10) ? 8 : 4;
+  s.per_cu = (160 << 10) / lds;
+  const int waves = 4 * any_waves(s.nb, s.km);
+  if (s.per_cu > waves / s.nw) s.per_cu = waves / s.nw;
+  return s;
+}
+
 template <class T>
 hipError_t launch_grouped(const GemmLaunch& L, bool gather) {
   if (L.n <= 0 || L.N <= 0 || L.R <= 0) return hipSuccess;
@@ -1082,8 +1345,14 @@ hipError_t launch_grouped(const GemmLaunch& L, bool gather) {
   constexpr int EVH = 16 / sizeof(T);
   const bool split = sizeof(T) == 4 && Kp <= SB_KMAX && Kp == L.K &&
                         reinterpret_cast<uintptr_t>(L.a) % 16 == 0 && L.K % EVH == 0;
+  // other float32 shapes, and those of one or two column blocks, where the
+  // split kernel's four multiply zeros (gather_mm, us: 64 -> 16 over 645K rows
+  // 149 there and 114 here, 128 -> 64 over 1.7M rows 422 and 386; with four
+  // blocks the split kernel stays ahead)
+  const bool any = sizeof(T) == 4 && L.K >= 4 && L.K <= ANY_KMAX && (!split || L.N <= 64);
+  const AnyShape as = any_shape(L.K, L.N);
   const bool f64 = sizeof(T) == 8 && Kp <= F64_KMAX && Kp == L.K && aligned16(L.a);
-  const int tm = split ? SB_TM : (f64 ? F64_TM : GBM);
+  const int tm = any ? 32 * as.nw : (split ? SB_TM : (f64 ? F64_TM : GBM));
   char* w = static_cast<char*>(L.workspace);
   T* bt = reinterpret_cast<T*>(w);
   const int64_t vals = L.R * L.N * Kp;
@@ -1093,7 +1362,7 @@ hipError_t launch_grouped(const GemmLaunch& L, bool gather) {
   w += b_region_bytes<T>(L.K, L.N, L.R);
   void* sink = w - ws_align(GEMM_SINK_BYTES);
 
-  if (split) {
+  if (split || any) {
     hipLaunchKernelGGL(split_b_kernel, dim3((unsigned)(L.R * slices)), dim3(BLOCK), 0, L.stream,
                        static_cast<const float*>(L.b), bt3, bflags, L.K, Kp, L.N, L.trans_b,
                        slices);
@@ -1125,6 +1394,38 @@ hipError_t launch_grouped(const GemmLaunch& L, bool gather) {
   constexpr int EV = 16 / sizeof(T);
   a.a_vec = (L.K % EV == 0) && (reinterpret_cast<uintptr_t>(L.a) % 16 == 0);
   a.out_vec = (L.N % EV == 0) && (reinterpret_cast<uintptr_t>(L.out) % 16 == 0);
+  if constexpr (sizeof(T) == 4) {
+    if (any) {
+      const int64_t ny = (L.N + 32 * as.nb - 1) / (32 * as.nb);
+      const int64_t mt = (L.n + tm - 1) / tm + L.R;  // upper bound of the tile count
+      int64_t wgs = 256 * as.per_cu / ny;
+      if (wgs < 1) wgs = 1;
+      if (wgs > mt) wgs = mt;
+      const int64_t per = (mt + wgs - 1) / wgs;
+      const dim3 grid((unsigned)wgs, (unsigned)ny);
+      const float* bsrc = static_cast<const float*>(L.b);
+#define MDGL_ANY_CASE(NB, KM, NW)                                                              \
+  if (as.nb == NB && as.km == KM) {                                                            \
+    if (gather)                                                                                \
+      hipLaunchKernelGGL((grouped_gemm_any_kernel<NB, KM, NW, true>), grid, dim3(64 * NW), 0,  \
+                         L.stream, a, bt3, bflags, slices, bsrc, L.trans_b, per, a.tile_ptr,   \
+                         a.group_off);                                                         \
+    else                                                                                       \
+      hipLaunchKernelGGL((grouped_gemm_any_kernel<NB, KM, NW, false>), grid, dim3(64 * NW), 0, \
+                         L.stream, a, bt3, bflags, slices, bsrc, L.trans_b, per, a.tile_ptr,   \
+                         a.group_off);                                                         \
+  }
+      MDGL_ANY_CASE(1, 64, 4)
+      MDGL_ANY_CASE(1, 128, 4)
+      MDGL_ANY_CASE(1, 256, 4)
+      MDGL_ANY_CASE(2, 64, 4)
+      MDGL_ANY_CASE(2, 128, 4)
+      MDGL_ANY_CASE(2, 256, 8)
+      MDGL_ANY_CASE(4, 128, 8)
+#undef MDGL_ANY_CASE
+      return hipGetLastError();
+    }
+  }
   const int64_t nt = (L.N + GBN - 1) / GBN;
   if constexpr (sizeof(T) == 4) {
     if (split) {
@@ -1162,28 +1463,39 @@ hipError_t launch_grouped(const GemmLaunch& L, bool gather) {
   }
   if constexpr (sizeof(T) == 8) {
     if (f64) {
-      // as for the split kernel: one workgroup per CU (its LDS block), each a
-      // contiguous range of tiles
+      // as for the split kernel: as many workgroups per CU as their LDS blocks
+      // fit, each a contiguous range of tiles; 32 or 64 columns take only
+      // their own column blocks (eight multiplied zeros for 16 x 32 products of
+      // 10.5M rows)
+      const int cb = L.N <= 32 ? 2 : (L.N <= 64 ? 4 : 8);
       const int64_t mt = (L.n + F64_TM - 1) / F64_TM + L.R;
-      int64_t wgs = 256 / nt;
+      int64_t wgs = 256 * (8 / cb) / nt;
       if (wgs < 1) wgs = 1;
       if (wgs > mt) wgs = mt;
       const int64_t per = (mt + wgs - 1) / wgs;
       const dim3 grid((unsigned)wgs, (unsigned)nt), block(64 * F64_NW);
-#define MDGL_F64_CASE(C)                                                                     \
-  case C:                                                                                    \
-    if (gather)                                                                              \
-      hipLaunchKernelGGL((grouped_gemm_f64_kernel<C, F64_RB, F64_NW, true>), grid, block, 0,  \
-                         L.stream, a, per, a.tile_ptr, a.group_off, static_cast<double*>(sink)); \
-    else                                                                                     \
-      hipLaunchKernelGGL((grouped_gemm_f64_kernel<C, F64_RB, F64_NW, false>), grid, block, 0, \
-                         L.stream, a, per, a.tile_ptr, a.group_off, static_cast<double*>(sink)); \
+#define MDGL_F64_LAUNCH(C, CB, G)                                                            \
+  hipLaunchKernelGGL((grouped_gemm_f64_kernel<C, F64_RB, F64_NW, CB, G>), grid, block, 0,    \
+                     L.stream, a, per, a.tile_ptr, a.group_off, static_cast<double*>(sink))
+#define MDGL_F64_CASE(C)                                                  \
+  case C:                                                                 \
+    if (cb == 2) {                                                        \
+      if (gather) MDGL_F64_LAUNCH(C, 2, true);                            \
+      else MDGL_F64_LAUNCH(C, 2, false);                                  \
+    } else if (cb == 4) {                                                 \
+      if (gather) MDGL_F64_LAUNCH(C, 4, true);                            \
+      else MDGL_F64_LAUNCH(C, 4, false);                                  \
+    } else {                                                              \
+      if (gather) MDGL_F64_LAUNCH(C, 8, true);                            \
+      else MDGL_F64_LAUNCH(C, 8, false);                                  \
+    }                                                                     \
     break;
       switch (Kp / 16) {
         MDGL_F64_CASE(1) MDGL_F64_CASE(2) MDGL_F64_CASE(3) MDGL_F64_CASE(4)
         MDGL_F64_CASE(5) MDGL_F64_CASE(6) MDGL_F64_CASE(7) MDGL_F64_CASE(8)
         default: return hipErrorInvalidValue;
       }
+#undef MDGL_F64_LAUNCH
 #undef MDGL_F64_CASE
       return hipGetLastError();
     }
@@ -1196,16 +1508,22 @@ hipError_t launch_grouped(const GemmLaunch& L, bool gather) {
 
 // ---------------------------------------------------------------- gradient of b
 // db[g] = sum over the rows of group g of a[row]^T grad[row] (D1 x D2 per
-// group). A group's rows are cut into chunks of `ch` rows; a workgroup (4
-// wavefronts, 2 x 2, each 64 x 64 of the tile as 4 x 4 MFMA blocks) forms the
-// 128 x 128 tile blockIdx.y of one chunk's product. The rows are the
-// contracted axis, walked BK at a time through row-major LDS tiles (double
-// buffered like the forward kernel; BK rows per stage, 16 when the rows come
-// through gather_mm's permutation): lane l feeds a[row k0 + l / 16][m0 + l %
-// 16] as A^T and grad[row k0 + l / 16][n0 + l % 16] as B; a row stride of 144
-// elements puts the four rows one 64-lane read touches in distinct banks.
-// Chunk products go to partials that tn_fold_kernel adds per group in chunk
-// order, so db is the same on every run.
+// group). A group's rows are cut into chunks of `ch` rows, one workgroup of 4
+// wavefronts each. The rows are the contracted axis of the MFMAs (four per
+// instruction): in a step lane (li, h) supplies a[row h][m0 + 16 i + li] as A^T
+// and grad[row h][n0 + 16 j + li] as B, so the operands are read straight from
+// the rows, 64 consecutive bytes of each, into registers (no LDS, no barrier,
+// any width and alignment), one step of 4 U rows ahead of their use. A
+// wavefront holds a tile of MB x NBK blocks of 16 x 16 in registers, sized to the
+// product (a 128 x 128 tile through LDS multiplied mostly zeros for narrower
+// ones: 100 x 47 over 2.5M rows took 1,306 us, here 440).
+// Products of several tiles: up to TW of them go to different wavefronts of
+// the workgroup, which read the same rows through its L1; the remaining
+// wavefronts (4 / TW streams) take alternate steps of the rows, and their
+// tiles are added through LDS in stream order at the end. Columns past the
+// width read the last one (their results are not stored); rows past the
+// chunk count as zero. Chunk products go to partials that tn_fold_kernel adds
+// per group in chunk order, so db is the same on every run.
 template <class T>
 struct TnArgs {
   const T* a;
@@ -1215,20 +1533,15 @@ struct TnArgs {
   const int32_t* group_off;  // R + 1
   const int32_t* chunk_ptr;  // R + 1, chunks per group (prefix)
   int64_t R, D1, D2, ch;
-  int a_vec, g_vec, tiles_n;
+  int tw, tiles_n, tiles;    // tiles per workgroup (1, 2 or 4), tiles along D2, tiles
 };
 
-template <class T, int BK, bool VECT, bool GATHER>
-__global__ __launch_bounds__(BLOCK) void grouped_tn_kernel(TnArgs<T> p) {
+template <class T, int MB, int NBK, bool GATHER>
+__global__ __launch_bounds__(BLOCK, MB * NBK * (int)sizeof(T) > 64 ? 2 : 3) void grouped_tn_kernel(TnArgs<T> p) {
   using M = Mfma<T>;
   using acc_t = typename M::acc_t;
-  constexpr int LD = GBM + 16;
-  constexpr int EV = 16 / sizeof(T);   // elements per 16-byte load
-  constexpr int CPR = GBM / EV;        // 16-byte chunks per 128-wide tile row
-  constexpr int RPP = BLOCK / CPR;     // tile rows per pass of the block
-  constexpr int PASSES = BK / RPP;
-  __shared__ __align__(16) T As[2][BK][LD];
-  __shared__ __align__(16) T Bs[2][BK][LD];
+  constexpr int U = 2;  // groups of four rows per step
+  __shared__ acc_t red[2][MB * NBK][WAVE];
 
   const int64_t c = blockIdx.x;
   if (c >= p.chunk_ptr[p.R]) return;  // uniform per workgroup
@@ -1241,130 +1554,120 @@ __global__ __launch_bounds__(BLOCK) void grouped_tn_kernel(TnArgs<T> p) {
   const int64_t r0 = p.group_off[grp] + (c - p.chunk_ptr[grp]) * p.ch;
   const int64_t g_end = p.group_off[grp + 1];
   const int64_t r_end = r0 + p.ch < g_end ? r0 + p.ch : g_end;
-  const int64_t m0 = (int64_t)(blockIdx.y / p.tiles_n) * GBM;
-  const int64_t n0 = (int64_t)(blockIdx.y % p.tiles_n) * GBN;
-  const int t = threadIdx.x;
-  const int lane = t & 63, w = t >> 6, wm = w >> 1, wn = w & 1;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int li = lane & 15, h = lane >> 4;
+  const int streams = WAVES_PER_BLOCK / p.tw, stream = w / p.tw;
+  const int tile_raw = (int)blockIdx.y * p.tw + w % p.tw;
+  const bool mine = tile_raw < p.tiles;  // else this wavefront repeats the last tile, unwritten
+  const int tile = mine ? tile_raw : p.tiles - 1;
+  const int m0 = tile / p.tiles_n * (16 * MB), n0 = tile % p.tiles_n * (16 * NBK);
+  const int D1 = (int)p.D1, D2 = (int)p.D2;
+  int ca[MB], cg[NBK];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) ca[i] = m0 + 16 * i + li < D1 ? m0 + 16 * i + li : D1 - 1;
+#pragma unroll
+  for (int j = 0; j < NBK; ++j) cg[j] = n0 + 16 * j + li < D2 ? n0 + 16 * j + li : D2 - 1;
 
-  T ra[PASSES][EV], rb[PASSES][EV];
-  // gather_mm's rows of a stage come through the permutation: they are
-  // requested one stage ahead (an unconditional load of a clamped index; the
-  // row test is applied where they are used), so no stage waits for them
-  auto stage_rows = [&](int64_t k0, int32_t (&rid)[PASSES]) {
+  acc_t acc[MB][NBK];
 #pragma unroll
-    for (int q = 0; q < PASSES; ++q) {
-      const int64_t pos = k0 + q * RPP + t / CPR;
-      if constexpr (GATHER) rid[q] = p.perm[pos < r_end ? pos : r_end - 1];
-      else rid[q] = 0;
-    }
-  };
-  // Each lane's 16-byte pieces of a stage (VECT: both operands' rows allow
-  // them): rows past the chunk and pieces past the width load row 0 /
-  // column 0 and are zeroed when the stage is written to LDS, at the end of
-  // the stage (a test right after a load would wait for the load there);
-  // otherwise element by element. The form is fixed at compile time: chosen
-  // at run time, the compiler merged both into element loads.
-  bool oka[PASSES], okb[PASSES];
-  auto load_stage = [&](int64_t k0, const int32_t (&rids)[PASSES]) {
+  for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int q = 0; q < PASSES; ++q) {
-      const int r = q * RPP + t / CPR;
-      const int col = (t % CPR) * EV;
-      const int64_t pos = k0 + r;
-      const bool ok = pos < r_end;
-      const int64_t rid = ok ? (GATHER ? (int64_t)rids[q] : pos) : 0;
-      const int64_t ca = m0 + col, cb = n0 + col;
-      if constexpr (VECT) {
-        oka[q] = ok && ca < p.D1;  // D1 and D2 are multiples of EV
-        okb[q] = ok && cb < p.D2;
-        load_vec<T>(p.a + rid * p.D1 + (ca < p.D1 ? ca : 0), ra[q]);
-        load_vec<T>(p.g + rid * p.D2 + (cb < p.D2 ? cb : 0), rb[q]);
-      } else {
-        oka[q] = okb[q] = true;
-#pragma unroll
-        for (int v = 0; v < EV; ++v) {
-          ra[q][v] = (ok && ca + v < p.D1) ? p.a[rid * p.D1 + ca + v] : T(0);
-          rb[q][v] = (ok && cb + v < p.D2) ? p.g[rid * p.D2 + cb + v] : T(0);
-        }
-      }
-    }
-  };
-  auto store_stage = [&](int buf) {
-#pragma unroll
-    for (int q = 0; q < PASSES; ++q) {
-      const int r = q * RPP + t / CPR;
-      const int col = (t % CPR) * EV;
-      T xa[EV], xb[EV];
-#pragma unroll
-      for (int v = 0; v < EV; ++v) {
-        xa[v] = oka[q] ? ra[q][v] : T(0);
-        xb[v] = okb[q] ? rb[q][v] : T(0);
-      }
-      store_vec<T>(&As[buf][r][col], xa);
-      store_vec<T>(&Bs[buf][r][col], xb);
-    }
-  };
-
-  acc_t acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < NBK; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = T(0);
 
-  const int64_t nstages = (r_end - r0 + BK - 1) / BK;  // a chunk holds at least one row
-  int32_t rid_a[PASSES], rid_b[PASSES];
-  stage_rows(r0, rid_a);
-  load_stage(r0, rid_a);
-  store_stage(0);
-  stage_rows(r0 + BK, rid_a);  // the next stage's rows
-  __syncthreads();
-  for (int64_t s = 0; s < nstages; ++s) {
-    const int buf = s & 1;
-    if (s + 1 < nstages) load_stage(r0 + (s + 1) * BK, rid_a);
-    stage_rows(r0 + (s + 2) * BK, rid_b);
+  struct Step {
+    T a[U][MB], g[U][NBK];
+  };
+  // row of a and grad behind position pos + 4u + h (past the chunk: its last)
+  auto rows = [&](int64_t pos, int32_t (&r)[U]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < PASSES; ++q) rid_a[q] = rid_b[q];
-    __builtin_amdgcn_s_setprio(1);  // MFMA issue first (as in the forward kernel)
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      T af[4], bf[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        af[i] = As[buf][kk + h][wm * 64 + i * 16 + li];
-        bf[i] = Bs[buf][kk + h][wn * 64 + i * 16 + li];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = M::step(af[i], bf[j], acc[i][j]);
+    for (int u = 0; u < U; ++u) {
+      int64_t q = pos + 4 * u + h;
+      q = q < r_end ? q : r_end - 1;
+      if constexpr (GATHER) r[u] = p.perm[q];
+      else r[u] = (int32_t)q;
     }
-    __builtin_amdgcn_s_setprio(0);
-    if (s + 1 < nstages) {
-      store_stage(buf ^ 1);
-      __syncthreads();
+  };
+  auto load = [&](const int32_t (&r)[U], Step& s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const T* ra = p.a + (int64_t)r[u] * D1;
+      const T* rg = p.g + (int64_t)r[u] * D2;
+#pragma unroll
+      for (int i = 0; i < MB; ++i) s.a[u][i] = load_global(ra + ca[i]);
+#pragma unroll
+      for (int j = 0; j < NBK; ++j) s.g[u][j] = load_global(rg + cg[j]);
+    }
+  };
+  auto multiply = [&](const Step& s, int64_t pos) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      T x[MB], y[NBK];
+      const bool in = pos + 4 * u + h < r_end;
+#pragma unroll
+      for (int i = 0; i < MB; ++i) x[i] = in ? s.a[u][i] : T(0);
+#pragma unroll
+      for (int j = 0; j < NBK; ++j) y[j] = in ? s.g[u][j] : T(0);
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NBK; ++j) acc[i][j] = M::step(x[i], y[j], acc[i][j]);
+    }
+  };
+  const int64_t stride = 4 * U * streams;
+  int64_t pos = r0 + 4 * U * stream;
+  if (pos < r_end) {  // uniform per wavefront
+    Step cur, nxt;
+    int32_t r[U];
+    rows(pos, r);
+    load(r, cur);
+    rows(pos + stride, r);  // the next step's rows, requested a step ahead of its loads
+    for (; pos < r_end; pos += stride) {
+      load(r, nxt);
+      rows(pos + 2 * stride, r);
+      multiply(cur, pos);
+      cur = nxt;
     }
   }
 
+  // the streams' tiles added in order: 2 and 3 to 0 and 1, then 1 to 0
+  for (int half = streams / 2; half >= 1; half /= 2) {  // uniform per workgroup
+    const int slot = (stream % half) * p.tw + w % p.tw;  // below 2
+    if (stream >= half && stream < 2 * half) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NBK; ++j) red[slot][i * NBK + j][lane] = acc[i][j];
+    }
+    __syncthreads();
+    if (stream < half) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NBK; ++j) acc[i][j] += red[slot][i * NBK + j][lane];
+    }
+    __syncthreads();
+  }
+  if (stream != 0 || !mine) return;
   T* out = p.part + c * p.D1 * p.D2;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < MB; ++i) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int64_t d1 = m0 + wm * 64 + i * 16 + M::row(h, r);
+      const int64_t d1 = m0 + i * 16 + M::row(h, r);
       if (d1 >= p.D1) continue;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int64_t d2 = n0 + wn * 64 + j * 16 + li;
+      for (int j = 0; j < NBK; ++j) {
+        const int64_t d2 = n0 + j * 16 + li;
         if (d2 < p.D2) out[d1 * p.D2 + d2] = acc[i][j][r];
       }
     }
   }
 }
 
-// db[g][e] = sum of part[c][e] over g's chunks in order (0 for an empty group).
+// db[g][e] = sum of part[c][e] over g's chunks in order (0 for an empty group),
+// eight partials requested at a time.
 template <class T>
 __global__ __launch_bounds__(BLOCK) void tn_fold_kernel(const T* __restrict__ part,
                                                         const int32_t* __restrict__ chunk_ptr,
@@ -1374,19 +1677,32 @@ __global__ __launch_bounds__(BLOCK) void tn_fold_kernel(const T* __restrict__ pa
        i += (int64_t)gridDim.x * BLOCK) {
     const int64_t g = i / E, e = i - g * E;
     T acc = T(0);
-    for (int64_t c = chunk_ptr[g]; c < chunk_ptr[g + 1]; ++c) acc += part[c * E + e];
+    int64_t c = chunk_ptr[g];
+    const int64_t c1 = chunk_ptr[g + 1];
+    for (; c + 8 <= c1; c += 8) {
+      T v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = part[(c + k) * E + e];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) acc += v[k];
+    }
+    for (; c < c1; ++c) acc += part[c * E + e];
     db[i] = acc;
   }
 }
 
-constexpr int64_t TN_CH = 4096;                 // rows per chunk, at least
+constexpr int64_t TN_CH = 256;                  // rows per chunk, at least
+constexpr int64_t TN_CHUNKS = 2048;             // chunks, about, when rows allow
 constexpr int64_t TN_PART_BYTES = 256ll << 20;  // partials kept below this when rows allow
 
-// Rows per chunk: TN_CH, doubled until the partials of the chunks (at most
-// n / ch + R of them) fit TN_PART_BYTES, and at most n (n < 2**31).
+// Rows per chunk: TN_CH, doubled while there are more than TN_CHUNKS chunks
+// (at most n / ch + R of them; eight workgroups a CU) or their partials pass
+// TN_PART_BYTES, and at most n (n < 2**31).
 inline int64_t tn_chunk_rows(int64_t n, int64_t D1, int64_t D2, int64_t R, int64_t es) {
   int64_t ch = TN_CH;
-  while (ch < n && ((n + ch - 1) / ch + R) * D1 * D2 * es > TN_PART_BYTES) ch *= 2;
+  while (ch < n && ((n + ch - 1) / ch > TN_CHUNKS ||
+                    ((n + ch - 1) / ch + R) * D1 * D2 * es > TN_PART_BYTES))
+    ch *= 2;
   return ch < n ? ch : (n > 0 ? n : 1);
 }
 
@@ -1441,26 +1757,36 @@ hipError_t launch_grouped_grad(const GemmGradLaunch& L, bool gather) {
   a.D1 = L.D1;
   a.D2 = L.D2;
   a.ch = ch;
-  constexpr int EV = 16 / sizeof(T);
-  a.a_vec = (L.D1 % EV == 0) && (reinterpret_cast<uintptr_t>(L.a) % 16 == 0);
-  a.g_vec = (L.D2 % EV == 0) && (reinterpret_cast<uintptr_t>(L.grad) % 16 == 0);
-  const int64_t tiles_m = (L.D1 + GBM - 1) / GBM;
-  a.tiles_n = (int)((L.D2 + GBN - 1) / GBN);
-  // rows gathered through the permutation wait longer: shallower stages,
-  // half the LDS, twice the workgroups per CU to cover them
-  const dim3 grid((unsigned)max_chunks, (unsigned)(tiles_m * a.tiles_n));
-  const bool vect = a.a_vec && a.g_vec;
-  if (perm && vect)
-    hipLaunchKernelGGL((grouped_tn_kernel<T, 16, true, true>), grid, dim3(BLOCK), 0, L.stream, a);
-  else if (perm)
-    hipLaunchKernelGGL((grouped_tn_kernel<T, 16, false, true>), grid, dim3(BLOCK), 0, L.stream,
-                       a);
-  else if (vect)
-    hipLaunchKernelGGL((grouped_tn_kernel<T, Mfma<T>::BK, true, false>), grid, dim3(BLOCK), 0,
-                       L.stream, a);
-  else
-    hipLaunchKernelGGL((grouped_tn_kernel<T, Mfma<T>::BK, false, false>), grid, dim3(BLOCK), 0,
-                       L.stream, a);
+  const int64_t b1 = (L.D1 + 15) / 16, b2 = (L.D2 + 15) / 16;
+  // the tile, of those built, with the fewest blocks in all (of equal ones the largest)
+  auto best = [](int64_t blocks, const int* sizes, int n) {
+    int got = sizes[0];
+    for (int k = 1; k < n; ++k)
+      if ((blocks + sizes[k] - 1) / sizes[k] * sizes[k] < (blocks + got - 1) / got * got)
+        got = sizes[k];
+    return got;
+  };
+  static constexpr int MS4[] = {8, 4, 2}, NS4[] = {4, 3, 2, 1}, MS8[] = {4, 2}, NS8[] = {4, 2, 1};
+  const int mb = sizeof(T) == 4 ? best(b1, MS4, 3) : best(b1, MS8, 2);
+  const int nb = sizeof(T) == 4 ? best(b2, NS4, 4) : best(b2, NS8, 3);
+  a.tiles_n = (int)((b2 + nb - 1) / nb);
+  a.tiles = (int)((b1 + mb - 1) / mb) * a.tiles_n;
+  a.tw = a.tiles > 2 ? 4 : a.tiles;
+  const dim3 grid((unsigned)max_chunks, (unsigned)((a.tiles + a.tw - 1) / a.tw));
+#define MDGL_TN_CASE(M, N)                                                                    \
+  if (mb == M && nb == N) {                                                                   \
+    if (perm)                                                                                 \
+      hipLaunchKernelGGL((grouped_tn_kernel<T, M, N, true>), grid, dim3(BLOCK), 0, L.stream, a); \
+    else                                                                                      \
+      hipLaunchKernelGGL((grouped_tn_kernel<T, M, N, false>), grid, dim3(BLOCK), 0, L.stream, a); \
+  }
+  if constexpr (sizeof(T) == 4) {
+    MDGL_TN_CASE(8, 4) MDGL_TN_CASE(8, 3) MDGL_TN_CASE(8, 2) MDGL_TN_CASE(8, 1)
+    MDGL_TN_CASE(4, 3) MDGL_TN_CASE(2, 3)
+  }
+  MDGL_TN_CASE(4, 4) MDGL_TN_CASE(4, 2) MDGL_TN_CASE(4, 1)
+  MDGL_TN_CASE(2, 4) MDGL_TN_CASE(2, 2) MDGL_TN_CASE(2, 1)
+#undef MDGL_TN_CASE
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int64_t E = L.D1 * L.D2;
