@@ -21,8 +21,10 @@ these follow the calculus of the forward ops and run on the same kernels:
     the arg edge; otherwise ``mdgl_gspmm_edge_grad`` writes the masked per-edge
     gradient M, then dX is a gspmm over the out-CSR of M (times d msg / dX) and dY is M
     times d msg / dY, per edge;
-* gsddmm(op, X at target tx, Y at target ty): the per-edge gradient times
-  d op / dX (dY) is reduced over the edges of each node of the operand's
+* gsddmm(op, X at target tx, Y at target ty): mul and dot between the two
+  endpoints take one gspmm per operand (the other operand's rows times the
+  per-edge gradient); otherwise the per-edge gradient times d op / dX (dY) is
+  reduced over the edges of each node of the operand's
   target by a gspmm copy_rhs sum (in-CSR for v, out-CSR for u; nothing for e);
 * edge_softmax: dX = a * (G - s[row]) with s[row] = sum over the row of G * a:
   gsddmm e_mul_e, gspmm copy_rhs sum over the CSR of norm_by, then
@@ -333,6 +335,16 @@ class GSDDMM(torch.autograd.Function):
         need_x = ctx.needs_input_grad[2] and x is not None
         need_y = ctx.needs_input_grad[3] and y is not None
         dx = dy = None
+        if op in ("mul", "dot") and {tx, ty} == {"u", "v"}:
+            # the per-edge gradient times the other endpoint's row, summed at
+            # this one: one gspmm, no per-edge tensor of products
+            if need_x:
+                p = _gspmm(g, "mul", "sum", y, G, kind="out" if tx == "u" else "in")
+                dx = _reduce_to(p, _padded(x.shape, p.shape)).reshape(x.shape)
+            if need_y:
+                p = _gspmm(g, "mul", "sum", x, G, kind="out" if ty == "u" else "in")
+                dy = _reduce_to(p, _padded(y.shape, p.shape)).reshape(y.shape)
+            return None, None, _back(dx, x0), _back(dy, y0), None, None
         if need_x:
             if op in ("copy_lhs", "add", "sub"):
                 p = G
