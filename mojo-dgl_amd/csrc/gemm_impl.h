@@ -1691,16 +1691,16 @@ __global__ __launch_bounds__(BLOCK) void tn_fold_kernel(const T* __restrict__ pa
   }
 }
 
-constexpr int64_t TN_CH = 256;                  // rows per chunk, at least
-constexpr int64_t TN_CHUNKS = 2048;             // chunks, about, when rows allow
-constexpr int64_t TN_PART_BYTES = 256ll << 20;  // partials kept below this when rows allow
+constexpr int64_t TN_CH = 256, TN_CH_MOST = 4096;  // rows per chunk, at least and usually at most
+constexpr int64_t TN_CHUNKS = 2048;                // chunks, about, when rows allow
+constexpr int64_t TN_PART_BYTES = 256ll << 20;     // partials kept below this when rows allow
 
-// Rows per chunk: TN_CH, doubled while there are more than TN_CHUNKS chunks
-// (at most n / ch + R of them; eight workgroups a CU) or their partials pass
-// TN_PART_BYTES, and at most n (n < 2**31).
+// Rows per chunk: TN_CH, doubled to TN_CH_MOST while there are more than
+// TN_CHUNKS chunks (at most n / ch + R of them; eight workgroups a CU) and
+// further while their partials pass TN_PART_BYTES, and at most n (n < 2**31).
 inline int64_t tn_chunk_rows(int64_t n, int64_t D1, int64_t D2, int64_t R, int64_t es) {
   int64_t ch = TN_CH;
-  while (ch < n && ((n + ch - 1) / ch > TN_CHUNKS ||
+  while (ch < n && ((ch < TN_CH_MOST && (n + ch - 1) / ch > TN_CHUNKS) ||
                     ((n + ch - 1) / ch + R) * D1 * D2 * es > TN_PART_BYTES))
     ch *= 2;
   return ch < n ? ch : (n > 0 ? n : 1);

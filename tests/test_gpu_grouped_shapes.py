@@ -1,0 +1,107 @@
+"""segment_mm / gather_mm and their gradients at the widths where the kernels'
+tiles end: K around the 16-deep chunks and the 4-float pieces, N around the
+column blocks, groups that are empty, of one row and just past a tile, rows
+that start on any 4-byte boundary, and rows with inf or NaN beside ordinary
+ones."""
+
+import numpy as np
+import pytest
+import torch
+
+import mojodgl.ops as ops
+
+pytestmark = pytest.mark.gpu
+
+KS = [1, 3, 4, 5, 6, 7, 15, 16, 17, 20, 31, 32, 33, 47, 64, 66, 97, 100, 127, 128, 130, 192, 255,
+      256, 257]
+NS = [1, 2, 15, 16, 17, 32, 33, 47, 64, 65, 100, 128, 129, 200, 256]
+
+
+def groups(seed, r=9):
+    """Lengths with empty groups, single rows and just past 32, 128 and 256."""
+    rng = np.random.default_rng(seed)
+    seg = np.array([0, 1, 33, 129, 0, 257, 31, 128, 100 + rng.integers(0, 50)])[:r]
+    return seg, np.repeat(np.arange(r), seg)
+
+
+def inputs(k, n, dtype, seed, lengths):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    rows = int(lengths.sum())
+
+    def draw(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen, dtype=torch.float64).to(dtype)
+
+    return draw(rows, k), draw(len(lengths), k, n), draw(rows, n)
+
+
+def product(a, b, group):
+    return torch.bmm(a.unsqueeze(1), b[group]).squeeze(1)
+
+
+def within(got, ref, bound, terms, dtype):
+    # a sum of `terms` products in any order: terms * eps of their magnitudes,
+    # and the three smallest part products left out (2^-24) for float32
+    tol = (terms + 4) * torch.finfo(dtype).eps
+    off = (got.double() - ref).abs()
+    assert bool((off <= tol * bound + 1e-300).all()), float((off / (bound + 1e-300)).max())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("k,n", [(k, NS[(i * 7 + j * 4) % len(NS)]) for i, k in enumerate(KS)
+                                 for j in range(3)] + [(64, n) for n in NS] + [(16, n) for n in NS])
+def test_products_and_gradients(dtype, k, n):
+    seg, grp = groups(k * 1000 + n)
+    a, b, G = inputs(k, n, dtype, k * 1000 + n, seg)
+    rng = np.random.default_rng(k + n)
+    order = rng.permutation(grp.size)
+    for by in ("segment", "gather"):
+        ids = grp if by == "segment" else grp[order]
+        group = torch.from_numpy(ids).cuda()
+        a.requires_grad_(True)
+        b.requires_grad_(True)
+        z = (ops.segment_mm(a, b, seg) if by == "segment"
+             else ops.gather_mm(a, b, idx_b=group))
+        da, db = torch.autograd.grad(z, (a, b), G)
+        a, b = a.detach(), b.detach()
+        A, B, D = a.double(), b.double(), G.double()
+        within(z.detach(), product(A, B, group), product(A.abs(), B.abs(), group), k, dtype)
+        bt = B.transpose(1, 2).contiguous()
+        within(da, product(D, bt, group), product(D.abs(), bt.abs(), group), n, dtype)
+        ref = torch.zeros_like(B)
+        bound = torch.zeros_like(B)
+        for r in range(len(seg)):
+            rows = (group == r).nonzero().view(-1)
+            ref[r] = A[rows].t().contiguous() @ D[rows]
+            bound[r] = A[rows].abs().t().contiguous() @ D[rows].abs()
+        within(db, ref, bound, int(seg.max()), dtype)
+
+
+@pytest.mark.parametrize("k,n", [(4, 5), (7, 17), (18, 33), (47, 64), (100, 47), (61, 20),
+                                 (130, 40), (255, 100)])
+def test_inf_and_nan_stay_in_their_rows(k, n):
+    """inf, NaN, zero and huge values: their rows as IEEE products give them,
+    the others as without them; the same for a block of b that holds them."""
+    seg, grp = groups(k)
+    a, b, _ = inputs(k, n, torch.float32, k, seg)
+    group = torch.from_numpy(grp).cuda()
+    clean = ops.segment_mm(a, b, seg)
+    for spot, value in ((0, float("inf")), (k - 1, float("nan")), (k - 1, -float("inf")),
+                        (k // 2, 1e38)):
+        x = a.clone()
+        x[5, spot] = value
+        got = ops.segment_mm(x, b, seg)
+        want = product(x.double(), b.double(), group).float()
+        keep = torch.ones(a.shape[0], dtype=torch.bool, device="cuda")
+        keep[5] = False
+        assert torch.equal(torch.isnan(got[5]), torch.isnan(want[5]))
+        assert torch.equal(torch.isinf(got[5]), torch.isinf(want[5]))
+        # rows that shared its wavefront may take the float32 path: same to rounding
+        bound = product(a.double().abs(), b.double().abs(), group)
+        within(got[keep], clean[keep].double(), bound[keep], 2 * k, torch.float32)
+    y = b.clone()
+    y[5, k - 1, n - 1] = float("inf")
+    got = ops.segment_mm(a, y, seg)
+    want = product(a.double(), y.double(), group)
+    rows = (group == 5).nonzero().view(-1)
+    assert torch.equal(torch.isinf(got), torch.isinf(want))
+    assert bool(torch.isinf(got[rows, n - 1]).all())
