@@ -222,6 +222,18 @@ int mdgl_gspmm_selected_sum(const int32_t* indptr, const int32_t* indices, const
                             const int32_t* heavy_ptr, int64_t num_heavy, void* workspace,
                             int64_t workspace_bytes, int flags, int dtype, void* stream);
 
+/* dot[i][h] = sum over the h-th of `groups` equal runs of columns of
+ * lhs[indices[i]] * rowop[row of slot i], for every CSR slot i (rows of d
+ * columns; `groups` values per slot, in slot order): an edge-wise dot between
+ * the endpoints with one of them read once per row. chunk_row / chunk_start as
+ * for mdgl_gspmm; no workspace. flags: MDGL_ANY_ALIGNMENT. MDGL_ENOTSUP for
+ * runs under 16 bytes or over 64 lanes of 16. The same sums in the same order as
+ * mdgl_gsddmm's dot (src/ported.mojo:273-293). */
+int mdgl_gspmm_row_dot(const int32_t* indptr, const int32_t* indices, const void* lhs,
+                       const void* rowop, void* dot, int64_t num_dst, int64_t d, int64_t groups,
+                       const int32_t* chunk_row, const int32_t* chunk_start, int64_t num_chunks,
+                       int32_t chunk_len, int flags, int dtype, void* stream);
+
 /* Workspace mdgl_gspmm needs for `num_chunks` chunk partials. */
 int64_t mdgl_gspmm_workspace_bytes(int64_t num_chunks, int64_t dout, int reduce_op, int dtype);
 

@@ -473,15 +473,16 @@ int mdgl_gsddmm(const int32_t* uids, const int32_t* vids, const void* lhs, const
   }
   const int vw = vec_width(dtype);
   if (dot) {
-    p.vec = (p.red % vw == 0 && dl % vw == 0 && dr % vw == 0 && aligned(lhs, vw * es) &&
-             aligned(rhs, vw * es)) ? vw : 1;
+    p.vec = p.red >= vw ? vw : 1;
     p.lmode = p.rmode = M_CONTIG;
-    p.out_vec = 0;
   } else {
-    p.vec = dout % vw == 0 ? vw : 1;
-    p.lmode = op == OP_COPY_RHS ? M_CONTIG : pick_mode(p.bc, true, dout, p.vec, dl, lhs, es);
-    p.rmode = op == OP_COPY_LHS ? M_CONTIG : pick_mode(p.bc, false, dout, p.vec, dr, rhs, es);
-    p.out_vec = p.vec > 1 && aligned(dst, p.vec * es);
+    // runs of the innermost axis after collapsing the broadcast (gspmm's lanes)
+    const int last = p.bc.nd - 1;
+    p.run_len = p.bc.shape[last];
+    p.vec = p.run_len >= vw ? vw : (p.run_len >= 2 && dtype == MDGL_FLOAT32 ? 2 : 1);
+    p.lpg = (int)((p.run_len + p.vec - 1) / p.vec);
+    p.lmode = op == OP_COPY_RHS || p.bc.lstride[last] == 1 ? M_CONTIG : M_SPLAT;
+    p.rmode = op == OP_COPY_LHS || p.bc.rstride[last] == 1 ? M_CONTIG : M_SPLAT;
   }
   hipError_t e = dtype == MDGL_FLOAT32 ? launch_gsddmm<float>(p) : launch_gsddmm<double>(p);
   return hip_status(e, "gsddmm");
@@ -699,7 +700,8 @@ int gspmm_common(const int32_t* indptr, const int32_t* indices, const int32_t* e
   p.num_heavy = num_heavy;
   p.heavy_rows = heavy_rows;
   p.heavy_ptr = heavy_ptr;
-  if (num_chunks > 0) {
+  const bool dot_only = dot_out && op == OP_COPY_LHS;
+  if (num_chunks > 0 && !dot_only) {
     const int64_t need = mdgl_gspmm_workspace_bytes(num_chunks, dout, reduce_op, dtype);
     if (workspace && !aligned(workspace, WS_ALIGN))
       return fail(MDGL_EINVAL, "workspace must be %lld-byte aligned", (long long)WS_ALIGN);
@@ -728,7 +730,7 @@ int gspmm_common(const int32_t* indptr, const int32_t* indices, const int32_t* e
     // aligned lanes; with it any run of at least 16 bytes, the lanes past the
     // run repeating its last columns and adding nothing
     const int vw = vec_width(dtype);
-    if (op != OP_MUL || reduce_op != RED_SUM)
+    if ((op != OP_MUL && !dot_only) || reduce_op != RED_SUM)
       return fail(MDGL_EINVAL, "gspmm dot: mul with sum only");
     if (!rowop) return fail(MDGL_EINVAL, "gspmm dot: null row operand");
     if (dr <= 0 || dout % dr != 0)
@@ -740,7 +742,7 @@ int gspmm_common(const int32_t* indptr, const int32_t* indices, const int32_t* e
     bool ok = D >= vw && lanes <= WAVE;
     if (!(flags & MDGL_ANY_ALIGNMENT))
       ok = ok && D == lanes * vw && aligned(lhs, vw * es) && aligned(rowop, vw * es);
-    for (int64_t k = 0; ok && k < dout; ++k)
+    for (int64_t k = 0; ok && !dot_only && k < dout; ++k)
       ok = bcast_off(p.bc, k, false) == k / D && bcast_off(p.bc, k, true) == k;
     if (!ok)
       return fail(MDGL_ENOTSUP, "gspmm dot: needs contiguous rows and the edge operand splat "
@@ -863,6 +865,20 @@ int mdgl_coo_locality(const int32_t* u, const int32_t* v, int64_t num_edges, int
   if (num_edges > 0 && (!u || !v)) return fail(MDGL_EINVAL, "coo_locality: null endpoints");
   return hip_status(launch_coo_locality(u, v, num_edges, window, partial, (hipStream_t)stream),
                     "coo_locality");
+}
+
+int mdgl_gspmm_row_dot(const int32_t* indptr, const int32_t* indices, const void* lhs,
+                       const void* rowop, void* dot, int64_t num_dst, int64_t d, int64_t groups,
+                       const int32_t* chunk_row, const int32_t* chunk_start, int64_t num_chunks,
+                       int32_t chunk_len, int flags, int dtype, void* stream) {
+  MDGL_RANGE();
+  if (num_dst > 0 && d > 0 && !dot) return fail(MDGL_EINVAL, "gspmm dot: null dot output");
+  if (flags != MDGL_ANY_ALIGNMENT) return fail(MDGL_EINVAL, "gspmm dot: bad flags");
+  // the heavy-row arrays are for partials, of which there are none
+  return gspmm_common(indptr, indices, nullptr, lhs, nullptr, dot, num_dst, OP_COPY_LHS, d, groups,
+                      d, RED_SUM, nullptr, 0, nullptr, nullptr, nullptr, nullptr, chunk_row,
+                      chunk_start, num_chunks, chunk_len, chunk_row, chunk_row,
+                      num_chunks > 0 ? 1 : 0, nullptr, 0, flags, dtype, stream, rowop, dot);
 }
 
 int mdgl_gspmm_mul_sum_dot_any(const int32_t* indptr, const int32_t* indices, const int32_t* eid,

@@ -1,15 +1,19 @@
 // Edge-parallel kernel behind gsddmm (included once per dtype).
 //
 // Elementwise ops: G consecutive lanes (power of two covering the output
-// row's vectors, at most 64) own one edge, so a wavefront writes 64 / G
+// row's lanes, at most 64) own one edge, so a wavefront writes 64 / G
 // consecutive output rows with coalesced stores; each lane gathers its VEC
 // columns from the two operand rows selected by the targets (u[e], v[e] or
-// e itself). One IEEE operation per element, so the result is bit-identical
+// e itself). As in gspmm the row is cut into runs of columns over which each
+// operand is consecutive or one value, and a run's last lane ends with it, so
+// every access is a whole vector at element alignment. One IEEE operation per element, so the result is bit-identical
 // to the reference's (src/ported.mojo:295-328).
 //
 // dot: G lanes own one (edge, output column) pair and split the contracted
-// axis `red` between them (VEC consecutive elements per lane per step), then
-// add the G lane partials with a butterfly of __shfl_xor; each wavefront
+// axis `red` between them (VEC consecutive elements per lane per step; the
+// last lane's end with the axis, the ones its neighbour holds counting as
+// zero: 67 columns took 64 lanes of one float and 2.5 times as long), then
+// add the G lane partials with a butterfly; each wavefront
 // serves DOT_U rounds of pairs with their loads issued together. The reference keeps
 // W lane partials and reduces them once (ported.mojo:273-293), so the two
 // agree to rounding, not bit for bit.
@@ -28,7 +32,8 @@ struct GsddmmArgs {
   T* out;
   int64_t num_edges, dl, dr, dout, red;
   Bcast bc;
-  int lt, rt, lmode, rmode, out_vec, G, S;
+  int lt, rt, lmode, rmode, G, S;
+  int run_len, lpg, nvec;  // columns per run, lanes per run, lanes per row
   int64_t num_tasks, num_waves, num_blocks;
 };
 
@@ -37,17 +42,14 @@ __device__ __forceinline__ int64_t target_row(int t, const int32_t* u, const int
 }
 
 template <class T, int VEC>
-__device__ __forceinline__ void fetch_rt(const T* __restrict__ row, int mode, const int (&off)[VEC],
+__device__ __forceinline__ void fetch_rt(const T* __restrict__ row, int mode, int off,
                                          T (&x)[VEC]) {
-  if (VEC > 1 && mode == M_CONTIG) {
-    if constexpr (VEC == VecOf<T>::n) load_vec<T>(row + off[0], x);
-  } else if (mode == M_SPLAT) {
-    const T s = row[off[0]];
+  if (mode == M_CONTIG) {
+    load_any<T, VEC>(row + off, x, false);
+  } else {
+    const T s = row[off];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) x[v] = s;
-  } else {
-#pragma unroll
-    for (int v = 0; v < VEC; ++v) x[v] = row[off[v]];
   }
 }
 
@@ -64,19 +66,15 @@ __global__ __launch_bounds__(BLOCK) void gsddmm_kernel(GsddmmArgs<T> a) {
   if (wave >= a.num_waves) return;
   const int G = a.G;
   const int grp = lane / G, gl = lane % G;
-  const int64_t slab = wave % a.S;
+  const int64_t slab = a.S > 1 ? wave % a.S : 0;
   const int64_t per_round = WAVE / G;
-  const int64_t e0 = (wave / a.S) * EW_U * per_round + grp;
-  const int64_t k0 = (slab * G + gl) * VEC;
-  if (k0 >= a.dout) return;
-
-  int loff[VEC], roff[VEC];
-#pragma unroll
-  for (int v = 0; v < VEC; ++v) {
-    const int64_t k = k0 + v < a.dout ? k0 + v : k0;
-    loff[v] = (int)bcast_off(a.bc, k, true);
-    roff[v] = (int)bcast_off(a.bc, k, false);
-  }
+  const int64_t e0 = (a.S > 1 ? wave / a.S : wave) * EW_U * per_round + grp;
+  const int li = (int)slab * G + gl;
+  if (li >= a.nvec) return;
+  const int run = a.lpg == a.nvec ? 0 : li / a.lpg, j = li - run * a.lpg;
+  const int c = j * VEC < a.run_len - VEC ? j * VEC : a.run_len - VEC;
+  const int64_t k0 = (int64_t)run * a.run_len + c;
+  const int loff = (int)bcast_off(a.bc, k0, true), roff = (int)bcast_off(a.bc, k0, false);
   T x[EW_U][VEC], y[EW_U][VEC];
 #pragma unroll
   for (int r = 0; r < EW_U; ++r) {
@@ -101,13 +99,7 @@ __global__ __launch_bounds__(BLOCK) void gsddmm_kernel(GsddmmArgs<T> a) {
       o[v] = message<OP>(xv, yv);
     }
     const int64_t base = e * a.dout + k0;
-    if (VEC > 1 && a.out_vec) {
-      if constexpr (VEC == VecOf<T>::n) store_n_stream<T, VEC>(a.out + base, o);
-    } else {
-#pragma unroll
-      for (int v = 0; v < VEC; ++v)
-        if (k0 + v < a.dout) a.out[base + v] = o[v];
-    }
+    store_stream_any<T, VEC>(a.out + base, o);
   }
 }
 
@@ -117,20 +109,44 @@ __global__ __launch_bounds__(BLOCK) void gsddmm_kernel(GsddmmArgs<T> a) {
 // the first product, so each lane has 2 * DOT_U row loads in flight.
 constexpr int DOT_U = 4;
 
+// VEC elements of two rows from k on; with `tail` (an axis that VEC does not
+// divide, red >= VEC) from min(k, red - VEC) on, those before k zero.
+template <class T, int VEC>
+__device__ __forceinline__ void dot_load(const T* __restrict__ l, const T* __restrict__ r, int64_t k,
+                                         int64_t red, bool tail, T (&x)[VEC], T (&y)[VEC]) {
+  const int64_t at = tail && k > red - VEC ? red - VEC : k;
+  typedef T V __attribute__((ext_vector_type(VEC == 1 ? 2 : VEC), aligned(sizeof(T))));
+  typedef const __attribute__((address_space(1))) V GV;
+  if constexpr (VEC == 1) {
+    x[0] = load_global(l + at);
+    y[0] = load_global(r + at);
+  } else {
+    const V a = *(GV*)(l + at), b = *(GV*)(r + at);
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) {
+      x[v] = a[v];
+      y[v] = b[v];
+    }
+    if (tail) {
+      const int dup = (int)(k - at);
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        x[v] = v < dup ? T(0) : x[v];
+        y[v] = v < dup ? T(0) : y[v];
+      }
+    }
+  }
+}
+
 template <class T, int VEC>
 __device__ __forceinline__ T dot_part(const T* __restrict__ l, const T* __restrict__ r,
                                       int64_t k0, int64_t red, int64_t step) {
   T part = T(0);
   for (int64_t k = k0; k < red; k += step) {
-    if constexpr (VEC > 1) {
-      T xv[VEC], yv[VEC];
-      load_global_n<T, VEC>(l + k, xv);
-      load_global_n<T, VEC>(r + k, yv);
+    T xv[VEC], yv[VEC];
+    dot_load<T, VEC>(l, r, k, red, red % VEC != 0, xv, yv);
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) part = part + xv[v] * yv[v];
-    } else {
-      part = part + load_global(l + k) * load_global(r + k);
-    }
+    for (int v = 0; v < VEC; ++v) part = part + xv[v] * yv[v];
   }
   return part;
 }
@@ -159,7 +175,11 @@ __global__ __launch_bounds__(BLOCK) void gsddmm_dot_kernel(GsddmmArgs<T> a) {
         lp[u] = a.lhs + target_row(a.lt, a.uids, a.vids, task[u]) * a.dl;
         rp[u] = a.rhs + target_row(a.rt, a.uids, a.vids, task[u]) * a.dr;
       } else {
-        const int64_t e = task[u] / a.dout, col = task[u] % a.dout;
+        // (32-bit where it fits: a 64-bit divide is several times the instructions)
+        const int64_t e = a.num_tasks < (int64_t(1) << 32)
+                              ? (int64_t)((uint32_t)task[u] / (uint32_t)a.dout)
+                              : task[u] / a.dout;
+        const int64_t col = task[u] - e * a.dout;
         lp[u] = a.lhs + target_row(a.lt, a.uids, a.vids, e) * a.dl +
                 bcast_off(a.bc, col, true) * a.red;
         rp[u] = a.rhs + target_row(a.rt, a.uids, a.vids, e) * a.dr +
@@ -168,18 +188,13 @@ __global__ __launch_bounds__(BLOCK) void gsddmm_dot_kernel(GsddmmArgs<T> a) {
     }
   }
   T part[DOT_U];
+  const bool tail = a.red % VEC != 0;
   if (a.red <= (int64_t)G * VEC) {
     T xv[DOT_U][VEC], yv[DOT_U][VEC];
 #pragma unroll
     for (int u = 0; u < DOT_U; ++u) {
       if (lp[u] && k0 < a.red) {
-        if constexpr (VEC > 1) {
-          load_global_n<T, VEC>(lp[u] + k0, xv[u]);
-          load_global_n<T, VEC>(rp[u] + k0, yv[u]);
-        } else {
-          xv[u][0] = load_global(lp[u] + k0);
-          yv[u][0] = load_global(rp[u] + k0);
-        }
+        dot_load<T, VEC>(lp[u], rp[u], k0, a.red, tail, xv[u], yv[u]);
       } else {
 #pragma unroll
         for (int v = 0; v < VEC; ++v) xv[u][v] = yv[u][v] = T(0);
@@ -199,8 +214,7 @@ __global__ __launch_bounds__(BLOCK) void gsddmm_dot_kernel(GsddmmArgs<T> a) {
   }
   // butterfly inside the lane group; every lane of the wavefront runs it
 #pragma unroll
-  for (int u = 0; u < DOT_U; ++u)
-    for (int off = G >> 1; off >= 1; off >>= 1) part[u] = part[u] + __shfl_xor(part[u], off);
+  for (int u = 0; u < DOT_U; ++u) part[u] = group_sum(part[u], G);
   if (G >= DOT_U) {
     // the wavefront's DOT_U * 64 / G tasks are consecutive: lane t takes
     // task wave * nt + t from its group's lanes and the results leave as one
@@ -241,7 +255,9 @@ hipError_t launch_gsddmm_vec(const GsddmmParams& p) {
   a.rt = p.rt;
   a.lmode = p.lmode;
   a.rmode = p.rmode;
-  a.out_vec = p.out_vec;
+  a.run_len = (int)p.run_len;
+  a.lpg = p.lpg;
+  a.nvec = p.run_len > 0 ? (int)(p.dout / p.run_len * p.lpg) : 0;
   if (p.op == OP_DOT) {
     const int64_t nvec = (p.red + VEC - 1) / VEC;
     int G = 1;
@@ -252,7 +268,7 @@ hipError_t launch_gsddmm_vec(const GsddmmParams& p) {
     const int64_t per_wave = (WAVE / G) * DOT_U;
     a.num_waves = (a.num_tasks + per_wave - 1) / per_wave;
   } else {
-    const int64_t nvec = (p.dout + VEC - 1) / VEC;
+    const int64_t nvec = a.nvec;
     int G = 1;
     while (G < nvec && G < WAVE) G <<= 1;
     a.G = G;
@@ -284,6 +300,9 @@ hipError_t launch_gsddmm_vec(const GsddmmParams& p) {
 template <class T>
 hipError_t launch_gsddmm(const GsddmmParams& p) {
   if (p.vec == VecOf<T>::n) return launch_gsddmm_vec<T, VecOf<T>::n>(p);
+  if constexpr (VecOf<T>::n == 4) {
+    if (p.vec == 2) return launch_gsddmm_vec<T, 2>(p);
+  }
   return launch_gsddmm_vec<T, 1>(p);
 }
 

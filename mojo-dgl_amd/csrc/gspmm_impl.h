@@ -94,33 +94,6 @@ struct GspmmArgs {
   int64_t row_limit;
 };
 
-// N consecutive elements at element alignment (one 4- to 32-byte access).
-template <class T, int N>
-__device__ __forceinline__ void load_any(const T* p, T (&out)[N], bool stream) {
-  if constexpr (N == 1) {
-    out[0] = stream ? __builtin_nontemporal_load(p) : *p;
-  } else {
-    typedef T V __attribute__((ext_vector_type(N), aligned(sizeof(T))));
-    const V v = stream ? __builtin_nontemporal_load(reinterpret_cast<const V*>(p))
-                       : *reinterpret_cast<const V*>(p);
-#pragma unroll
-    for (int i = 0; i < N; ++i) out[i] = v[i];
-  }
-}
-
-template <class T, int N>
-__device__ __forceinline__ void store_any_stream(T* p, const T (&in)[N]) {
-  if constexpr (N == 1) {
-    *p = in[0];
-  } else {
-    typedef T V __attribute__((ext_vector_type(N), aligned(sizeof(T))));
-    V v;
-#pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = in[i];
-    __builtin_nontemporal_store(v, reinterpret_cast<V*>(p));
-  }
-}
-
 // The VEC columns a lane reads from an operand row (off: their offsets; only
 // off[0] unless the mode is gather). Edge rows are read once per edge and
 // stream past the caches, so they do not displace source rows that other
@@ -163,37 +136,6 @@ __device__ __forceinline__ double row_bcast(double v) {
   return __longlong_as_double(row_bcast<N>((int64_t)__double_as_longlong(v)));
 }
 
-template <class V>
-__device__ __forceinline__ V lane_xor_dpp(V v, int step) {
-  auto mov = [&](int w) {
-    return step == 0   ? __builtin_amdgcn_mov_dpp(w, 0xB1, 0xF, 0xF, false)    // quad [1,0,3,2]
-           : step == 1 ? __builtin_amdgcn_mov_dpp(w, 0x4E, 0xF, 0xF, false)    // quad [2,3,0,1]
-           : step == 2 ? __builtin_amdgcn_mov_dpp(w, 0x141, 0xF, 0xF, false)   // row_half_mirror
-                       : __builtin_amdgcn_mov_dpp(w, 0x140, 0xF, 0xF, false);  // row_mirror
-  };
-  if constexpr (sizeof(V) == 4) {
-    return __builtin_bit_cast(V, mov(__builtin_bit_cast(int, v)));
-  } else {
-    const uint64_t b = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = (uint32_t)mov((int)(uint32_t)b), hi = (uint32_t)mov((int)(b >> 32));
-    return __builtin_bit_cast(V, ((uint64_t)hi << 32) | lo);
-  }
-}
-
-// Sum over groups of `lanes` (a power of two) consecutive lanes, in every
-// lane of the group: the butterfly's partners 1, 2, 4, 8 lanes away by DPP (a
-// mirror stands in for 4 and 8, whose partners already hold equal sums).
-template <class T>
-__device__ __forceinline__ T group_sum(T v, int lanes) {
-  if (lanes > 1) v = v + lane_xor_dpp(v, 0);
-  if (lanes > 2) v = v + lane_xor_dpp(v, 1);
-  if (lanes > 4) v = v + lane_xor_dpp(v, 2);
-  if (lanes > 8) v = v + lane_xor_dpp(v, 3);
-  if (lanes > 16) v = v + __shfl_xor(v, 16);
-  if (lanes > 32) v = v + __shfl_xor(v, 32);
-  return v;
-}
-
 // A lambda kept out of line would put the arrays it captures in memory.
 #define MDGL_INLINE __attribute__((always_inline))
 
@@ -210,13 +152,14 @@ __device__ __forceinline__ void for_each(F f) {
 // How ids reach the lanes of a unit (see the top): by G.
 enum { LAY_ROW = 0, LAY_WIDE = 1 };
 
-template <class T, int OP, int RED, int VEC, int LM, int RM, int LAY, bool DOT = false,
+// DOT: 1 beside the sum, 2 alone (nothing folded or written but the dots).
+template <class T, int OP, int RED, int VEC, int LM, int RM, int LAY, int DOT = 0,
           bool SEL = false>
 __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, int64_t wave,
                                            int lane) {
   // edges in flight per lane: 8 (4 in the dot pass, whose per-edge
   // butterflies already hide the loads; 8 there cost 14 %)
-  constexpr int U = DOT ? 4 : 8;
+  constexpr int U = DOT == 1 ? 4 : 8;
   constexpr bool ARG = (RED == RED_MAX || RED == RED_MIN);
   constexpr bool HAS_L = OP != OP_COPY_RHS, HAS_R = OP != OP_COPY_LHS;
   const int G = LAY == LAY_WIDE ? WAVE : 1 << a.gshift;
@@ -383,9 +326,10 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
       for_each<U>([&](auto iu) MDGL_INLINE {
         if (FULL || decltype(iu)::value < rem) dot(iu);
       });
-    for_each<U>([&](auto iu) MDGL_INLINE {
-      if (FULL || decltype(iu)::value < rem) fold(iu);
-    });
+    if constexpr (DOT != 2)
+      for_each<U>([&](auto iu) MDGL_INLINE {
+        if (FULL || decltype(iu)::value < rem) fold(iu);
+      });
   };
   const int64_t lbytes = a.lstride * (int64_t)sizeof(T), rbytes = a.dr * (int64_t)sizeof(T);
 
@@ -467,7 +411,7 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
     }
   }
 
-  if (!ok || !feat_ok) return;
+  if (DOT == 2 || !ok || !feat_ok) return;
   if (chunk) {
     const int64_t o = unit * a.dout + k0;
 #pragma unroll
@@ -495,13 +439,13 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
       }
   }
   const int64_t o = row * a.dout + k0;
-  store_any_stream<T, VEC>(a.out + o, acc);
+  store_stream_any<T, VEC>(a.out + o, acc);
   if constexpr (ARG) {
     auto put = [&](int32_t* dst, const int32_t* id) {
       int32_t x[VEC];
 #pragma unroll
       for (int v = 0; v < VEC; ++v) x[v] = at[v] >= 0 ? id[at[v]] : -1;
-      store_any_stream<int32_t, VEC>(dst + o, x);
+      store_stream_any<int32_t, VEC>(dst + o, x);
     };
     if (a.arg_u) put(a.arg_u, a.indices);
     if (a.arg_e) put(a.arg_e, a.eid);
@@ -514,10 +458,11 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
 // edge), or any modes. The scalar one is loaded with the ids and broadcast like
 // them: read per lane and edge through the any-modes path it cost a GCN
 // aggregation over 128 columns 4x the time of the same gather without it.
-// P_SEL (copy / sum) adds a gathered value only where the selection's entry is
+// P_DOT (copy / sum) writes only the dots of every gathered row with the row's
+// own. P_SEL (copy / sum) adds a gathered value only where the selection's entry is
 // the edge itself: the gradient of a max or min without a tensor of per-edge
 // gradients in between.
-enum { P_CC = 0, P_CS = 1, P_DYN = 2, P_CS_DOT = 3, P_CW = 4, P_SEL = 5 };
+enum { P_CC = 0, P_CS = 1, P_DYN = 2, P_CS_DOT = 3, P_CW = 4, P_SEL = 5, P_DOT = 6 };
 
 // Wavefronts per SIMD asked of the register allocation: what each path needs
 // plus a few registers would otherwise round down to one wavefront less (98
@@ -551,9 +496,11 @@ gspmm_kernel(GspmmArgs<T> a) {
   else if constexpr (PATH == P_CW)
     gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SCALAR, LAY>(a, chunk, wave, lane);
   else if constexpr (PATH == P_SEL)
-    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_CONTIG, LAY, false, true>(a, chunk, wave, lane);
+    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_CONTIG, LAY, 0, true>(a, chunk, wave, lane);
+  else if constexpr (PATH == P_DOT)
+    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_CONTIG, LAY, 2>(a, chunk, wave, lane);
   else if constexpr (PATH == P_CS_DOT)
-    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SPLAT, LAY, true>(a, chunk, wave, lane);
+    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SPLAT, LAY, 1>(a, chunk, wave, lane);
   else
     gspmm_body<T, OP, RED, VEC, M_DYN, M_DYN, LAY>(a, chunk, wave, lane);
 }
@@ -704,6 +651,17 @@ hipError_t launch_gspmm_op(const GspmmParams& p) {
           hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CS_DOT, LAY_ROW>), grid, block, 0,
                              p.stream, a);
         launched = true;
+      }
+    }
+    if constexpr (OP == OP_COPY_LHS && RED == RED_SUM && VEC == VecOf<T>::n) {
+      if (p.dot_out) {
+        if (G == WAVE)
+          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_DOT, LAY_WIDE>), grid, block, 0,
+                             p.stream, a);
+        else
+          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_DOT, LAY_ROW>), grid, block, 0,
+                             p.stream, a);
+        return hipGetLastError();  // no partials to fold
       }
     }
     if (!launched) {

@@ -154,6 +154,33 @@ __device__ __forceinline__ void load_n_stream(const T* p, T (&out)[N]) {
   for (int i = 0; i < N; ++i) out[i] = v[i];
 }
 
+// N consecutive elements at element alignment (one 4- to 32-byte access).
+template <class T, int N>
+__device__ __forceinline__ void load_any(const T* p, T (&out)[N], bool stream) {
+  if constexpr (N == 1) {
+    out[0] = stream ? __builtin_nontemporal_load(p) : *p;
+  } else {
+    typedef T V __attribute__((ext_vector_type(N), aligned(sizeof(T))));
+    const V v = stream ? __builtin_nontemporal_load(reinterpret_cast<const V*>(p))
+                       : *reinterpret_cast<const V*>(p);
+#pragma unroll
+    for (int i = 0; i < N; ++i) out[i] = v[i];
+  }
+}
+
+template <class T, int N>
+__device__ __forceinline__ void store_stream_any(T* p, const T (&in)[N]) {
+  if constexpr (N == 1) {
+    *p = in[0];
+  } else {
+    typedef T V __attribute__((ext_vector_type(N), aligned(sizeof(T))));
+    V v;
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = in[i];
+    __builtin_nontemporal_store(v, reinterpret_cast<V*>(p));
+  }
+}
+
 template <class T>
 __device__ __forceinline__ T seed(int red) {
   if (red == RED_MAX) return -__builtin_huge_val();
@@ -193,6 +220,37 @@ __device__ __forceinline__ int wave_max_int(int v) {
     int o = __shfl_xor(v, off);
     v = o > v ? o : v;
   }
+  return v;
+}
+
+template <class V>
+__device__ __forceinline__ V lane_xor_dpp(V v, int step) {
+  auto mov = [&](int w) {
+    return step == 0   ? __builtin_amdgcn_mov_dpp(w, 0xB1, 0xF, 0xF, false)    // quad [1,0,3,2]
+           : step == 1 ? __builtin_amdgcn_mov_dpp(w, 0x4E, 0xF, 0xF, false)    // quad [2,3,0,1]
+           : step == 2 ? __builtin_amdgcn_mov_dpp(w, 0x141, 0xF, 0xF, false)   // row_half_mirror
+                       : __builtin_amdgcn_mov_dpp(w, 0x140, 0xF, 0xF, false);  // row_mirror
+  };
+  if constexpr (sizeof(V) == 4) {
+    return __builtin_bit_cast(V, mov(__builtin_bit_cast(int, v)));
+  } else {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)mov((int)(uint32_t)b), hi = (uint32_t)mov((int)(b >> 32));
+    return __builtin_bit_cast(V, ((uint64_t)hi << 32) | lo);
+  }
+}
+
+// Sum over groups of `lanes` (a power of two) consecutive lanes, in every
+// lane of the group: the butterfly's partners 1, 2, 4, 8 lanes away by DPP (a
+// mirror stands in for 4 and 8, whose partners already hold equal sums).
+template <class T>
+__device__ __forceinline__ T group_sum(T v, int lanes) {
+  if (lanes > 1) v = v + lane_xor_dpp(v, 0);
+  if (lanes > 2) v = v + lane_xor_dpp(v, 1);
+  if (lanes > 4) v = v + lane_xor_dpp(v, 2);
+  if (lanes > 8) v = v + lane_xor_dpp(v, 3);
+  if (lanes > 16) v = v + __shfl_xor(v, 16);
+  if (lanes > 32) v = v + __shfl_xor(v, 32);
   return v;
 }
 

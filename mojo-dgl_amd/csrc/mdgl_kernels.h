@@ -52,7 +52,7 @@ struct GspmmParams {
   // optional (mul / sum with the edge operand splat over groups of
   // dot_lanes * vec columns): a feature row per CSR row and, per CSR slot and
   // group, dot_out[slot][group] = sum over the group of lhs[indices[slot]] *
-  // rowop[row]
+  // rowop[row]; with copy_lhs / sum nothing else is computed (dr groups)
   const void* rowop;
   void* dot_out;
   int dot_lanes;
@@ -118,8 +118,9 @@ struct GsddmmParams {
   Bcast bc;
   int lt, rt, op;
   int lmode, rmode;
-  int out_vec;
   int vec;
+  int64_t run_len;  // columns per run of consecutive operand columns (>= vec; not for dot)
+  int lpg;          // lanes per run
   hipStream_t stream;
 };
 

@@ -100,6 +100,8 @@ _SIGNATURES = {
                                 _P, _P, _P, _I64, _I32, _P, _P, _I64, _P, _I64, _C, _P], _C),
     "mdgl_gspmm_mul_sum_dot_any": ([_P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _C, _P,
                                 _P, _P, _P, _I64, _I32, _P, _P, _I64, _P, _I64, _C, _C, _P], _C),
+    "mdgl_gspmm_row_dot": ([_P, _P, _P, _P, _P, _I64, _I64, _I64, _P, _P, _I64, _I32, _C, _C, _P],
+                           _C),
     "mdgl_gspmm_selected_sum": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _P, _P, _I64, _I32, _P, _P,
                                  _I64, _P, _I64, _C, _C, _P], _C),
     "mdgl_segment_reduce": ([_P, _P, _P, _I64, _I64, _C, _I64, _C, _C, _P], _C),

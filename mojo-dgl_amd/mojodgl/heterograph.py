@@ -264,6 +264,7 @@ class DGLGraph(object):
         self._draw = {}
         self._dcsr = {}
         self._locality = None
+        self._dots = 0  # edge dots computed without the CSR (_dot_csr)
         self._launches = {}  # gspmm call shapes seen on this graph (ops/spmm.py)
 
     def _source_locality(self):
@@ -365,6 +366,22 @@ class DGLGraph(object):
             cached = _DeviceCSR(self._device_raw(kind), params)
             self._dcsr[kind] = cached
         return cached
+
+    def _dot_csr(self):
+        """The in-CSR for an edge-wise dot in slot order (ops/sddmm.py), or
+        None while that would have to build it: the first dot of a graph that
+        has none takes the edges as they come, later ones build it (about the
+        time that one of them saves). Nothing is built under HIP graph
+        capture."""
+        csr = self._current_csr("in")
+        if torch.cuda.is_current_stream_capturing():
+            return csr if csr is not None and csr._slot_of_eid is not None else None
+        if csr is None:
+            self._dots += 1
+            if self._dots < 2:
+                return None
+            csr = self._device_csr("in")
+        return csr
 
     def _device_coo(self):
         """int32 GPU copies of the edge endpoints, in edge-id order."""

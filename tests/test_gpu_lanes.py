@@ -170,3 +170,27 @@ def test_selected_sum_is_the_max_gradient(dtype, d, op):
             yy = y.clone().requires_grad_(True)
             want, _ = torch.autograd.grad(ops.gspmm(g, op, red, x, yy), (x, yy), G)
         assert torch.equal(dx, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shape", [(64,), (100,), (3, 67)])
+@pytest.mark.parametrize("swap", [False, True])
+def test_edge_dot_in_slot_order(dtype, shape, swap, monkeypatch):
+    """u_dot_v / v_dot_u computed slot by slot of the in-CSR equal the same
+    dots taken edge by edge, bit for bit; the first call on a graph without a
+    CSR does not build one."""
+    from mojodgl.ops import sddmm
+
+    monkeypatch.setattr(sddmm, "DOT_SLOT_MIN_EDGES", 1)
+    u, v, n = ragged_graph(sum(shape))
+    g = dgl.graph((torch.from_numpy(u).cuda(), torch.from_numpy(v).cuda()), num_nodes=n)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    x, y = (torch.randn(n, *shape, device="cuda", generator=gen, dtype=torch.float64).to(dtype)
+            for _ in range(2))
+    dot = ops.v_dot_u if swap else ops.u_dot_v
+    first = dot(g, x, y)
+    assert g._current_csr("in") is None
+    second = dot(g, x, y)
+    assert g._current_csr("in") is not None and g._current_csr("in")._slot_of_eid is not None
+    assert first.shape == second.shape and torch.equal(first, second)
