@@ -200,6 +200,15 @@ int mdgl_gspmm_layout(int op, int64_t dl, int64_t dr, int64_t dout, int nd,
                       const void* rhs, int flags, int dtype, int64_t* vec, int64_t* group,
                       int64_t* lanes);
 
+/* Graph endpoints given as int64 on the GPU, in one pass: u32 / v32 receive
+ * their low 32 bits, partial[2b], partial[2b + 1] (device int64,
+ * MDGL_COO_INGEST_BLOCKS pairs) the smallest and largest id among workgroup b's
+ * edges (INT64_MAX / INT64_MIN without any), for the caller to check. No
+ * counterpart in the reference (it checks on the host, heterograph.py:45-66). */
+#define MDGL_COO_INGEST_BLOCKS 512
+int mdgl_coo_ingest(const int64_t* u, const int64_t* v, int32_t* u32, int32_t* v32,
+                    int64_t num_edges, int64_t* partial, void* stream);
+
 /* Locality of a graph for mdgl_gspmm's MDGL_NARROW_SLABS: partial[b]
  * (device int64, MDGL_COO_LOCALITY_BLOCKS of them) receives workgroup b's
  * count of the edges i (COO u, v on the GPU, int32) with |u[i] - v[i]| <

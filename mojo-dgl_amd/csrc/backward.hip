@@ -52,9 +52,11 @@ __global__ __launch_bounds__(BLOCK) void rows_by_degree_kernel(const int32_t* __
                                                                T* __restrict__ y, int64_t rows,
                                                                int64_t d) {
   const int64_t total = rows * d;
+  // (a 64-bit divide costs several times the loads around it)
+  const bool small = total < (int64_t(1) << 32);
   for (int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x; i < total;
        i += (int64_t)gridDim.x * BLOCK) {
-    const int64_t r = i / d;
+    const int64_t r = small ? (int64_t)((uint32_t)i / (uint32_t)d) : i / d;
     const int32_t deg = indptr[r + 1] - indptr[r];
     y[i] = x[i] / T(deg > 1 ? deg : 1);
   }

@@ -855,6 +855,19 @@ int mdgl_gspmm_lanes(int op, int64_t dl, int64_t dr, int64_t dout, int nd,
                            vec, group, nullptr);
 }
 
+static_assert(MDGL_COO_INGEST_BLOCKS == COO_INGEST_BLOCKS, "one pair per workgroup");
+
+int mdgl_coo_ingest(const int64_t* u, const int64_t* v, int32_t* u32, int32_t* v32,
+                    int64_t num_edges, int64_t* partial, void* stream) {
+  MDGL_RANGE();
+  if (num_edges < 0) return fail(MDGL_EINVAL, "coo_ingest: negative size");
+  if (!partial) return fail(MDGL_EINVAL, "coo_ingest: null output");
+  if (num_edges > 0 && (!u || !v || !u32 || !v32))
+    return fail(MDGL_EINVAL, "coo_ingest: null endpoints");
+  return hip_status(launch_coo_ingest(u, v, u32, v32, num_edges, partial, (hipStream_t)stream),
+                    "coo_ingest");
+}
+
 static_assert(MDGL_COO_LOCALITY_BLOCKS == COO_LOCALITY_BLOCKS, "one count per workgroup");
 
 int mdgl_coo_locality(const int32_t* u, const int32_t* v, int64_t num_edges, int64_t window,

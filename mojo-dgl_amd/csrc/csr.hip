@@ -324,6 +324,54 @@ hipError_t launch_build_csr(const int32_t* key, const int32_t* other, int64_t nu
   return hipGetLastError();
 }
 
+// u32[i] = u[i], v32[i] = v[i], and per workgroup the smallest and largest id
+// of its edges (partial[2b], partial[2b + 1]): one pass over the endpoints in
+// place of two conversions and a minimum and maximum of each (a mini-batch's
+// graph of 400K edges: 12 launches less).
+__global__ __launch_bounds__(BLOCK) void coo_ingest_kernel(const int64_t* __restrict__ u,
+                                                           const int64_t* __restrict__ v,
+                                                           int32_t* __restrict__ u32,
+                                                           int32_t* __restrict__ v32, int64_t n,
+                                                           int64_t* __restrict__ partial) {
+  __shared__ int64_t lo_s[WAVES_PER_BLOCK], hi_s[WAVES_PER_BLOCK];
+  int64_t lo = INT64_MAX, hi = INT64_MIN;
+  for (int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * BLOCK) {
+    const int64_t a = __builtin_nontemporal_load(u + i), b = __builtin_nontemporal_load(v + i);
+    u32[i] = (int32_t)a;
+    v32[i] = (int32_t)b;
+    lo = a < lo ? a : lo;
+    lo = b < lo ? b : lo;
+    hi = a > hi ? a : hi;
+    hi = b > hi ? b : hi;
+  }
+  for (int off = 32; off >= 1; off >>= 1) {
+    const int64_t l = __shfl_xor((long long)lo, off), h = __shfl_xor((long long)hi, off);
+    lo = l < lo ? l : lo;
+    hi = h > hi ? h : hi;
+  }
+  if ((threadIdx.x & 63) == 0) {
+    lo_s[threadIdx.x >> 6] = lo;
+    hi_s[threadIdx.x >> 6] = hi;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < WAVES_PER_BLOCK; ++w) {
+      lo = lo_s[w] < lo ? lo_s[w] : lo;
+      hi = hi_s[w] > hi ? hi_s[w] : hi;
+    }
+    partial[2 * blockIdx.x] = lo;
+    partial[2 * blockIdx.x + 1] = hi;
+  }
+}
+
+hipError_t launch_coo_ingest(const int64_t* u, const int64_t* v, int32_t* u32, int32_t* v32,
+                             int64_t n, int64_t* partial, hipStream_t s) {
+  hipLaunchKernelGGL(coo_ingest_kernel, dim3(COO_INGEST_BLOCKS), dim3(BLOCK), 0, s, u, v, u32,
+                     v32, n, partial);
+  return hipGetLastError();
+}
+
 hipError_t launch_coo_locality(const int32_t* u, const int32_t* v, int64_t n, int64_t window,
                                int64_t* partial, hipStream_t s) {
   hipLaunchKernelGGL(coo_locality_kernel, dim3(COO_LOCALITY_BLOCKS), dim3(BLOCK), 0, s, u, v, n,

@@ -69,6 +69,12 @@ struct GspmmParams {
 template <class T, int RED>
 hipError_t launch_gspmm_red(const GspmmParams& p);
 
+// int64 endpoints to int32 and per-block smallest and largest ids, into
+// partial[0 .. 2 * COO_INGEST_BLOCKS) (csr.hip).
+constexpr int COO_INGEST_BLOCKS = 512;
+hipError_t launch_coo_ingest(const int64_t* u, const int64_t* v, int32_t* u32, int32_t* v32,
+                             int64_t n, int64_t* partial, hipStream_t s);
+
 // Per-block counts of the edges i with |u[i] - v[i]| < window, into
 // partial[0 .. COO_LOCALITY_BLOCKS) (csr.hip).
 constexpr int COO_LOCALITY_BLOCKS = 1024;

@@ -83,6 +83,10 @@ def chunk_plan(indptr: np.ndarray, chunk_len: int):
     return heavy, ptr, row, start
 
 
+def _longest_row(indptr: np.ndarray) -> int:
+    return int((indptr[1:] - indptr[:-1]).max()) if indptr.size > 1 else 0
+
+
 def split_length(indptr: np.ndarray, chunk_len: int) -> int:
     """The chunk length of a CSR's gspmm schedule: `chunk_len`, or, when no
     row is more than a quarter longer than that, the longest row's length, so
@@ -90,21 +94,27 @@ def split_length(indptr: np.ndarray, chunk_len: int) -> int:
     quarter after its chunks would, and saves the write of its partials and
     their fold (a 50-block community graph whose longest rows hold 513-593
     slots: 3-4 % faster unsplit)."""
-    longest = int((indptr[1:] - indptr[:-1]).max()) if indptr.size > 1 else 0
+    return _split_length(_longest_row(indptr), chunk_len)
+
+
+def _split_length(longest: int, chunk_len: int) -> int:
     if chunk_len < longest <= chunk_len + chunk_len // 4:
         return longest
     return int(chunk_len)
 
 
 class _Chunks:
-    """gspmm heavy-row schedule of one CSR, on the GPU."""
+    """gspmm heavy-row schedule of one CSR, on the GPU. `indptr()` gives its
+    host row pointers, asked for only when the longest row is split."""
 
-    def __init__(self, indptr: np.ndarray, chunk_len: int):
-        heavy, ptr, row, start = chunk_plan(indptr, chunk_len)
+    def __init__(self, indptr, longest: int, chunk_len: int):
         self.chunk_len = int(chunk_len)
-        self.num_heavy = int(heavy.size)
-        self.num_chunks = int(row.size)
-        if heavy.size == 0:
+        self.num_heavy = self.num_chunks = 0
+        if longest > chunk_len:
+            heavy, ptr, row, start = chunk_plan(indptr(), chunk_len)
+            self.num_heavy = int(heavy.size)
+            self.num_chunks = int(row.size)
+        if self.num_heavy == 0:
             self.chunk_row = self.chunk_start = self.heavy_rows = self.heavy_ptr = None
             return
         self.chunk_row = _lib.i32_device(row)
@@ -135,17 +145,54 @@ def build_device_csr(key: torch.Tensor, other, num_rows: int):
     return indptr, indices, eid
 
 
-class _DeviceCSR:
-    """A CSR view on the GPU (int32) with its gspmm and softmax schedules;
-    the host keeps indptr (int64) for the schedules."""
+def _ingest_coo(u, v):
+    """int64 GPU endpoints as (int32 pair, smallest id, largest id): one launch
+    and one small read back, which also waits for the pair."""
+    E = u.shape[0]
+    pair = (torch.empty(E, dtype=torch.int32, device=u.device),
+            torch.empty(E, dtype=torch.int32, device=u.device))
+    part = torch.empty((_lib.COO_INGEST_BLOCKS, 2), dtype=torch.int64, device=u.device)
+    _lib.check(_lib.lib().mdgl_coo_ingest(u.data_ptr(), v.data_ptr(), pair[0].data_ptr(),
+                                          pair[1].data_ptr(), E, part.data_ptr(),
+                                          _lib.stream()), "coo_ingest")
+    part = part.cpu().numpy()
+    return pair, int(part[:, 0].min()), int(part[:, 1].max())
 
-    def __init__(self, arrays, chunk_len):
-        self.host_indptr, self.indptr, self.indices, self.eid = arrays
-        self.chunks = _Chunks(self.host_indptr, split_length(self.host_indptr, chunk_len))
+
+class _RawCSR:
+    """The CSR arrays on the GPU and the longest row; the host row pointers
+    are read back when first asked for (rows to split, pull, host queries: a
+    mini-batch's graph needs none of them)."""
+
+    def __init__(self, indptr, indices, eid):
+        self.indptr, self.indices, self.eid = indptr, indices, eid
+        # the read back also waits for the build, so the arrays can be shared
+        self.longest = int((indptr[1:] - indptr[:-1]).max()) if indptr.shape[0] > 1 else 0
+        self._host = None
+
+    def host_indptr(self):
+        if self._host is None:
+            self._host = self.indptr.cpu().numpy().astype(np.int64)
+        return self._host
+
+
+class _DeviceCSR:
+    """A CSR view on the GPU (int32) with its gspmm and softmax schedules."""
+
+    def __init__(self, raw, chunk_len):
+        self._raw = raw
+        self.indptr, self.indices, self.eid = raw.indptr, raw.indices, raw.eid
+        self.chunks = _Chunks(raw.host_indptr, raw.longest,
+                              _split_length(raw.longest, chunk_len))
         self.params = int(chunk_len)
         self._softmax = {}
         self._slot_of_eid = None
         self._split = {}
+
+    @property
+    def host_indptr(self):
+        """int64 row pointers on the host."""
+        return self._raw.host_indptr()
 
     def chunks_for(self, chunk_len):
         """The heavy-row schedule for another chunk length (cached)."""
@@ -153,7 +200,8 @@ class _DeviceCSR:
             return self.chunks
         got = self._split.get(int(chunk_len))
         if got is None:
-            got = self._split[int(chunk_len)] = _Chunks(self.host_indptr, int(chunk_len))
+            got = self._split[int(chunk_len)] = _Chunks(self._raw.host_indptr,
+                                                        self._raw.longest, int(chunk_len))
         return got
 
     def slot_of_eid(self):
@@ -220,7 +268,11 @@ class DGLGraph(object):
                 raise DGLError("u and v must have the same length")
             E = int(u.numel())
             lo = hi = 0
-            if E:
+            coo = None
+            if E and E < 2 ** 31 and u.dtype == v.dtype == torch.int64 \
+                    and u.device == v.device == _lib.device():
+                coo, lo, hi = _ingest_coo(u.contiguous(), v.contiguous())
+            elif E:
                 lo, hi = torch.stack((torch.minimum(u.min(), v.min()),
                                       torch.maximum(u.max(), v.max()))).tolist()
             if num_nodes is None:
@@ -234,10 +286,12 @@ class DGLGraph(object):
             self._E = E
             self._num_nodes = num_nodes
             self._check_int32()
-            dev = _lib.device()
-            self._dcoo = (u.to(device=dev, dtype=torch.int32).contiguous(),
-                          v.to(device=dev, dtype=torch.int32).contiguous())
-            _lib.settle()
+            if coo is None:
+                dev = _lib.device()
+                coo = (u.to(device=dev, dtype=torch.int32).contiguous(),
+                       v.to(device=dev, dtype=torch.int32).contiguous())
+                _lib.settle()
+            self._dcoo = coo
         else:
             u = i64(u)
             v = i64(v)
@@ -320,7 +374,8 @@ class DGLGraph(object):
             raw = self._draw.get(kind)
             if raw is not None:
                 # read back the GPU build rather than sorting again on the host
-                indptr, indices, eid = raw[0], raw[2].cpu().numpy(), raw[3].cpu().numpy()
+                indptr, indices, eid = (raw.host_indptr(), raw.indices.cpu().numpy(),
+                                        raw.eid.cpu().numpy())
                 self._csr[kind] = (indptr, indices.astype(np.int64), eid.astype(np.int64),
                                    np.diff(indptr))
             else:
@@ -338,15 +393,13 @@ class DGLGraph(object):
             raise DGLError("graphs with 2**31 or more nodes or edges are not supported on the GPU")
 
     def _device_raw(self, kind):
-        """(host int64 indptr, GPU indptr, indices, eid) of the in ("in") or
-        out ("out") CSR, built once on the GPU from the edge endpoints."""
+        """The in ("in") or out ("out") CSR (_RawCSR), built once on the GPU
+        from the edge endpoints."""
         raw = self._draw.get(kind)
         if raw is None:
             u, v = self._device_coo()
             key, other = (v, u) if kind == "in" else (u, v)
-            indptr, indices, eid = build_device_csr(key, other, self._num_nodes)
-            host = indptr.cpu().numpy().astype(np.int64)
-            raw = (host, indptr, indices, eid)
+            raw = _RawCSR(*build_device_csr(key, other, self._num_nodes))
             self._draw[kind] = raw
         return raw
 
