@@ -270,7 +270,7 @@ class DGLGraph(object):
             lo = hi = 0
             coo = None
             if E and E < 2 ** 31 and u.dtype == v.dtype == torch.int64 \
-                    and u.device == v.device == _lib.device():
+                    and u.get_device() == v.get_device() == _lib.current_device():
                 coo, lo, hi = _ingest_coo(u.contiguous(), v.contiguous())
             elif E:
                 lo, hi = torch.stack((torch.minimum(u.min(), v.min()),
