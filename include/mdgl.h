@@ -209,6 +209,20 @@ int mdgl_gspmm_layout(int op, int64_t dl, int64_t dr, int64_t dout, int nd,
 int mdgl_coo_ingest(const int64_t* u, const int64_t* v, int32_t* u32, int32_t* v32,
                     int64_t num_edges, int64_t* partial, void* stream);
 
+/* dst[i] = src[g[i]] for one value per element and a permutation g of 0 .. n - 1
+ * that many blocks are moved by, in two passes through LDS instead of a gather
+ * (a 128-byte line per value). The plan, with src cut into tiles and dst into
+ * regions of MDGL_PERMUTE_TILE elements (the last ones shorter): tmp region r
+ * holds the elements of dst region r, in the order of their number; entry j of
+ * tile t's part of `put` and `pick` says that tmp[put[j]] is element pick[j] of
+ * the tile, sorted by put; `from` gives dst element i as element from[i] of its
+ * region of tmp. Places put outside [0, n) are not checked. tmp: n values of
+ * scratch. No counterpart in the reference. */
+#define MDGL_PERMUTE_TILE 16384
+int mdgl_permute_values(const void* src, const uint16_t* pick, const int32_t* put,
+                        const uint16_t* from, void* tmp, void* dst, int64_t n, int dtype,
+                        void* stream);
+
 /* Locality of a graph for mdgl_gspmm's MDGL_NARROW_SLABS: partial[b]
  * (device int64, MDGL_COO_LOCALITY_BLOCKS of them) receives workgroup b's
  * count of the edges i (COO u, v on the GPU, int32) with |u[i] - v[i]| <

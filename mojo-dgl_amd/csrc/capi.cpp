@@ -365,6 +365,21 @@ int mdgl_scatter_rows(const void* src, const int32_t* idx, void* dst, int64_t n,
                     "scatter_rows");
 }
 
+static_assert(MDGL_PERMUTE_TILE == PERMUTE_TILE, "the plan's tiles are the kernel's");
+
+int mdgl_permute_values(const void* src, const uint16_t* pick, const int32_t* put,
+                        const uint16_t* from, void* tmp, void* dst, int64_t n, int dtype,
+                        void* stream) {
+  MDGL_RANGE();
+  if (!dtype_ok(dtype)) return fail(MDGL_EINVAL, "permute_values: bad dtype %d", dtype);
+  if (n < 0 || n >= (int64_t(1) << 31)) return fail(MDGL_EINVAL, "permute_values: bad size");
+  if (n > 0 && (!src || !pick || !put || !from || !tmp || !dst))
+    return fail(MDGL_EINVAL, "permute_values: null argument");
+  return hip_status(
+      launch_permute_values(src, pick, put, from, tmp, dst, n, dtype, (hipStream_t)stream),
+      "permute_values");
+}
+
 int mdgl_keep_where(const void* mask, const void* src, void* dst, int64_t n, int dtype,
                     void* stream) {
   MDGL_RANGE();

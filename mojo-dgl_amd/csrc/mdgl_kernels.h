@@ -69,6 +69,13 @@ struct GspmmParams {
 template <class T, int RED>
 hipError_t launch_gspmm_red(const GspmmParams& p);
 
+// dst[i] = src[g[i]] for a permutation g planned as pick, put and from
+// (array.hip, mdgl_permute_values).
+constexpr int PERMUTE_TILE = 16384;
+hipError_t launch_permute_values(const void* src, const uint16_t* pick, const int32_t* put,
+                                 const uint16_t* from, void* tmp, void* dst, int64_t n, int dtype,
+                                 hipStream_t s);
+
 // int64 endpoints to int32 and per-block smallest and largest ids, into
 // partial[0 .. 2 * COO_INGEST_BLOCKS) (csr.hip).
 constexpr int COO_INGEST_BLOCKS = 512;

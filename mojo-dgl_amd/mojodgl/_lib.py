@@ -56,6 +56,7 @@ LHS_LINE_ROWS = 8  # mdgl_gspmm: lhs rows copied to start on 128-byte lines
 NARROW_SLABS = 32  # mdgl_gspmm: 32-lane column slabs for wide rows (a local graph)
 ANY_ALIGNMENT = 64  # mdgl_gspmm: 16-byte lanes for odd widths, heads and addresses too
 COO_INGEST_BLOCKS = 512  # pairs written by mdgl_coo_ingest
+PERMUTE_TILE = 16384  # mdgl_permute_values: elements per tile and region of its plan
 COO_LOCALITY_BLOCKS = 1024  # counts written by mdgl_coo_locality
 SEGMENTS_SHORT = 4  # mdgl_segment_reduce: no segment longer than SEGMENT_SPLIT_ROWS
 SEGMENTS_SKIP_LONG = 8  # mdgl_segment_reduce: longer segments left for a LONG_ONLY call
@@ -88,6 +89,7 @@ _SIGNATURES = {
     "mdgl_gspmm_lanes": ([_C, _I64, _I64, _I64, _C, _P, _P, _P, _P, _C, _C, _P, _P], _C),
     "mdgl_gspmm_layout": ([_C, _I64, _I64, _I64, _C, _P, _P, _P, _P, _C, _C, _P, _P, _P], _C),
     "mdgl_coo_ingest": ([_P, _P, _P, _P, _I64, _P, _P], _C),
+    "mdgl_permute_values": ([_P, _P, _P, _P, _P, _P, _I64, _C, _P], _C),
     "mdgl_coo_locality": ([_P, _P, _I64, _I64, _P, _P], _C),
     "mdgl_edge_softmax_positional": ([_P, _I64, _P, _I64, _I64, _P, _P, _I64, _P, _P, _P, _P, _P,
                                       _P, _I64, _C, _P], _C),

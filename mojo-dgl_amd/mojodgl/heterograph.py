@@ -57,6 +57,9 @@ CHUNK_LEN = 512
 # 1 / PULL_FULL_PASS of the edges, else a subgraph of their in-edges
 PULL_ROWS_MAX_DEGREE = 4096
 PULL_FULL_PASS = 8
+# _ValueOrder: elements from which on a plan pays, and gathers before it is built
+VALUE_ORDER_MIN = 1 << 20
+VALUE_ORDER_CALLS = 10
 # a graph is local when at least LOCAL_FRACTION of its edges join nodes whose
 # ids differ by less than LOCAL_WINDOW (the rows whose 512-byte column slabs
 # fill an XCD's 4 MB L2); gspmm then cuts wide rows into narrower slabs
@@ -159,6 +162,66 @@ def _ingest_coo(u, v):
     return pair, int(part[:, 0].min()), int(part[:, 1].max())
 
 
+class _ValueOrder:
+    """One value per element put in the order of a permutation (out[i] =
+    in[gather[i]], `place` its inverse), for a graph whose edge values are
+    moved call after call. The first calls gather; once they have cost about
+    what the plan of mdgl_permute_values takes to build (two radix groupings,
+    a few passes over the indices: VALUE_ORDER_CALLS gathers), it is built
+    and used from then on. 8 bytes per element."""
+
+    def __init__(self, gather, place):
+        self._gather, self._place = gather, place  # `place()` gives the inverse
+        self._calls = 0
+        self._plan = None
+
+    def planned(self):
+        """Whether the plan is there, counting the caller as one who would use
+        it (its build is the caller's, and never under HIP graph capture)."""
+        self._calls += 1
+        if self._plan is None and self._gather.shape[0] >= VALUE_ORDER_MIN \
+                and self._calls > VALUE_ORDER_CALLS \
+                and not torch.cuda.is_current_stream_capturing():
+            self._plan = self._build()
+        return self._plan is not None
+
+    def __call__(self, values, dtype_code):
+        """A new tensor shaped like `values` (n or n x 1, contiguous)."""
+        n = self._gather.shape[0]
+        out = torch.empty_like(values)
+        plan = self._plan
+        if plan is None:
+            _lib.check(_lib.lib().mdgl_gather_rows(values.data_ptr(), self._gather.data_ptr(),
+                                                   out.data_ptr(), n, 1, dtype_code,
+                                                   _lib.stream()), "gather_rows")
+            return out
+        tmp = torch.empty_like(values)
+        pick, put, source = plan
+        _lib.check(_lib.lib().mdgl_permute_values(
+            values.data_ptr(), pick.data_ptr(), put.data_ptr(), source.data_ptr(), tmp.data_ptr(),
+            out.data_ptr(), n, dtype_code, _lib.stream()), "permute_values")
+        return out
+
+    def _build(self):
+        n, dev, size = self._gather.shape[0], self._gather.device, _lib.PERMUTE_TILE
+        parts = -(-n // size)
+        # tmp: the elements by region of the result, in order of their number
+        region = torch.div(self._place(), size, rounding_mode="floor")
+        element = build_device_csr(region, None, parts)[2].long()
+        del region
+        at = torch.empty(n, dtype=torch.int32, device=dev)
+        at[element] = torch.arange(n, dtype=torch.int32, device=dev)
+        source = torch.remainder(at[self._gather.long()], size).to(torch.int16)
+        del at
+        # the places of tmp by tile of the input, in order
+        tile = torch.div(element, size, rounding_mode="floor").to(torch.int32)
+        put = build_device_csr(tile, None, parts)[2]
+        del tile
+        pick = torch.remainder(element[put.long()], size).to(torch.int16)
+        _lib.settle()
+        return pick, put, source
+
+
 class _RawCSR:
     """The CSR arrays on the GPU and the longest row; the host row pointers
     are read back when first asked for (rows to split, pull, host queries: a
@@ -187,6 +250,7 @@ class _DeviceCSR:
         self.params = int(chunk_len)
         self._softmax = {}
         self._slot_of_eid = None
+        self._edge_values = self._slot_values = None
         self._split = {}
 
     @property
@@ -214,6 +278,18 @@ class _DeviceCSR:
             _lib.settle()
             self._slot_of_eid = pos
         return self._slot_of_eid
+
+    def edge_values(self):
+        """_ValueOrder from edge-id order to CSR slot order."""
+        if self._edge_values is None:
+            self._edge_values = _ValueOrder(self.eid, self.slot_of_eid)
+        return self._edge_values
+
+    def slot_values(self):
+        """_ValueOrder from CSR slot order to edge-id order."""
+        if self._slot_values is None:
+            self._slot_values = _ValueOrder(self.slot_of_eid(), lambda: self.eid)
+        return self._slot_values
 
     def softmax_plan(self, slots, chunk_len):
         """Degree-sorted row order, packed edge ids and chunks for a softmax
@@ -428,7 +504,7 @@ class DGLGraph(object):
         capture."""
         csr = self._current_csr("in")
         if torch.cuda.is_current_stream_capturing():
-            return csr if csr is not None and csr._slot_of_eid is not None else None
+            return csr if csr is not None and csr._slot_values is not None else None
         if csr is None:
             self._dots += 1
             if self._dots < 2:

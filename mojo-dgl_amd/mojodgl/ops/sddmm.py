@@ -208,7 +208,7 @@ def gsddmm(g, op, lhs_data, rhs_data, lhs_target="u", rhs_target="v"):
 # edges on, when a dot's rows have this many bytes or more: a destination's row
 # then stays in registers, one gathered row per edge less, for the results'
 # move into edge-id order (128 columns, 20M edges: 3,187 us edge by edge,
-# 1,484 slot by slot and 363 for that move; 2,658 us with the destinations' rows read again from
+# 1,484 slot by slot and for that move 363, later 107 (_ValueOrder); 2,658 us with the destinations' rows read again from
 # cache for every slot)
 DOT_SLOT_MIN_EDGES = 1 << 20
 DOT_SLOT_MIN_ROW = 128
@@ -229,6 +229,10 @@ def _slot_dot(csr, x, y, num_edges, num_nodes, d, dout, fshape, dtype):
     if rc == _lib.ENOTSUP:
         return None
     _lib.check(rc, "gspmm_row_dot")
+    if dout == 1:
+        order = csr.slot_values()
+        order.planned()
+        return order(tmp, code).reshape((num_edges,) + fshape)
     out = torch.empty((num_edges,) + fshape, dtype=tdt, device=gdev)
     _lib.check(lib.mdgl_gather_rows(tmp.data_ptr(), csr.slot_of_eid().data_ptr(), out.data_ptr(),
                                     num_edges, dout, code, st), "gather_rows")

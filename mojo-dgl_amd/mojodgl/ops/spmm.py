@@ -269,21 +269,21 @@ def _run(g, op, reduce_op, lhs_data, rhs_data, replace_inf=False, want_arg=False
         sched = csr.chunks
         if narrow_split and packed and narrow_split < sched.chunk_len:
             sched = csr.chunks_for(narrow_split)
-        if rhs is not None and code not in (OP_COPY_LHS, OP_COPY_RHS) and dr == 1 \
-                and num_edges and (slabs > 1 or (not packed and num_edges >= CSR_ORDER_MIN_EDGES)):
-            # a scalar edge operand read by several column slabs: put it in
-            # CSR slot order once, so every slab streams it; also for rows of
-            # one whole-wavefront slab, whose walk would otherwise wait on a
-            # gather by edge id every 64 slots (256 columns: 3-7 % faster;
-            # packed rows, several to a wavefront, do better without it)
-            perm = torch.empty(num_edges, dtype=tdt, device=gdev)
-            _lib.check(_lib.lib().mdgl_gather_rows(rhs.data_ptr(), csr.eid.data_ptr(),
-                                                   perm.data_ptr(), num_edges, 1, dcode,
-                                                   _lib.stream()),
-                       "gather_rows")
-            rhs = perm
-            flags |= _lib.RHS_CSR_ORDER
+        if rhs is not None and code not in (OP_COPY_LHS, OP_COPY_RHS) and dr == 1 and num_edges \
+                and (slabs > 1 or num_edges >= CSR_ORDER_MIN_EDGES):
+            # a scalar edge operand put in CSR slot order once: read by several
+            # column slabs, every slab then streams it; for one slab of a whole
+            # wavefront the walk would otherwise wait on a gather by edge id
+            # every 64 slots (256 columns: 3-7 % faster); rows packed several to
+            # a wavefront gain only when the order takes no gather itself (a
+            # line per edge either way: 47 columns, 20M edges, forward and
+            # backward 2,283 us by edge id, 1,771 in the planned order)
+            order = csr.edge_values()
+            planned = order.planned()
             replay = False
+            if planned or slabs > 1 or not packed:
+                rhs = order(rhs, dcode)
+                flags |= _lib.RHS_CSR_ORDER
         ws = None
         nbytes = 0
         if sched.num_chunks:
