@@ -355,6 +355,10 @@ constexpr int any_waves(int nb, int km) {
   return nb == 4 || nb * km > 256 ? 2 : (nb == 2 || km == 256 ? 3 : 5);
 }
 
+// Chunks in flight: with one narrow column block two, for a fifth wavefront
+// per SIMD (four chunks would spill there).
+constexpr int any_depth(int nb, int km) { return nb == 1 && km < 256 ? 2 : 4; }
+
 // bt3[g][q][n][k] (bf16 bit patterns): part q of b[g][k_of(k)][n] (of
 // b[g][n][k_of(k)] with `given_t`), zero where k_of gives none. Workgroup (g, s) splits slice s of
 // group g's N x Kp values and sets flags[g * slices + s] when the slice holds
@@ -630,7 +634,7 @@ __global__ __launch_bounds__(SB_THREADS, 1) void grouped_gemm_split_kernel(
 // products of 2.5M rows take 85 us of MFMA against 0.3 ms of traffic. The
 // general kernel moved the same rows through LDS a float at a time with
 // float32 MFMAs on 128-column tiles. Before and after, us: 100 x 47 (2.5M rows)
-// with both gradients 3,168 -> 1,576; 16 x 16 over 29.5M rows 4,969 -> 856;
+// with both gradients 3,168 -> 1,254; 16 x 16 over 29.5M rows 4,969 -> 856;
 // 128 -> 64 over 1.7M rows (the split kernel before) 422 -> 386.
 //
 // Work mapping. A workgroup of NW wavefronts holds the group's b block (NB
@@ -638,8 +642,11 @@ __global__ __launch_bounds__(SB_THREADS, 1) void grouped_gemm_split_kernel(
 // contiguous range of 32 NW-row tiles; wavefront w owns 32 rows of a tile and
 // all NB blocks. The block is small (14 to 104 KB), so up to eight workgroups
 // share a CU and their wavefronts cover each other's waits: the loads of a row
-// run only two 16-deep chunks ahead, without the split kernel's exact wait
-// counts.
+// run four 16-deep chunks ahead (two with one narrow block), without the split
+// kernel's exact wait counts. Two chunks requested at a time instead of one:
+// 100 x 47 392 us instead of 454 (2.5M rows; the L1 asked the L2 for
+// 2.75 times the rows' lines before), with the last 1 to 3 columns of a row in
+// one store instead of one each (40% of the write requests) included.
 //
 // K axis. Lane (lr, hf) reads chunk c of its row as two 4-float pieces at
 // 16c + 8hf and 4 floats on, at the row's own alignment. A piece that would
@@ -655,6 +662,10 @@ __global__ __launch_bounds__(64 * NW, any_waves(NB, KMAX)) void grouped_gemm_any
   typedef float f32x16 __attribute__((ext_vector_type(16)));
   constexpr int LD = KMAX + 8;  // bf16 per LDS row: an odd number of 16-byte pieces
   constexpr int NC = 32 * NB, NT = 64 * NW, TM = 32 * NW;
+  // chunks of a row in flight: four, requested in pairs (a pair is a 128-byte
+  // line or two of each row, which an L1 shared by a dozen wavefronts' 32 rows
+  // does not keep until the next chunk), where the registers allow
+  constexpr int D = any_depth(NB, KMAX);
   __shared__ __align__(16) uint16_t Bs[3][NC][LD];
   const int t = threadIdx.x;
   const int lane = t & 63, w = t >> 6;
@@ -668,6 +679,7 @@ __global__ __launch_bounds__(64 * NW, any_waves(NB, KMAX)) void grouped_gemm_any
   const int nch = (int)((p.K + 15) / 16);
   const int full = (int)(p.K / 16);  // chunks wholly inside a row
   const int K = (int)p.K;
+  const int rem = (int)(p.N & 3);  // columns of a row's last piece, 0: four
 
   // the row of a behind tile row 32w + lr of tile tl in group gg (-1: none)
   auto row_of = [&](int64_t tl, int64_t gg) -> int32_t {
@@ -706,9 +718,10 @@ __global__ __launch_bounds__(64 * NW, any_waves(NB, KMAX)) void grouped_gemm_any
   }
   int32_t rid = row_of(tile, g);
   const float* row = p.a + (int64_t)(rid < 0 ? 0 : rid) * p.K;
-  float af[2][8];
-  load_chunk(row, 0, af[0]);
-  if (nch > 1) load_chunk(row, 1, af[1]);
+  float af[D][8];
+#pragma unroll
+  for (int i = 0; i < D; ++i)
+    if (i == 0 || i < nch) load_chunk(row, i, af[i]);
 
   int64_t cur_g = -1;
   bool b_whole = false;  // the group's b block has a value that does not split
@@ -746,7 +759,7 @@ __global__ __launch_bounds__(64 * NW, any_waves(NB, KMAX)) void grouped_gemm_any
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
-    auto step = [&](float (&x)[8], int c, int slot) __attribute__((always_inline)) {
+    auto step = [&](float (&x)[8], int c) __attribute__((always_inline)) {
       if (c >= full) {
 #pragma unroll
         for (int i = 0; i < 8; ++i)
@@ -793,14 +806,29 @@ __global__ __launch_bounds__(64 * NW, any_waves(NB, KMAX)) void grouped_gemm_any
           }
         }
       }
-      // the chunk's values are used: request the one two on, or the next
-      // tile's first ones
-      if (c + 2 < nch) load_chunk(row, c + 2, x);
-      else if (slot < nch) load_chunk(row1, slot, x);
     };
-    for (int c = 0; c < nch; c += 2) {
-      step(af[0], c, 0);
-      if (c + 1 < nch) step(af[1], c + 1, 1);
+    // chunk c's values are used: request the one D on, or the next tile's
+    auto refill = [&](float (&x)[8], int c, int slot) __attribute__((always_inline)) {
+      const bool more = c + D < nch;
+      if constexpr (D == 2) {
+        if (more) load_chunk(row, c + D, x);
+        else load_chunk(row1, slot, x);
+      } else {
+        load_chunk(more ? row : row1, more ? c + D : slot, x);
+      }
+    };
+    for (int c = 0; c < nch; c += D) {
+#pragma unroll
+      for (int i = 0; i < D; i += 2) {
+        const int c0 = c + i;
+        if (i > 0 && c0 >= nch) break;
+        const bool two = c0 + 1 < nch;
+        step(af[i], c0);
+        if (D == 2) refill(af[i], c0, i);
+        if (two) step(af[i + 1], c0 + 1);
+        if (D > 2) refill(af[i], c0, i);
+        if (two) refill(af[i + 1], c0 + 1, i + 1);
+      }
     }
     // lane (lr, hf) holds column lr of rows 8q + 4hf + r in acc[j][4q + r];
     // the quad transpose gives lane 4 k4 + s4 row 8q + 4hf + s4 at columns
@@ -820,10 +848,14 @@ __global__ __launch_bounds__(64 * NW, any_waves(NB, KMAX)) void grouped_gemm_any
           if (n + 4 <= p.N) {
             typedef float V __attribute__((ext_vector_type(4), aligned(4)));
             *reinterpret_cast<V*>(o) = V{x[0], x[1], x[2], x[3]};
+          } else if (rem == 3) {
+            typedef float V __attribute__((ext_vector_type(3), aligned(4)));
+            *reinterpret_cast<V*>(o) = V{x[0], x[1], x[2]};
+          } else if (rem == 2) {
+            typedef float V __attribute__((ext_vector_type(2), aligned(4)));
+            *reinterpret_cast<V*>(o) = V{x[0], x[1]};
           } else {
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-              if (n + v < p.N) o[v] = x[v];
+            o[0] = x[0];
           }
         }
       }
@@ -1318,9 +1350,9 @@ int64_t grouped_workspace_bytes(int64_t n, int64_t K, int64_t N, int64_t R, bool
 
 // grouped_gemm_any_kernel's instance for a shape: column blocks, LDS depth,
 // wavefronts, and workgroups per CU (what 160 KB of LDS and the registers
-// allow). Four column blocks only for K of 65 to 128: beyond, they would need
-// more LDS than a CU has, and below, two blocks twice (a is then the smaller
-// side, read again from L2) leave more wavefronts to a SIMD.
+// allow). Four column blocks past 64 columns, so that a row is read and split
+// once (47 x 100 over 2.5M rows, us: two blocks twice 523, four 348), but not
+// for K past 128, where they would need more LDS than a CU has.
 struct AnyShape {
   int nb, km, nw, per_cu;
 };
@@ -1329,9 +1361,9 @@ inline AnyShape any_shape(int64_t K, int64_t N) {
   AnyShape s;
   const int64_t k16 = (K + 15) / 16 * 16;
   s.km = k16 <= 64 ? 64 : (k16 <= 128 ? 128 : 256);
-  s.nb = N <= 32 ? 1 : (N <= 64 || s.km != 128 ? 2 : 4);
+  s.nb = N <= 32 ? 1 : (N <= 64 || s.km == 256 ? 2 : 4);
   const int lds = 3 * 32 * s.nb * (s.km + 8) * 2;
-  s.nw = lds > (54 << 10) ? 8 : 4;
+  s.nw = lds > (56 << 10) ? 8 : 4;
   s.per_cu = (160 << 10) / lds;
   const int waves = 4 * any_waves(s.nb, s.km);
   if (s.per_cu > waves / s.nw) s.per_cu = waves / s.nw;
@@ -1421,6 +1453,7 @@ hipError_t launch_grouped(const GemmLaunch& L, bool gather) {
       MDGL_ANY_CASE(2, 64, 4)
       MDGL_ANY_CASE(2, 128, 4)
       MDGL_ANY_CASE(2, 256, 8)
+      MDGL_ANY_CASE(4, 64, 4)
       MDGL_ANY_CASE(4, 128, 8)
 #undef MDGL_ANY_CASE
       return hipGetLastError();
@@ -1513,10 +1546,11 @@ hipError_t launch_grouped(const GemmLaunch& L, bool gather) {
 // instruction): in a step lane (li, h) supplies a[row h][m0 + 16 i + li] as A^T
 // and grad[row h][n0 + 16 j + li] as B, so the operands are read straight from
 // the rows, 64 consecutive bytes of each, into registers (no LDS, no barrier,
-// any width and alignment), one step of 4 U rows ahead of their use. A
+// any width and alignment), two steps of 4 U rows ahead of their use (one step
+// ahead, copied to the current one, waited for its loads at once). A
 // wavefront holds a tile of MB x NBK blocks of 16 x 16 in registers, sized to the
 // product (a 128 x 128 tile through LDS multiplied mostly zeros for narrower
-// ones: 100 x 47 over 2.5M rows took 1,306 us, here 440).
+// ones: 100 x 47 over 2.5M rows took 1,306 us, here 413; 453 on 8 blocks a step ahead).
 // Products of several tiles: up to TW of them go to different wavefronts of
 // the workgroup, which read the same rows through its L1; the remaining
 // wavefronts (4 / TW streams) take alternate steps of the rows, and their
@@ -1615,19 +1649,27 @@ __global__ __launch_bounds__(BLOCK, MB * NBK * (int)sizeof(T) > 64 ? 2 : 3) void
         for (int j = 0; j < NBK; ++j) acc[i][j] = M::step(x[i], y[j], acc[i][j]);
     }
   };
+  // two steps in flight behind the one multiplied, each in registers of its
+  // own (a copy from one to the next would wait for the loads it copies)
   const int64_t stride = 4 * U * streams;
   int64_t pos = r0 + 4 * U * stream;
   if (pos < r_end) {  // uniform per wavefront
-    Step cur, nxt;
+    Step ring[3];
     int32_t r[U];
     rows(pos, r);
-    load(r, cur);
-    rows(pos + stride, r);  // the next step's rows, requested a step ahead of its loads
-    for (; pos < r_end; pos += stride) {
-      load(r, nxt);
-      rows(pos + 2 * stride, r);
-      multiply(cur, pos);
-      cur = nxt;
+    load(r, ring[0]);
+    rows(pos + stride, r);
+    load(r, ring[1]);
+    rows(pos + 2 * stride, r);  // a step's rows, requested a step ahead of its loads
+    while (pos < r_end) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        load(r, ring[(k + 2) % 3]);
+        rows(pos + 3 * stride, r);
+        multiply(ring[k], pos);
+        pos += stride;
+        if (pos >= r_end) break;
+      }
     }
   }
 
@@ -1766,12 +1808,25 @@ hipError_t launch_grouped_grad(const GemmGradLaunch& L, bool gather) {
         got = sizes[k];
     return got;
   };
-  static constexpr int MS4[] = {8, 4, 2}, NS4[] = {4, 3, 2, 1}, MS8[] = {4, 2}, NS8[] = {4, 2, 1};
-  const int mb = sizeof(T) == 4 ? best(b1, MS4, 3) : best(b1, MS8, 2);
+  static constexpr int MS4[] = {8, 7, 6, 5, 4, 3, 2}, NS4[] = {4, 3, 2, 1};
+  static constexpr int MS8[] = {4, 2}, NS8[] = {4, 2, 1};
+  int mb = sizeof(T) == 4 ? best(b1, MS4, 7) : best(b1, MS8, 2);
   const int nb = sizeof(T) == 4 ? best(b2, NS4, 4) : best(b2, NS8, 3);
   a.tiles_n = (int)((b2 + nb - 1) / nb);
-  a.tiles = (int)((b1 + mb - 1) / mb) * a.tiles_n;
-  a.tw = a.tiles > 2 ? 4 : a.tiles;
+  auto cut = [&] {
+    a.tiles = (int)((b1 + mb - 1) / mb) * a.tiles_n;
+    a.tw = a.tiles > 2 ? 4 : a.tiles;
+    return max_chunks * ((a.tiles + a.tw - 1) / a.tw);
+  };
+  // several tiles and fewer workgroups than two per CU: tiles of 2, 4 or 8
+  // blocks, which are more of them (208 x 130 over 32K rows of 105 groups, us:
+  // 7-block tiles 63, 2-block ones 55; 152 x 246 over 771K rows the other way
+  // round, 3,305 with 2-block tiles for the step and 2,890 with 5-block ones)
+  static constexpr int MS4_FEW[] = {8, 4, 2};
+  if (cut() < 512 && sizeof(T) == 4 && b1 > 8) {
+    mb = best(b1, MS4_FEW, 3);
+    cut();
+  }
   const dim3 grid((unsigned)max_chunks, (unsigned)((a.tiles + a.tw - 1) / a.tw));
 #define MDGL_TN_CASE(M, N)                                                                    \
   if (mb == M && nb == N) {                                                                   \
@@ -1782,6 +1837,10 @@ hipError_t launch_grouped_grad(const GemmGradLaunch& L, bool gather) {
   }
   if constexpr (sizeof(T) == 4) {
     MDGL_TN_CASE(8, 4) MDGL_TN_CASE(8, 3) MDGL_TN_CASE(8, 2) MDGL_TN_CASE(8, 1)
+    MDGL_TN_CASE(7, 4) MDGL_TN_CASE(7, 3) MDGL_TN_CASE(7, 2) MDGL_TN_CASE(7, 1)
+    MDGL_TN_CASE(6, 4) MDGL_TN_CASE(6, 3) MDGL_TN_CASE(6, 2) MDGL_TN_CASE(6, 1)
+    MDGL_TN_CASE(5, 4) MDGL_TN_CASE(5, 3) MDGL_TN_CASE(5, 2) MDGL_TN_CASE(5, 1)
+    MDGL_TN_CASE(3, 4) MDGL_TN_CASE(3, 3) MDGL_TN_CASE(3, 2) MDGL_TN_CASE(3, 1)
     MDGL_TN_CASE(4, 3) MDGL_TN_CASE(2, 3)
   }
   MDGL_TN_CASE(4, 4) MDGL_TN_CASE(4, 2) MDGL_TN_CASE(4, 1)

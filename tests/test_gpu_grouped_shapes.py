@@ -48,7 +48,12 @@ def within(got, ref, bound, terms, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("k,n", [(k, NS[(i * 7 + j * 4) % len(NS)]) for i, k in enumerate(KS)
-                                 for j in range(3)] + [(64, n) for n in NS] + [(16, n) for n in NS])
+                                 for j in range(3)] + [(64, n) for n in NS] + [(16, n) for n in NS]
+                         # four column blocks of a narrow K, each length of a
+                         # row's last piece; gradient tiles of 3, 5, 6 and 7
+                         # blocks whole and cut
+                         + [(47, 100), (17, 66), (50, 131), (5, 257), (48, 15), (80, 47), (79, 33),
+                            (96, 64), (95, 18), (112, 49), (111, 16)])
 def test_products_and_gradients(dtype, k, n):
     seg, grp = groups(k * 1000 + n)
     a, b, G = inputs(k, n, dtype, k * 1000 + n, seg)
