@@ -162,16 +162,27 @@ def _ingest_coo(u, v):
     return pair, int(part[:, 0].min()), int(part[:, 1].max())
 
 
+def _inverse_permutation(index):
+    """The int32 permutation p with p[index[i]] = i."""
+    n = index.shape[0]
+    out = torch.empty(n, dtype=torch.int32, device=index.device)
+    out[index.to(torch.int64)] = torch.arange(n, dtype=torch.int32, device=index.device)
+    return out
+
+
 class _ValueOrder:
     """One value per element put in the order of a permutation (out[i] =
-    in[gather[i]], `place` its inverse), for a graph whose edge values are
-    moved call after call. The first calls gather; once they have cost about
+    in[gather[i]], `inverse` the inverse permutation where the caller has it),
+    for a graph whose edge values are moved call after call. It holds index
+    tensors only, nothing that leads back to the CSR which holds it: a graph's
+    GPU memory is given back with its last reference, not with a later pass of
+    the cyclic collector. The first calls gather; once they have cost about
     what the plan of mdgl_permute_values takes to build (two radix groupings,
     a few passes over the indices: VALUE_ORDER_CALLS gathers), it is built
     and used from then on. 8 bytes per element."""
 
-    def __init__(self, gather, place):
-        self._gather, self._place = gather, place  # `place()` gives the inverse
+    def __init__(self, gather, inverse=None):
+        self._gather, self._inverse = gather, inverse
         self._calls = 0
         self._plan = None
 
@@ -205,8 +216,11 @@ class _ValueOrder:
     def _build(self):
         n, dev, size = self._gather.shape[0], self._gather.device, _lib.PERMUTE_TILE
         parts = -(-n // size)
+        inverse = self._inverse
+        if inverse is None:
+            inverse = _inverse_permutation(self._gather)
         # tmp: the elements by region of the result, in order of their number
-        region = torch.div(self._place(), size, rounding_mode="floor")
+        region = torch.div(inverse, size, rounding_mode="floor")
         element = build_device_csr(region, None, parts)[2].long()
         del region
         at = torch.empty(n, dtype=torch.int32, device=dev)
@@ -271,10 +285,7 @@ class _DeviceCSR:
     def slot_of_eid(self):
         """The inverse of `eid`: the CSR slot of every edge id (cached)."""
         if self._slot_of_eid is None:
-            E = self.eid.shape[0]
-            pos = torch.empty(E, dtype=torch.int32, device=self.eid.device)
-            pos[self.eid.to(torch.int64)] = torch.arange(E, dtype=torch.int32,
-                                                         device=self.eid.device)
+            pos = _inverse_permutation(self.eid)
             _lib.settle()
             self._slot_of_eid = pos
         return self._slot_of_eid
@@ -282,13 +293,13 @@ class _DeviceCSR:
     def edge_values(self):
         """_ValueOrder from edge-id order to CSR slot order."""
         if self._edge_values is None:
-            self._edge_values = _ValueOrder(self.eid, self.slot_of_eid)
+            self._edge_values = _ValueOrder(self.eid, self._slot_of_eid)
         return self._edge_values
 
     def slot_values(self):
         """_ValueOrder from CSR slot order to edge-id order."""
         if self._slot_values is None:
-            self._slot_values = _ValueOrder(self.slot_of_eid(), lambda: self.eid)
+            self._slot_values = _ValueOrder(self.slot_of_eid(), self.eid)
         return self._slot_values
 
     def softmax_plan(self, slots, chunk_len):
