@@ -163,10 +163,22 @@ def _ingest_coo(u, v):
 
 
 def _inverse_permutation(index):
-    """The int32 permutation p with p[index[i]] = i."""
+    """The int32 permutation p with p[index[i]] = i (by an int32 scatter:
+    torch's own indexing would first take a copy of `index` in int64)."""
     n = index.shape[0]
     out = torch.empty(n, dtype=torch.int32, device=index.device)
-    out[index.to(torch.int64)] = torch.arange(n, dtype=torch.int32, device=index.device)
+    src = torch.arange(n, dtype=torch.int32, device=index.device)
+    # rows of one 32-bit value, moved as they are
+    _lib.check(_lib.lib().mdgl_scatter_rows(src.data_ptr(), index.data_ptr(), out.data_ptr(), n, 1,
+                                            0, _lib.stream()), "scatter_rows")
+    return out
+
+
+def _take(values, index):
+    """values[index] of int32 tensors, likewise."""
+    out = torch.empty(index.shape[0], dtype=torch.int32, device=index.device)
+    _lib.check(_lib.lib().mdgl_gather_rows(values.data_ptr(), index.data_ptr(), out.data_ptr(),
+                                           index.shape[0], 1, 0, _lib.stream()), "gather_rows")
     return out
 
 
@@ -185,53 +197,65 @@ class _ValueOrder:
         self._gather, self._inverse = gather, inverse
         self._calls = 0
         self._plan = None
+        self._declined = False
 
     def planned(self):
         """Whether the plan is there, counting the caller as one who would use
-        it (its build is the caller's, and never under HIP graph capture)."""
+        it (its build is the caller's, and never under HIP graph capture). A
+        plan that the GPU's memory has no room for is given up: the call, and
+        the ones after it, gather as before."""
         self._calls += 1
-        if self._plan is None and self._gather.shape[0] >= VALUE_ORDER_MIN \
+        if self._plan is None and not self._declined \
+                and self._gather.shape[0] >= VALUE_ORDER_MIN \
                 and self._calls > VALUE_ORDER_CALLS \
                 and not torch.cuda.is_current_stream_capturing():
-            self._plan = self._build()
+            try:
+                self._plan = self._build()
+            except torch.OutOfMemoryError:
+                self._declined = True
         return self._plan is not None
 
     def __call__(self, values, dtype_code):
         """A new tensor shaped like `values` (n or n x 1, contiguous)."""
         n = self._gather.shape[0]
         out = torch.empty_like(values)
-        plan = self._plan
-        if plan is None:
+        tmp = None
+        if self._plan is not None:
+            try:
+                tmp = torch.empty_like(values)
+            except torch.OutOfMemoryError:
+                pass  # a gather needs no second buffer
+        if tmp is None:
             _lib.check(_lib.lib().mdgl_gather_rows(values.data_ptr(), self._gather.data_ptr(),
                                                    out.data_ptr(), n, 1, dtype_code,
                                                    _lib.stream()), "gather_rows")
             return out
-        tmp = torch.empty_like(values)
-        pick, put, source = plan
+        pick, put, source = self._plan
         _lib.check(_lib.lib().mdgl_permute_values(
             values.data_ptr(), pick.data_ptr(), put.data_ptr(), source.data_ptr(), tmp.data_ptr(),
             out.data_ptr(), n, dtype_code, _lib.stream()), "permute_values")
         return out
 
     def _build(self):
-        n, dev, size = self._gather.shape[0], self._gather.device, _lib.PERMUTE_TILE
-        parts = -(-n // size)
+        size = _lib.PERMUTE_TILE  # a power of two
+        shift = size.bit_length() - 1
+        parts = -(-self._gather.shape[0] // size)
         inverse = self._inverse
         if inverse is None:
             inverse = _inverse_permutation(self._gather)
         # tmp: the elements by region of the result, in order of their number
-        region = torch.div(inverse, size, rounding_mode="floor")
-        element = build_device_csr(region, None, parts)[2].long()
+        region = torch.bitwise_right_shift(inverse, shift)
+        del inverse
+        element = build_device_csr(region, None, parts)[2]
         del region
-        at = torch.empty(n, dtype=torch.int32, device=dev)
-        at[element] = torch.arange(n, dtype=torch.int32, device=dev)
-        source = torch.remainder(at[self._gather.long()], size).to(torch.int16)
+        at = _inverse_permutation(element)
+        source = _take(at, self._gather).bitwise_and_(size - 1).to(torch.int16)
         del at
         # the places of tmp by tile of the input, in order
-        tile = torch.div(element, size, rounding_mode="floor").to(torch.int32)
+        tile = torch.bitwise_right_shift(element, shift)
         put = build_device_csr(tile, None, parts)[2]
         del tile
-        pick = torch.remainder(element[put.long()], size).to(torch.int16)
+        pick = _take(element, put).bitwise_and_(size - 1).to(torch.int16)
         _lib.settle()
         return pick, put, source
 
@@ -405,7 +429,7 @@ class DGLGraph(object):
         self._draw = {}
         self._dcsr = {}
         self._locality = None
-        self._dots = 0  # edge dots computed without the CSR (_dot_csr)
+        self._dots = 0  # edge dots computed without the CSR, -1: all are (_dot_csr)
         self._launches = {}  # gspmm call shapes seen on this graph (ops/spmm.py)
 
     def _source_locality(self):
@@ -512,7 +536,9 @@ class DGLGraph(object):
         None while that would have to build it: the first dot of a graph that
         has none takes the edges as they come, later ones build it (about the
         time that one of them saves). Nothing is built under HIP graph
-        capture."""
+        capture, nor again after its memory could not be had."""
+        if self._dots < 0:
+            return None
         csr = self._current_csr("in")
         if torch.cuda.is_current_stream_capturing():
             return csr if csr is not None and csr._slot_values is not None else None

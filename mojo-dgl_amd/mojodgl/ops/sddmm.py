@@ -186,12 +186,17 @@ def gsddmm(g, op, lhs_data, rhs_data, lhs_target="u", rhs_target="v"):
     if op == "dot" and num_edges >= DOT_SLOT_MIN_EDGES and L.shape[1:] == R.shape[1:] \
             and dtype.itemsize * dl >= DOT_SLOT_MIN_ROW * dout \
             and {lhs_target, rhs_target} == {"u", "v"}:
-        csr = g._dot_csr()
-        if csr is not None:
-            out = _slot_dot(csr, *((lhs, rhs) if lhs_target == "u" else (rhs, lhs)), num_edges,
-                            num_nodes, dl, dout, tuple(fshape), dtype)
-            if out is not None:
-                return _lib.give_back(out, as_torch, dev)
+        try:
+            csr = g._dot_csr()
+            out = None if csr is None else _slot_dot(
+                csr, *((lhs, rhs) if lhs_target == "u" else (rhs, lhs)), num_edges, num_nodes, dl,
+                dout, tuple(fshape), dtype)
+        except torch.OutOfMemoryError:
+            # no room for the CSR, its slot order or the second set of results:
+            # edge by edge below, which needs none of them, from now on
+            g._dots, out = -1, None
+        if out is not None:
+            return _lib.give_back(out, as_torch, dev)
     uids, vids = g._device_coo()
     # allocated in its final shape: the same row-major bytes as (E, dout)
     out = torch.empty((num_edges,) + tuple(fshape), dtype=_lib.torch_dtype(dtype),

@@ -1,19 +1,25 @@
 """The orders a CSR keeps for moving edge values (heterograph._ValueOrder),
-host side: their lifetime, on CPU index tensors."""
+their lifetime on CPU index tensors, and what is left where the GPU's memory
+has no room for them."""
 
 import gc
 import weakref
 
+import numpy as np
 import pytest
 import torch
 
+import mojodgl as dgl
 import mojodgl.heterograph as hg
+import mojodgl.ops as ops
 from mojodgl import _lib
 
 
 @pytest.fixture
 def csr(monkeypatch):
     monkeypatch.setattr(_lib, "settle", lambda: None)
+    monkeypatch.setattr(hg, "_inverse_permutation",
+                        lambda p: torch.argsort(p.long()).to(torch.int32))
     indptr = torch.tensor([0, 2, 3, 5], dtype=torch.int32)
     indices = torch.tensor([0, 1, 2, 1, 0], dtype=torch.int32)
     eid = torch.tensor([3, 0, 4, 2, 1], dtype=torch.int32)
@@ -36,3 +42,67 @@ def test_orders_do_not_outlive_their_csr(csr):
         assert gone() is None
     finally:
         gc.enable()
+
+
+def test_a_plan_without_room_is_given_up(csr, monkeypatch):
+    """The call that would build the plan gathers instead, and no later call
+    tries again."""
+    monkeypatch.setattr(hg, "VALUE_ORDER_MIN", 1)
+    monkeypatch.setattr(hg, "VALUE_ORDER_CALLS", 1)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    order = csr[0].edge_values()
+    tried = []
+
+    def build():
+        tried.append(1)
+        raise torch.OutOfMemoryError("no room")
+
+    monkeypatch.setattr(order, "_build", build)
+    assert [order.planned() for _ in range(4)] == [False] * 4
+    assert len(tried) == 1
+
+
+@pytest.mark.gpu
+def test_a_move_without_room_for_its_second_buffer_gathers(monkeypatch):
+    monkeypatch.setattr(hg, "VALUE_ORDER_MIN", 1)
+    monkeypatch.setattr(hg, "VALUE_ORDER_CALLS", 0)
+    rng = np.random.default_rng(3)
+    g = dgl.graph((rng.integers(0, 500, 40001), rng.integers(0, 500, 40001)), num_nodes=500)
+    csr = g._device_csr("in")
+    order = csr.edge_values()
+    w = torch.rand(40001, 1, device="cuda")
+    assert order.planned()
+    real, made = torch.empty_like, []
+
+    def empty_like(t):
+        made.append(1)
+        if len(made) == 2:
+            raise torch.OutOfMemoryError("no room")
+        return real(t)
+
+    monkeypatch.setattr(torch, "empty_like", empty_like)
+    got = order(w, 0)
+    monkeypatch.setattr(torch, "empty_like", real)
+    assert len(made) == 2
+    assert torch.equal(got, w[csr.eid.long()]) and torch.equal(order(w, 0), got)
+
+
+@pytest.mark.gpu
+def test_a_dot_without_room_for_the_slot_order_goes_edge_by_edge(monkeypatch):
+    from mojodgl.ops import sddmm
+
+    monkeypatch.setattr(sddmm, "DOT_SLOT_MIN_EDGES", 1)
+    rng = np.random.default_rng(4)
+    g = dgl.graph((rng.integers(0, 90, 3000), rng.integers(0, 90, 3000)), num_nodes=90)
+    x = torch.randn(90, 40, device="cuda")
+    want = ops.gsddmm(g, "dot", x, x)  # the first dot of a graph: edge by edge
+    tried = []
+
+    def slot_dot(*args):
+        tried.append(1)
+        raise torch.OutOfMemoryError("no room")
+
+    monkeypatch.setattr(sddmm, "_slot_dot", slot_dot)
+    for _ in range(3):
+        assert torch.equal(ops.gsddmm(g, "dot", x, x), want)
+    assert len(tried) == 1
