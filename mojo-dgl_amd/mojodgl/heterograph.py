@@ -57,8 +57,17 @@ CHUNK_LEN = 512
 # 1 / PULL_FULL_PASS of the edges, else a subgraph of their in-edges
 PULL_ROWS_MAX_DEGREE = 4096
 PULL_FULL_PASS = 8
-# _ValueOrder: elements from which on a plan pays, and gathers before it is built
-VALUE_ORDER_MIN = 1 << 20
+# _ValueOrder: the elements from which on a planned move is enough faster than a
+# gather, and the calls that gather before the plan is built: the smallest
+# number of moves whose savings pay for it, near enough. us for a gather, a
+# planned move and the build, float32, and the moves that pay for the build:
+#   1M   9  22     -     -       8M   137   42    880    9
+#   2M  23  26     -     -      20M   369  107  2,260    9
+#   3M  40  29   350    30     114M 2,175  895 14,400   11
+#   4M  57  31   410    15
+# (float64 alike: 20M 392, 162; 114M 2,460, 1,230). Below 4M values the gather's
+# lines stay in the caches
+VALUE_ORDER_MIN = 1 << 22
 VALUE_ORDER_CALLS = 10
 # a graph is local when at least LOCAL_FRACTION of its edges join nodes whose
 # ids differ by less than LOCAL_WINDOW (the rows whose 512-byte column slabs
@@ -188,10 +197,12 @@ class _ValueOrder:
     for a graph whose edge values are moved call after call. It holds index
     tensors only, nothing that leads back to the CSR which holds it: a graph's
     GPU memory is given back with its last reference, not with a later pass of
-    the cyclic collector. The first calls gather; once they have cost about
-    what the plan of mdgl_permute_values takes to build (two radix groupings,
-    a few passes over the indices: VALUE_ORDER_CALLS gathers), it is built
-    and used from then on. 8 bytes per element."""
+    the cyclic collector. The first VALUE_ORDER_CALLS calls gather; once the
+    time that planned moves would have saved them is about what the plan of
+    mdgl_permute_values takes to build (two radix groupings and a few passes
+    over the indices), it is built and used from then on: a graph whose calls
+    end sooner pays for no plan, one whose calls end just then has paid for one
+    without use, at most what it could have saved. 8 bytes per element."""
 
     def __init__(self, gather, inverse=None):
         self._gather, self._inverse = gather, inverse
