@@ -104,12 +104,14 @@ class _Launch:
     (operand, result and workspace addresses, the stream) filled in at each
     call. Taken only for GPU tensors that the full path would use in place
     (contiguous, on the current GPU, one float dtype) and calls whose
-    choices depend on shapes alone (no line-row copy, no CSR-order edge
-    operand). It holds the CSR it was made for and is dropped when the graph
-    holds another one (a new chunk length)."""
+    choices depend on shapes alone (no line-row copy, no edge operand put in
+    CSR order). It holds the CSR it was made for and is dropped when the graph
+    holds another one (a new chunk length). A call that would put its edge
+    operand in CSR order once that is planned counts its replays towards the
+    plan (`order`) and takes the full path when it is there."""
 
     __slots__ = ("csr", "args", "shape", "tdt", "gdev", "arg", "arg_dtype", "nbytes", "local",
-                 "dev", "sp")
+                 "dev", "sp", "order")
 
     def run(self, lhs, rhs):
         gdev = self.gdev
@@ -186,7 +188,8 @@ def _run(g, op, reduce_op, lhs_data, rhs_data, replace_inf=False, want_arg=False
     if key is not None:
         launch = g._launches.get(key)
         if launch is not None and launch.csr is g._current_csr(kind) \
-                and (launch.local is None or g._local() is launch.local):
+                and (launch.local is None or g._local() is launch.local) \
+                and (launch.order is None or not launch.order.planned()):
             # the copy ops read one operand; the other is passed as null
             return launch.run(None if op == "copy_rhs" else lhs_data,
                               None if op == "copy_lhs" else rhs_data)
@@ -269,6 +272,7 @@ def _run(g, op, reduce_op, lhs_data, rhs_data, replace_inf=False, want_arg=False
         sched = csr.chunks
         if narrow_split and packed and narrow_split < sched.chunk_len:
             sched = csr.chunks_for(narrow_split)
+        order = None
         if rhs is not None and code not in (OP_COPY_LHS, OP_COPY_RHS) and dr == 1 and num_edges \
                 and (slabs > 1 or num_edges >= CSR_ORDER_MIN_EDGES):
             # a scalar edge operand put in CSR slot order once: read by several
@@ -279,11 +283,10 @@ def _run(g, op, reduce_op, lhs_data, rhs_data, replace_inf=False, want_arg=False
             # line per edge either way: 47 columns, 20M edges, forward and
             # backward 2,283 us by edge id, 1,771 in the planned order)
             order = csr.edge_values()
-            planned = order.planned()
-            replay = False
-            if planned or slabs > 1 or not packed:
+            if order.planned() or slabs > 1 or not packed:
                 rhs = order(rhs, dcode)
                 flags |= _lib.RHS_CSR_ORDER
+                replay = False
         ws = None
         nbytes = 0
         if sched.num_chunks:
@@ -304,7 +307,7 @@ def _run(g, op, reduce_op, lhs_data, rhs_data, replace_inf=False, want_arg=False
         _lib.check(_lib.lib().mdgl_gspmm(*args), "gspmm")
         if replay:
             launch = _Launch()
-            launch.csr, launch.sp, launch.local = csr, sp, local
+            launch.csr, launch.sp, launch.local, launch.order = csr, sp, local, order
             launch.shape, launch.tdt, launch.gdev, launch.dev = shape, tdt, gdev, dev
             launch.arg, launch.arg_dtype, launch.nbytes = arg, arg_dtype, nbytes
             for i in (_A_LHS, _A_RHS, _A_OUT, _A_ARG_U, _A_ARG_E, _A_WS, _A_STREAM):

@@ -117,3 +117,28 @@ def test_a_plan_is_built_only_where_its_moves_are_faster(n, plans, monkeypatch):
     monkeypatch.setattr(order, "_build", lambda: (None,) * 3)
     assert not any(order.planned() for _ in range(hg.VALUE_ORDER_CALLS))
     assert order.planned() == plans
+
+
+@pytest.mark.gpu
+def test_scalar_weights_of_packed_rows_replay_until_the_plan(monkeypatch):
+    """Rows packed several to a wavefront read a scalar weight by edge id until
+    its order is planned: such calls replay their launch, count towards the
+    plan, and take the full path from then on, with the same bits."""
+    from mojodgl.ops import spmm
+
+    monkeypatch.setattr(hg, "VALUE_ORDER_MIN", 1)
+    monkeypatch.setattr(hg, "VALUE_ORDER_CALLS", 4)
+    monkeypatch.setattr(spmm, "CSR_ORDER_MIN_EDGES", 1)
+    rng = np.random.default_rng(5)
+    n, e = 300, 20000
+    g = dgl.graph((rng.integers(0, n, e), rng.integers(0, n, e)), num_nodes=n)
+    h, w = torch.randn(n, 24, device="cuda"), torch.rand(e, 1, device="cuda")
+    want = ops.u_mul_e_sum(g, h, w)
+    assert len(g._launches) == 1
+    order = next(iter(g._launches.values())).order
+    for _ in range(3):
+        assert torch.equal(ops.u_mul_e_sum(g, h, w), want)
+    assert order._plan is None
+    for _ in range(3):
+        assert torch.equal(ops.u_mul_e_sum(g, h, w), want)
+    assert order._plan is not None and order is g._device_csr("in").edge_values()
