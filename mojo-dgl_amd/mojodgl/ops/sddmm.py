@@ -184,7 +184,7 @@ def gsddmm(g, op, lhs_data, rhs_data, lhs_target="u", rhs_target="v"):
     lhs = _lib.on_device(L, dtype) if L is not None else None
     rhs = _lib.on_device(R, dtype) if R is not None else None
     if op == "dot" and num_edges >= DOT_SLOT_MIN_EDGES and L.shape[1:] == R.shape[1:] \
-            and dtype.itemsize * dl >= DOT_SLOT_MIN_ROW * dout \
+            and DOT_SLOT_MIN_ROW * dout <= dtype.itemsize * dl <= DOT_SLOT_MAX_ROW * dout \
             and {lhs_target, rhs_target} == {"u", "v"}:
         try:
             csr = g._dot_csr()
@@ -212,28 +212,27 @@ def gsddmm(g, op, lhs_data, rhs_data, lhs_target="u", rhs_target="v"):
 # an edge-wise dot between the endpoints runs in CSR slot order from this many
 # edges on, when a dot's rows have this many bytes or more: a destination's row
 # then stays in registers, one gathered row per edge less, for the results'
-# move into edge-id order (128 columns, 20M edges: 3,187 us edge by edge,
-# 1,484 slot by slot and for that move 363, later 107 (_ValueOrder); 2,658 us with the destinations' rows read again from
-# cache for every slot)
+# move into edge-id order (128 columns, 20M edges: 3,187 us edge by edge, 1,484
+# slot by slot and 107 for the planned move, 370 until that is planned
+# (_ValueOrder); 2,658 us with the destinations' rows read again from cache for
+# every slot). The most is what 64 lanes of 16 bytes hold: wider rows go edge by
+# edge, which is decided before the in-CSR would be built for them
 DOT_SLOT_MIN_EDGES = 1 << 20
 DOT_SLOT_MIN_ROW = 128
+DOT_SLOT_MAX_ROW = 1024
 
 
 def _slot_dot(csr, x, y, num_edges, num_nodes, d, dout, fshape, dtype):
     """The dot of every edge between its source's row of `x` and its
     destination's of `y` (mdgl_gspmm_row_dot: the same sums, and so the same
-    bits, as edge by edge) in edge-id order, or None for rows that kernel does
-    not take."""
+    bits, as edge by edge) in edge-id order."""
     lib, code, st = _lib.lib(), _lib.dtype_code(dtype), _lib.stream()
     tdt, gdev, sched = _lib.torch_dtype(dtype), _lib.device(), csr.chunks
     tmp = torch.empty((num_edges, dout), dtype=tdt, device=gdev)
-    rc = lib.mdgl_gspmm_row_dot(csr.indptr.data_ptr(), csr.indices.data_ptr(), x.data_ptr(),
-                                y.data_ptr(), tmp.data_ptr(), num_nodes, d, dout,
-                                _lib.ptr(sched.chunk_row), _lib.ptr(sched.chunk_start),
-                                sched.num_chunks, sched.chunk_len, _lib.ANY_ALIGNMENT, code, st)
-    if rc == _lib.ENOTSUP:
-        return None
-    _lib.check(rc, "gspmm_row_dot")
+    _lib.check(lib.mdgl_gspmm_row_dot(
+        csr.indptr.data_ptr(), csr.indices.data_ptr(), x.data_ptr(), y.data_ptr(), tmp.data_ptr(),
+        num_nodes, d, dout, _lib.ptr(sched.chunk_row), _lib.ptr(sched.chunk_start),
+        sched.num_chunks, sched.chunk_len, _lib.ANY_ALIGNMENT, code, st), "gspmm_row_dot")
     if dout == 1:
         order = csr.slot_values()
         order.planned()

@@ -142,3 +142,22 @@ def test_scalar_weights_of_packed_rows_replay_until_the_plan(monkeypatch):
     for _ in range(3):
         assert torch.equal(ops.u_mul_e_sum(g, h, w), want)
     assert order._plan is not None and order is g._device_csr("in").edge_values()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,d,slots", [(torch.float32, 256, True), (torch.float32, 257, False),
+                                           (torch.float64, 128, True), (torch.float64, 129, False)])
+def test_dots_too_wide_for_the_slot_kernel_build_no_csr(dtype, d, slots, monkeypatch):
+    """64 lanes of 16 bytes hold a destination's row; a wider dot goes edge by
+    edge and asks for neither the in-CSR nor a second buffer."""
+    from mojodgl.ops import sddmm
+
+    monkeypatch.setattr(sddmm, "DOT_SLOT_MIN_EDGES", 1)
+    rng = np.random.default_rng(d)
+    u, v = rng.integers(0, 50, 700), rng.integers(0, 50, 700)
+    g = dgl.graph((u, v), num_nodes=50)
+    x, y = (torch.randint(-8, 9, (50, d), device="cuda").to(dtype) for _ in range(2))
+    for _ in range(3):  # whole numbers: exact in any order
+        got = ops.u_dot_v(g, x, y)
+        assert torch.equal(got, (x[u] * y[v]).sum(-1, keepdim=True))
+    assert (g._current_csr("in") is not None) == slots
