@@ -83,6 +83,7 @@ struct GspmmArgs {
   int32_t* part_u;
   int32_t* part_e;
   int64_t chunk_waves, row_waves, chunk_blocks, num_blocks;
+  int64_t first_block;  // of this launch (launch_gspmm_op)
   // waves per slab (with several, every unit's slab s comes before slab s + 1,
   // so the rows of neighbouring units share cache lines across wavefronts)
   int64_t chunk_uwaves, row_uwaves;
@@ -480,7 +481,7 @@ constexpr int gspmm_waves(int op, int red, int path, int lay, int vec, int size)
 template <class T, int OP, int RED, int VEC, int PATH, int LAY>
 __global__ __launch_bounds__(BLOCK, gspmm_waves(OP, RED, PATH, LAY, VEC, sizeof(T))) void
 gspmm_kernel(GspmmArgs<T> a) {
-  const int64_t b = blockIdx.x;
+  const int64_t b = a.first_block + blockIdx.x;
   const bool chunk = b < a.chunk_blocks;
   const int64_t blk =
       chunk ? xcd_remap(b, a.chunk_blocks) : xcd_remap(b - a.chunk_blocks, a.num_blocks - a.chunk_blocks);
@@ -635,33 +636,28 @@ hipError_t launch_gspmm_op(const GspmmParams& p) {
   a.dot_lanes = p.dot_lanes;
   a.rows = p.rows;
   a.row_limit = p.row_limit;
-  if (a.num_blocks > 0) {
-    const bool copy_l = OP == OP_COPY_LHS, copy_r = OP == OP_COPY_RHS;
-    const int lm = copy_r ? a.rmode : a.lmode;
-    const int rm = copy_l ? a.lmode : (!copy_r && a.rmode == M_SPLAT && a.dr == 1 ? M_SCALAR : a.rmode);
-    const dim3 grid((unsigned)a.num_blocks), block(BLOCK);
+  const bool copy_l = OP == OP_COPY_LHS, copy_r = OP == OP_COPY_RHS;
+  const int lm = copy_r ? a.rmode : a.lmode;
+  const int rm = copy_l ? a.lmode : (!copy_r && a.rmode == M_SPLAT && a.dr == 1 ? M_SCALAR : a.rmode);
+  const dim3 block(BLOCK);
+  // HIP refuses a launch of 2**32 or more work-items, which 16 lanes a row
+  // reach at 2**28 rows and 64 at 2**26: longer work lists take several
+  // (of whole rounds over the XCDs, so the remap holds)
+  for (a.first_block = 0; a.first_block < a.num_blocks; a.first_block += MAX_LAUNCH_BLOCKS) {
+    const int64_t left = a.num_blocks - a.first_block;
+    const dim3 grid((unsigned)(left < MAX_LAUNCH_BLOCKS ? left : MAX_LAUNCH_BLOCKS));
     bool launched = false;
-    if constexpr (OP == OP_MUL && RED == RED_SUM && VEC == VecOf<T>::n) {
+    if constexpr ((OP == OP_MUL || OP == OP_COPY_LHS) && RED == RED_SUM && VEC == VecOf<T>::n) {
       if (p.dot_out) {
         // the caller checked: contiguous lhs rows, rhs splat over the groups
+        constexpr int PATH = OP == OP_MUL ? P_CS_DOT : P_DOT;
         if (G == WAVE)
-          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CS_DOT, LAY_WIDE>), grid, block, 0,
+          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, PATH, LAY_WIDE>), grid, block, 0,
                              p.stream, a);
         else
-          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CS_DOT, LAY_ROW>), grid, block, 0,
+          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, PATH, LAY_ROW>), grid, block, 0,
                              p.stream, a);
         launched = true;
-      }
-    }
-    if constexpr (OP == OP_COPY_LHS && RED == RED_SUM && VEC == VecOf<T>::n) {
-      if (p.dot_out) {
-        if (G == WAVE)
-          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_DOT, LAY_WIDE>), grid, block, 0,
-                             p.stream, a);
-        else
-          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_DOT, LAY_ROW>), grid, block, 0,
-                             p.stream, a);
-        return hipGetLastError();  // no partials to fold
       }
     }
     if (!launched) {
@@ -673,6 +669,7 @@ hipError_t launch_gspmm_op(const GspmmParams& p) {
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
   }
+  if (OP == OP_COPY_LHS && p.dot_out) return hipSuccess;  // no partials to fold
   if (p.num_heavy > 0) {
     const int64_t n = p.num_heavy * p.dout;
     hipLaunchKernelGGL((gspmm_combine_kernel<T, RED>), dim3((unsigned)((n + BLOCK - 1) / BLOCK)),

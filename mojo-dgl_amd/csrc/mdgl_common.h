@@ -31,6 +31,9 @@ enum Mode { M_CONTIG = 0, M_SPLAT = 1, M_GATHER = 2 };
 constexpr int WAVE = 64;
 constexpr int BLOCK = 256;
 constexpr int WAVES_PER_BLOCK = BLOCK / WAVE;
+// Workgroups of BLOCK that one launch takes (fewer than 2**32 work-items), in
+// whole rounds over the XCDs.
+constexpr int64_t MAX_LAUNCH_BLOCKS = ((int64_t(1) << 32) - 1) / BLOCK / 8 * 8;
 constexpr int MAX_DIMS = 6;
 
 // NumPy broadcasting of two operands against an output feature shape,

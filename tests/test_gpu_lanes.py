@@ -194,3 +194,27 @@ def test_edge_dot_in_slot_order(dtype, shape, swap, monkeypatch):
     second = dot(g, x, y)
     assert g._current_csr("in") is not None and g._current_csr("in")._slot_of_eid is not None
     assert first.shape == second.shape and torch.equal(first, second)
+
+
+@pytest.mark.gpu
+def test_rows_past_one_launch():
+    """16 lanes a row are 2**32 work-items at 2**28 rows, more than HIP launches
+    at once: the rows beyond are reduced too (every 2**20th row and the last
+    two hold one edge, the others none)."""
+    n = (1 << 28) + 4097
+    filled = torch.cat([torch.arange(0, n, 1 << 20, device="cuda"),
+                        torch.tensor([n - 2, n - 1], device="cuda")])
+    E = filled.numel()
+    indptr = torch.zeros(n + 1, dtype=torch.int32, device="cuda")
+    indptr[filled + 1] = 1
+    indptr = torch.cumsum(indptr, 0, dtype=torch.int32)
+    index = torch.arange(E, dtype=torch.int32, device="cuda")
+    x = torch.arange(1, E + 1, dtype=torch.float32, device="cuda")
+    out = torch.full((n,), -1.0, device="cuda")
+    _lib.check(_lib.lib().mdgl_gspmm(
+        indptr.data_ptr(), index.data_ptr(), index.data_ptr(), x.data_ptr(), None, out.data_ptr(),
+        n, _lib.OP_COPY_LHS, 1, 1, 1, 0, None, 0, None, None, None, None, None, None, 0, 0, None,
+        None, 0, None, 0, _lib.ANY_ALIGNMENT, 0, _lib.stream()), "gspmm")
+    want = torch.zeros(n, device="cuda")
+    want[filled] = x
+    assert torch.equal(out, want)
