@@ -45,7 +45,7 @@ template <class T, int VEC>
 __device__ __forceinline__ void fetch_rt(const T* __restrict__ row, int mode, int off,
                                          T (&x)[VEC]) {
   if (mode == M_CONTIG) {
-    load_any<T, VEC>(row + off, x, false);
+    load_any<false, T, VEC>(row + off, x);
   } else {
     const T s = row[off];
 #pragma unroll

@@ -95,16 +95,31 @@ struct GspmmArgs {
   int64_t row_limit;
 };
 
+// Edge rows of consecutive columns from this many bytes on are read past the
+// caches: each is read once, and so does not displace source rows that other
+// edges will gather. Narrower ones share their lines with other edges' rows,
+// which the caches may still hold when those are read. Time of streamed reads
+// over cached ones, float32 sums by edge id, copy_e and u_mul_e, each warm and
+// after the caches were overwritten:
+//   bytes        1M edges                6M edges                60M edges
+//     16   1.33 1.14  1.31 1.13    1.31 1.29  1.26 1.16    1.05 1.23  1.01 1.01
+//     64   1.29 0.92  1.28 0.90    1.23 0.96  1.03 0.92    0.99 1.03  0.90 0.90
+//     96   1.23 0.90  1.06 0.90    1.12 0.94  0.96 0.91    0.97 1.01  0.87 0.87
+//    128   1.25 0.65  1.21 0.76    0.96 0.81  0.97 0.89    0.96 0.98  0.85 0.86
+//    256   1.19 0.55  0.94 0.67    0.96 0.87  0.99 0.92      -
+// (100,000 edges: 1.0 warm at any width, after an overwrite 1.09 at 16 bytes, 0.98
+// at 96, 0.74 at 256.)
+constexpr int64_t STREAM_ROW_BYTES = 96;
+
 // The VEC columns a lane reads from an operand row (off: their offsets; only
-// off[0] unless the mode is gather). Edge rows are read once per edge and
-// stream past the caches, so they do not displace source rows that other
-// edges will gather.
-template <class T, int VEC, int M, bool STREAM>
+// off[0] unless the mode is gather), past the caches with STREAM; rows of
+// consecutive columns not with NEAR.
+template <class T, int VEC, int M, bool STREAM, bool NEAR>
 __device__ __forceinline__ void fetch(const T* __restrict__ row, int mode_rt, const int (&off)[VEC],
                                       T (&x)[VEC]) {
   const int m = (M == M_DYN) ? mode_rt : M;
   if (m == M_CONTIG) {
-    load_any<T, VEC>(row + off[0], x, STREAM);
+    load_any<STREAM && !NEAR, T, VEC>(row + off[0], x);
   } else if (m == M_SPLAT) {
     const T s = STREAM ? __builtin_nontemporal_load(row + off[0]) : row[off[0]];
 #pragma unroll
@@ -154,8 +169,9 @@ __device__ __forceinline__ void for_each(F f) {
 enum { LAY_ROW = 0, LAY_WIDE = 1 };
 
 // DOT: 1 beside the sum, 2 alone (nothing folded or written but the dots).
+// NEAR: edge rows are read through the caches.
 template <class T, int OP, int RED, int VEC, int LM, int RM, int LAY, int DOT = 0,
-          bool SEL = false>
+          bool SEL = false, bool NEAR = false>
 __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, int64_t wave,
                                            int lane) {
   // edges in flight per lane: 8 (4 in the dot pass, whose per-edge
@@ -230,7 +246,7 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
   if constexpr (DOT) {
 #pragma unroll
     for (int v = 0; v < VEC; ++v) rowv[v] = T(0);
-    if (ok) load_any<T, VEC>(a.rowop + row * a.dout + k0, rowv, false);
+    if (ok) load_any<false, T, VEC>(a.rowop + row * a.dout + k0, rowv);
   }
 
   T acc[VEC];
@@ -276,15 +292,14 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
       constexpr int u = decltype(iu)::value;
       if constexpr (HAS_L) {
         const int64_t lo = lo_of(iu);
-        fetch<T, VEC, LM, false>(reinterpret_cast<const T*>(lbase + lo), a.lmode, loff, x[u]);
+        fetch<T, VEC, LM, false, false>(reinterpret_cast<const T*>(lbase + lo), a.lmode, loff, x[u]);
         if constexpr (SEL)
-          load_any<int32_t, VEC>(
-              reinterpret_cast<const int32_t*>(sbase + lo / (int64_t)(sizeof(T) / 4)), sel[u],
-              false);
+          load_any<false, int32_t, VEC>(
+              reinterpret_cast<const int32_t*>(sbase + lo / (int64_t)(sizeof(T) / 4)), sel[u]);
       }
       if constexpr (ROW_R)
-        fetch<T, VEC, RM, true>(reinterpret_cast<const T*>(rbase + ro_of(iu)), a.rmode, roff,
-                                y[u]);
+        fetch<T, VEC, RM, true, NEAR>(reinterpret_cast<const T*>(rbase + ro_of(iu)), a.rmode, roff,
+                                      y[u]);
     };
     auto fold = [&](auto iu) MDGL_INLINE {
       constexpr int u = decltype(iu)::value;
@@ -462,8 +477,10 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
 // P_DOT (copy / sum) writes only the dots of every gathered row with the row's
 // own. P_SEL (copy / sum) adds a gathered value only where the selection's entry is
 // the edge itself: the gradient of a max or min without a tensor of per-edge
-// gradients in between.
-enum { P_CC = 0, P_CS = 1, P_DYN = 2, P_CS_DOT = 3, P_CW = 4, P_SEL = 5, P_DOT = 6 };
+// gradients in between. The _NEAR ones read edge rows through the caches (see
+// STREAM_ROW_BYTES).
+enum { P_CC = 0, P_CS = 1, P_DYN = 2, P_CS_DOT = 3, P_CW = 4, P_SEL = 5, P_DOT = 6, P_CC_NEAR = 7,
+       P_DYN_NEAR = 8 };
 
 // Wavefronts per SIMD asked of the register allocation: what each path needs
 // plus a few registers would otherwise round down to one wavefront less (98
@@ -472,9 +489,10 @@ enum { P_CC = 0, P_CS = 1, P_DYN = 2, P_CS_DOT = 3, P_CW = 4, P_SEL = 5, P_DOT =
 // Sums only: the other reducers' selected slots and a divide's temporaries
 // would spill.
 constexpr int gspmm_waves(int op, int red, int path, int lay, int vec, int size) {
-  if (red != RED_SUM || op == OP_DIV || path == P_DYN || vec * size > 16) return 1;
+  if (red != RED_SUM || op == OP_DIV || path == P_DYN || path == P_DYN_NEAR || vec * size > 16)
+    return 1;
   if (path == P_SEL) return size == 8 ? 4 : 5;
-  if (path == P_CC && op != OP_COPY_LHS && op != OP_COPY_RHS) return lay == LAY_WIDE ? 6 : 5;
+  if ((path == P_CC || path == P_CC_NEAR) && op != OP_COPY_LHS && op != OP_COPY_RHS) return lay == LAY_WIDE ? 6 : 5;
   return size == 8 ? 6 : 7;
 }
 
@@ -492,6 +510,8 @@ gspmm_kernel(GspmmArgs<T> a) {
   if (wave >= (chunk ? a.chunk_waves : a.row_waves)) return;
   if constexpr (PATH == P_CC)
     gspmm_body<T, OP, RED, VEC, M_CONTIG, M_CONTIG, LAY>(a, chunk, wave, lane);
+  else if constexpr (PATH == P_CC_NEAR)
+    gspmm_body<T, OP, RED, VEC, M_CONTIG, M_CONTIG, LAY, 0, false, true>(a, chunk, wave, lane);
   else if constexpr (PATH == P_CS)
     gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SPLAT, LAY>(a, chunk, wave, lane);
   else if constexpr (PATH == P_CW)
@@ -502,6 +522,8 @@ gspmm_kernel(GspmmArgs<T> a) {
     gspmm_body<T, OP, RED, VEC, M_CONTIG, M_CONTIG, LAY, 2>(a, chunk, wave, lane);
   else if constexpr (PATH == P_CS_DOT)
     gspmm_body<T, OP, RED, VEC, M_CONTIG, M_SPLAT, LAY, 1>(a, chunk, wave, lane);
+  else if constexpr (PATH == P_DYN_NEAR)
+    gspmm_body<T, OP, RED, VEC, M_DYN, M_DYN, LAY, 0, false, true>(a, chunk, wave, lane);
   else
     gspmm_body<T, OP, RED, VEC, M_DYN, M_DYN, LAY>(a, chunk, wave, lane);
 }
@@ -575,16 +597,30 @@ void launch_path(const GspmmArgs<T>& a, dim3 grid, dim3 block, int lm, int rm, h
       return;
     }
   }
-  if constexpr (OP == OP_COPY_LHS || OP == OP_COPY_RHS)
-    hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CC, LAY>), grid, block, 0, st, a);
-  else if (lm == M_CONTIG && rm == M_CONTIG)
-    hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CC, LAY>), grid, block, 0, st, a);
-  else if (lm == M_CONTIG && rm == M_SCALAR)
-    hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CW, LAY>), grid, block, 0, st, a);
-  else if (lm == M_CONTIG && rm == M_SPLAT)
-    hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_CS, LAY>), grid, block, 0, st, a);
-  else
-    hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, P_DYN, LAY>), grid, block, 0, st, a);
+  const bool near = a.dr * (int64_t)sizeof(T) < STREAM_ROW_BYTES;
+  auto go = [&](auto path) {
+    hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, decltype(path)::value, LAY>), grid, block, 0,
+                       st, a);
+  };
+#define MDGL_PATH(P) go(std::integral_constant<int, P>{})
+  if constexpr (OP == OP_COPY_LHS) {
+    MDGL_PATH(P_CC);
+  } else if constexpr (OP == OP_COPY_RHS) {
+    if (near) MDGL_PATH(P_CC_NEAR);
+    else MDGL_PATH(P_CC);
+  } else if (lm == M_CONTIG && rm == M_CONTIG) {
+    if (near) MDGL_PATH(P_CC_NEAR);
+    else MDGL_PATH(P_CC);
+  } else if (lm == M_CONTIG && rm == M_SCALAR) {
+    MDGL_PATH(P_CW);
+  } else if (lm == M_CONTIG && rm == M_SPLAT) {
+    MDGL_PATH(P_CS);
+  } else if (near) {
+    MDGL_PATH(P_DYN_NEAR);
+  } else {
+    MDGL_PATH(P_DYN);
+  }
+#undef MDGL_PATH
 }
 
 template <class T, int OP, int RED, int VEC>

@@ -157,15 +157,21 @@ __device__ __forceinline__ void load_n_stream(const T* p, T (&out)[N]) {
   for (int i = 0; i < N; ++i) out[i] = v[i];
 }
 
-// N consecutive elements at element alignment (one 4- to 32-byte access).
-template <class T, int N>
-__device__ __forceinline__ void load_any(const T* p, T (&out)[N], bool stream) {
+// N consecutive elements at element alignment (one 4- to 32-byte access). With
+// STREAM, a template parameter, past the caches: two loads of one address that a
+// run-time flag chooses between are merged into one without the hint (edge rows of
+// 64 columns by id, 100,000 of them, cold caches, us: float32 17.6 and 13.0
+// streamed, float64 26.6 and 17.1).
+template <bool STREAM, class T, int N>
+__device__ __forceinline__ void load_any(const T* p, T (&out)[N]) {
   if constexpr (N == 1) {
-    out[0] = stream ? __builtin_nontemporal_load(p) : *p;
+    if constexpr (STREAM) out[0] = __builtin_nontemporal_load(p);
+    else out[0] = *p;
   } else {
     typedef T V __attribute__((ext_vector_type(N), aligned(sizeof(T))));
-    const V v = stream ? __builtin_nontemporal_load(reinterpret_cast<const V*>(p))
-                       : *reinterpret_cast<const V*>(p);
+    V v;
+    if constexpr (STREAM) v = __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
+    else v = *reinterpret_cast<const V*>(p);
 #pragma unroll
     for (int i = 0; i < N; ++i) out[i] = v[i];
   }

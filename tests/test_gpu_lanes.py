@@ -14,7 +14,7 @@ import torch
 import mojodgl as dgl
 import mojodgl.ops as ops
 import oracle
-from mojodgl import _lib
+from mojodgl import _lib, heterograph
 
 # 1 to 64 lanes of 4, 2 or 1 columns, remainders on both sides, 2 to 5 slabs
 WIDTHS = [1, 2, 3, 4, 5, 7, 9, 15, 16, 17, 31, 33, 47, 63, 66, 97, 127, 130, 255, 257, 258, 515]
@@ -218,3 +218,28 @@ def test_rows_past_one_launch():
     want = torch.zeros(n, device="cuda")
     want[filled] = x
     assert torch.equal(out, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,widths", [(np.float32, (23, 24, 25)), (np.float64, (11, 12, 13))])
+def test_edge_rows_either_side_of_streaming(dtype, widths, monkeypatch):
+    """Edge rows of 96 bytes or more are read past the caches: the same bits on
+    both sides, with the node operand consecutive, one value per row, and
+    absent."""
+    monkeypatch.setattr(heterograph, "CHUNK_LEN", 1 << 20)  # no row split
+    u, v, n = ragged_graph(widths[0])
+    g = dgl.graph((u, v), num_nodes=n)
+    rng = np.random.default_rng(6)
+    for d in widths:
+        w = rng.normal(size=(u.size, d)).astype(dtype)
+        wt = torch.from_numpy(w).cuda()
+        for red in ("sum", "max"):
+            want = oracle.gspmm(u, v, n, "copy_rhs", red, None, w, dtype)
+            got = ops.gspmm(g, "copy_rhs", red, None, wt)
+            np.testing.assert_array_equal(got.cpu().numpy(), want)
+            for dl in (d, 1):
+                h = rng.normal(size=(n, dl)).astype(dtype)
+                got = ops.gspmm(g, "mul", red, torch.from_numpy(h).cuda(), wt)
+                want = oracle.gspmm(u, v, n, "mul", red, np.broadcast_to(h, (n, d)).copy(), w,
+                                    dtype)
+                np.testing.assert_array_equal(got.cpu().numpy(), want)
