@@ -64,6 +64,12 @@ extern "C" {
  * before it), so odd widths and heads load and store whole vectors. Results
  * are the same bit for bit; only the lane layout changes. */
 #define MDGL_ANY_ALIGNMENT 64
+/* mdgl_gspmm, _selected_sum, _mul_sum_dot_any: a row of fewer than 16 lanes takes
+ * the power of two covering them, at least 2 (4), instead of 16 -- for graphs of
+ * few edges a row (about 6, 12 on average). Results are the same bit for bit; only
+ * the lane layout changes. At most one of the two. */
+#define MDGL_ROW_LANES_2 128
+#define MDGL_ROW_LANES_4 256
 /* mdgl_segment_reduce(_arg): the caller knows that no segment has more than
  * MDGL_SEGMENT_SPLIT_ROWS rows, so the pass that splits longer segments is
  * not launched (a longer segment is then still reduced whole, in row order) */

@@ -592,8 +592,9 @@ int64_t gspmm_row_lanes(const GspmmParams& p, int64_t dout) {
   return p.run_len > 0 ? dout / p.run_len * p.lpg : 0;
 }
 
-// Lanes per row slab: the power of two covering the row's lanes, at least 16
-// (gspmm_impl.h says why) and at most 64. With MDGL_NARROW_SLABS, rows wider than 64 vectors take 32-lane slabs
+// Lanes per row slab: the power of two covering the row's lanes, at least 16, or
+// 2 or 4 where the caller says so (gspmm_impl.h says why), and at most 64. With
+// MDGL_NARROW_SLABS, rows wider than 64 vectors take 32-lane slabs
 // (two rows per wavefront) when that makes at most GSPMM_NARROW_MAX_SLABS of
 // them: each slab walks all of a row's edges again, and on a graph whose
 // sources lie near their destinations the 512-byte slabs of a block of
@@ -606,7 +607,7 @@ int gspmm_group(int64_t nvec, int flags, bool dot) {
   if ((flags & MDGL_NARROW_SLABS) && !dot && nvec > WAVE &&
       (nvec + WAVE / 2 - 1) / (WAVE / 2) <= GSPMM_NARROW_MAX_SLABS)
     gmax = WAVE / 2;
-  int g = 16;
+  int g = flags & MDGL_ROW_LANES_2 ? 2 : flags & MDGL_ROW_LANES_4 ? 4 : 16;
   while (g < nvec && g < gmax) g <<= 1;
   return g;
 }
@@ -815,7 +816,8 @@ int mdgl_gspmm_selected_sum(const int32_t* indptr, const int32_t* indices, const
   MDGL_RANGE();
   if (num_dst > 0 && d > 0 && (!sel || !eid))
     return fail(MDGL_EINVAL, "gspmm_selected_sum: null selection or eid");
-  if (flags & ~MDGL_ANY_ALIGNMENT) return fail(MDGL_EINVAL, "gspmm_selected_sum: bad flags");
+  if (flags & ~(MDGL_ANY_ALIGNMENT | MDGL_ROW_LANES_2 | MDGL_ROW_LANES_4))
+    return fail(MDGL_EINVAL, "gspmm_selected_sum: bad flags");
   return gspmm_common(indptr, indices, eid, lhs, nullptr, dst, num_dst, OP_COPY_LHS, d, d, d,
                       RED_SUM, nullptr, 0, nullptr, nullptr, nullptr, nullptr, chunk_row,
                       chunk_start, num_chunks, chunk_len, heavy_rows, heavy_ptr, num_heavy,

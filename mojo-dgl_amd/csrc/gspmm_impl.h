@@ -9,7 +9,8 @@
 // neighbouring destinations share its L2 (a community graph's chunks dealt
 // round-robin over the XCDs held its L2 hit rate at 70 %). A unit is processed
 // by G consecutive lanes (G = the power of two covering the row's lanes, at
-// least 16 and at most 64), so a wavefront packs 64 / G units; output rows wider than
+// most 64 and at least 16, or 2 or 4 for rows of few edges), so a wavefront packs
+// 64 / G units; output rows wider than
 // 64 lanes are cut into S slabs, one wavefront per slab.
 //
 // Lane columns. A row is made of dout / L runs of L columns over which each
@@ -39,12 +40,18 @@
 //               broadcast by DPP (row_newbcast, one VALU operation per word;
 //               ds_bpermute with a 64-bit multiply per lane and edge took 45
 //               instructions per two edges).
-// Rows of fewer than 16 lanes take 16 all the same, the lanes past the row
-// repeating its last columns: with only the lanes they need, 1 to 8, a row had
-// as few edges in flight as lanes (one id per lane), and a wavefront of 8 to
-// 64 rows waited for the longest of them (4 columns on 4.9M edges of a
-// power-law graph: 1,121 us that way, 398 with 8 ids per lane instead, 192 at
-// 16 lanes; 16 columns on 89M edges, forward and backward: 7.7, 7.1, 6.6 ms).
+//   G < 16      every lane loads the ids of its own row, U at a time (one load
+//               each, the same address across a unit).
+// The caller says which of the last two a row of fewer than 16 lanes takes, by
+// the edges its rows have on average. With many, 16 lanes, those past the row
+// repeating its last columns: a wavefront of 8 to 64 rows waits for the longest
+// of them (4 columns on 4.9M edges of a power-law graph, 16 a row: 1,121 us with
+// an edge in flight per lane of a packed row, 398 with 8, 192 at 16 lanes). With
+// few, the lanes it needs, at least 2 or 4: most rows end within the first U
+// edges, and 16 lanes would be 4 rows a wavefront where 16 or 32 fit (one column,
+// 2 edges a row, 4M rows: 311 us for copy_u, 113 with 2 lanes, 118 with one lane
+// and one edge in flight; 4 random edges a row: 362 and 223; MDGL_ROW_LANES_2 and
+// _4, whose caller has the line and both sides).
 // Ids past a row repeat its last one, so id loads need no branch; operand rows
 // are requested and folded without one except in the batch that ends a row.
 #pragma once
@@ -166,7 +173,7 @@ __device__ __forceinline__ void for_each(F f) {
 }
 
 // How ids reach the lanes of a unit (see the top): by G.
-enum { LAY_ROW = 0, LAY_WIDE = 1 };
+enum { LAY_ROW = 0, LAY_WIDE = 1, LAY_LANE = 2 };
 
 // DOT: 1 beside the sum, 2 alone (nothing folded or written but the dots).
 // NEAR: edge rows are read through the caches.
@@ -386,6 +393,35 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
         else
           batch(std::false_type{}, start + base + F, rem, lo_of, ro_of, w_of, e_of);
       });
+    }
+  } else if constexpr (LAY == LAY_LANE) {
+    // ---- every lane loads its own row's ids, those of a batch at a time
+    for (int base = 0; base < n; base += U) {
+      int32_t s[U], e[U];
+      T w[U];
+      const int rem = n - base;
+      for_each<U>([&](auto iu) MDGL_INLINE {
+        constexpr int u = decltype(iu)::value;
+        s[u] = e[u] = 0;
+        w[u] = T(0);
+        if (u < rem) {
+          const int i = start + base + u;
+          if constexpr (HAS_L) s[u] = a.indices[i];
+          if constexpr (HAS_R || SEL) {
+            e[u] = i;
+            if (need_e) e[u] = a.eid[i];
+          }
+        }
+      });
+      if constexpr (SCALAR)
+        for_each<U>([&](auto iu) MDGL_INLINE {
+          if (decltype(iu)::value < rem) w[decltype(iu)::value] = a.rhs[e[decltype(iu)::value]];
+        });
+      auto lo_of = [&](auto iu) MDGL_INLINE { return (int64_t)s[decltype(iu)::value] * lbytes; };
+      auto ro_of = [&](auto iu) MDGL_INLINE { return (int64_t)e[decltype(iu)::value] * rbytes; };
+      auto w_of = [&](auto iu) MDGL_INLINE { return w[decltype(iu)::value]; };
+      auto e_of = [&](auto iu) MDGL_INLINE { return e[decltype(iu)::value]; };
+      batch(std::false_type{}, start + base, rem, lo_of, ro_of, w_of, e_of);
     }
   } else {
     // ---- 64 ids per load, broadcast by v_readlane (n is uniform here)
@@ -623,6 +659,13 @@ void launch_path(const GspmmArgs<T>& a, dim3 grid, dim3 block, int lm, int rm, h
 #undef MDGL_PATH
 }
 
+// (lanes of 32 bytes are for rows of more than 64 of 16)
+template <class T, int OP, int RED, int VEC>
+void launch_lane(const GspmmArgs<T>& a, dim3 grid, dim3 block, int lm, int rm, hipStream_t st) {
+  if constexpr (VEC <= VecOf<T>::n)
+    launch_path<T, OP, RED, VEC, LAY_LANE>(a, grid, block, lm, rm, st);
+}
+
 template <class T, int OP, int RED, int VEC>
 hipError_t launch_gspmm_op(const GspmmParams& p) {
   GspmmArgs<T> a;
@@ -690,6 +733,9 @@ hipError_t launch_gspmm_op(const GspmmParams& p) {
         if (G == WAVE)
           hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, PATH, LAY_WIDE>), grid, block, 0,
                              p.stream, a);
+        else if (G < 16)
+          hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, PATH, LAY_LANE>), grid, block, 0,
+                             p.stream, a);
         else
           hipLaunchKernelGGL((gspmm_kernel<T, OP, RED, VEC, PATH, LAY_ROW>), grid, block, 0,
                              p.stream, a);
@@ -699,6 +745,8 @@ hipError_t launch_gspmm_op(const GspmmParams& p) {
     if (!launched) {
       if (G == WAVE)
         launch_path<T, OP, RED, VEC, LAY_WIDE>(a, grid, block, lm, rm, p.stream);
+      else if (G < 16)
+        launch_lane<T, OP, RED, VEC>(a, grid, block, lm, rm, p.stream);
       else
         launch_path<T, OP, RED, VEC, LAY_ROW>(a, grid, block, lm, rm, p.stream);
     }

@@ -55,6 +55,8 @@ RHS_CSR_ORDER = 2
 LHS_LINE_ROWS = 8  # mdgl_gspmm: lhs rows copied to start on 128-byte lines
 NARROW_SLABS = 32  # mdgl_gspmm: 32-lane column slabs for wide rows (a local graph)
 ANY_ALIGNMENT = 64  # mdgl_gspmm: 16-byte lanes for odd widths, heads and addresses too
+ROW_LANES_2 = 128  # mdgl_gspmm: rows of few lanes take at least 2 instead of 16
+ROW_LANES_4 = 256  # and at least 4
 COO_INGEST_BLOCKS = 512  # pairs written by mdgl_coo_ingest
 PERMUTE_TILE = 16384  # mdgl_permute_values: elements per tile and region of its plan
 COO_LOCALITY_BLOCKS = 1024  # counts written by mdgl_coo_locality

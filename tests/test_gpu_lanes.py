@@ -243,3 +243,62 @@ def test_edge_rows_either_side_of_streaming(dtype, widths, monkeypatch):
                 want = oracle.gspmm(u, v, n, "mul", red, np.broadcast_to(h, (n, d)).copy(), w,
                                     dtype)
                 np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("d", [1, 2, 3, 5, 8, 9, 16, 17, 31, 33])
+@pytest.mark.parametrize("lanes", [_lib.ROW_LANES_2, _lib.ROW_LANES_4])
+def test_rows_of_few_lanes(dtype, d, lanes, monkeypatch):
+    """Rows that take only the lanes they need, each lane loading its row's ids:
+    the oracle's bits for whole rows of 0 to 40 edges and a hub, and the same
+    bits as 16 lanes a row for split rows and the backward passes' kernels."""
+    u, v, n = ragged_graph(d)
+    rng = np.random.default_rng(d + 7)
+    x = rng.normal(size=(n, d)).astype(dtype)
+    w = (rng.random((u.size, 1)) + 0.5).astype(dtype)
+    e = rng.normal(size=(u.size, d)).astype(dtype)
+    operands = (("copy_lhs", x, None), ("copy_rhs", None, e), ("mul", x, w), ("add", x, e),
+                ("div", x[:, :1].copy(), e))
+
+    def gpu(a):
+        return None if a is None else torch.from_numpy(a).cuda()
+
+    with monkeypatch.context() as m:
+        m.setattr(ops.spmm, "_row_lanes", lambda num_edges, num_rows: lanes)
+        m.setattr(heterograph, "CHUNK_LEN", 1 << 20)
+        g = dgl.graph((u, v), num_nodes=n)
+        for op, a, b in operands:
+            wide = None if a is None else np.ascontiguousarray(np.broadcast_to(a, (n, d)))
+            for red in ("sum", "mean", "max", "min"):
+                got, (au, ae) = ops.spmm._gspmm(g, op, red, gpu(a), gpu(b))
+                what = "{} {}".format(op, red)
+                if red in ("max", "min"):
+                    want, ru, re_ = oracle.gspmm(u, v, n, op, red, wide, b, dtype, with_arg=True)
+                    if op != "copy_rhs":
+                        np.testing.assert_array_equal(au.cpu().numpy(), ru, err_msg=what)
+                    if op != "copy_lhs":
+                        np.testing.assert_array_equal(ae.cpu().numpy(), re_, err_msg=what)
+                else:
+                    want = oracle.gspmm(u, v, n, op, red, wide, b, dtype)
+                np.testing.assert_array_equal(got.cpu().numpy(), want, err_msg=what)
+
+    def backward(fewest):
+        with monkeypatch.context() as m:
+            m.setattr(ops.spmm, "_row_lanes", lambda num_edges, num_rows: fewest)
+            g = dgl.graph((u, v), num_nodes=n)
+            out = []
+            for op, a, b in operands:
+                leaves = [gpu(t).requires_grad_(True) for t in (a, b) if t is not None]
+                for red in ("sum", "max"):
+                    z = ops.gspmm(g, op, red, *((None,) if a is None else ()), *leaves,
+                                  *((None,) if b is None else ()))
+                    G = torch.cos(torch.arange(z.numel(), device="cuda").reshape(z.shape)).to(z)
+                    out += [z.detach(), *torch.autograd.grad(z, leaves, G)]
+                if op in ("copy_lhs", "add"):  # the node operand alone
+                    z = ops.gspmm(g, op, "max", leaves[0], None if b is None else gpu(b))
+                    out += torch.autograd.grad(z, leaves[:1], G)
+            return out
+
+    for got, want in zip(backward(lanes), backward(0)):
+        assert torch.equal(got, want)
