@@ -1574,7 +1574,9 @@ template <class T, int MB, int NBK, bool GATHER>
 __global__ __launch_bounds__(BLOCK, MB * NBK * (int)sizeof(T) > 64 ? 2 : 3) void grouped_tn_kernel(TnArgs<T> p) {
   using M = Mfma<T>;
   using acc_t = typename M::acc_t;
-  constexpr int U = 2;  // groups of four rows per step
+  // groups of four rows per step: one where the registers of doubles would not
+  // hold three steps of two
+  constexpr int U = sizeof(T) == 8 && (GATHER || MB * NBK >= 16) ? 1 : 2;
   __shared__ acc_t red[2][MB * NBK][WAVE];
 
   const int64_t c = blockIdx.x;

@@ -77,3 +77,13 @@ def test_edge_rows_stream_past_the_caches(kernels, pattern):
             rows = re.findall(r"global_load_dwordx4 .*", _asm(kernel))
             hinted = sum(bool(re.search(r"\bnt\b", r)) for r in rows)
             assert (hinted >= 8) if hints else (rows and hinted == 0), name
+
+
+def test_gradient_of_b_keeps_its_registers(kernels):
+    """No instance of the gradient of b spills: three steps of a 64 x 64 tile of
+    doubles did, two groups of four rows each."""
+    for name, (mangled, path) in _named(kernels, r"grouped_tn_(tile_)?kernel<").items():
+        notes = _run(LLVM + "/llvm-readelf", "--notes", path)
+        entry = next(e for e in notes.split("- .agpr_count")
+                     if re.search(r"\.name: +" + re.escape(mangled) + r"\s", e))
+        assert re.search(r"\.private_segment_fixed_size: 0\b", entry), name
