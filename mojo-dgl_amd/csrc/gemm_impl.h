@@ -1810,10 +1810,26 @@ hipError_t launch_grouped_grad(const GemmGradLaunch& L, bool gather) {
         got = sizes[k];
     return got;
   };
-  static constexpr int MS4[] = {8, 7, 6, 5, 4, 3, 2}, NS4[] = {4, 3, 2, 1};
+  static constexpr int MS4[] = {8, 7, 6, 5, 4, 3, 2};
   static constexpr int MS8[] = {4, 2}, NS8[] = {4, 2, 1};
   int mb = sizeof(T) == 4 ? best(b1, MS4, 7) : best(b1, MS8, 2);
-  const int nb = sizeof(T) == 4 ? best(b2, NS4, 4) : best(b2, NS8, 3);
+  // float32 along D2: up to four blocks as they are, of more the tile that costs
+  // least: its blocks, those of idle wavefronts counted, times about 12 + 9 q^2 us
+  // over 2.5M rows for the loads per MFMA q (measured 15 for 8 x 4 and 8 x 3, 16.5
+  // for 3 x 3, 21 for 3 x 2, 20 for 7 x 1). 80 x 80 over 10M rows in tiles of 5 x 1
+  // 3,165 us, of 5 x 3 1,840; 100 x 100 4,333 in 7 x 1 and 2,984 in 7 x 4
+  auto spread = [&](int nb) {  // blocks, those of idle wavefronts counted
+    const int64_t tiles = (b1 + mb - 1) / mb * ((b2 + nb - 1) / nb), tw = tiles > 2 ? 4 : tiles;
+    return (tiles + tw - 1) / tw * tw * mb * nb;
+  };
+  auto cost = [&](int nb) {
+    const double q = (double)(mb + nb) / (mb * nb);
+    return (double)spread(nb) * (12 + 9 * q * q);
+  };
+  int nb = sizeof(T) == 8 ? best(b2, NS8, 3) : b2 <= 4 ? (int)b2 : 4;
+  if (sizeof(T) == 4 && b2 > 4)
+    for (int k = 3; k >= 1; --k)
+      if (cost(k) < cost(nb)) nb = k;
   a.tiles_n = (int)((b2 + nb - 1) / nb);
   auto cut = [&] {
     a.tiles = (int)((b1 + mb - 1) / mb) * a.tiles_n;

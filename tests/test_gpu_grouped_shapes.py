@@ -81,6 +81,68 @@ def test_products_and_gradients(dtype, k, n):
         within(db, ref, bound, int(seg.max()), dtype)
 
 
+def gradient_of_b(a, G, group, r):
+    """a^T G per group in float64, and the sum of the products' magnitudes."""
+    ref = torch.zeros(r, a.shape[1], G.shape[1], dtype=torch.float64, device="cuda")
+    bound = torch.zeros_like(ref)
+    for i in range(r):
+        rows = (group == i).nonzero().view(-1)
+        x, y = a[rows].double(), G[rows].double()
+        ref[i] = x.t().contiguous() @ y
+        bound[i] = x.abs().t().contiguous() @ y.abs()
+    return ref, bound
+
+
+# float32 gradients of b: widths that fill tiles of 128 x 128 (whole, cut, several,
+# just under), register tiles of every width along the second axis, both at and
+# off a 16-byte boundary
+@pytest.mark.parametrize("k,n", [(128, 128), (120, 124), (128, 112), (112, 124), (108, 128),
+                                 (256, 128), (124, 256), (252, 244), (512, 120), (100, 100),
+                                 (80, 80), (64, 80), (144, 144), (160, 160), (200, 200), (72, 176)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_gradient_tiles(k, n, shift):
+    seg, grp = groups(k + n)
+    rng = np.random.default_rng(k * n)
+    a, b, G = inputs(k, n, torch.float32, k * n, seg)
+
+    def off(x):  # a copy that starts `shift` elements into its buffer
+        buf = torch.empty(x.numel() + shift, device="cuda")
+        view = buf[shift:].view(x.shape)
+        return view.copy_(x)
+
+    a, G = off(a), off(G)
+    b.requires_grad_(True)
+    for by in ("segment", "gather"):
+        group = torch.from_numpy(grp if by == "segment" else grp[rng.permutation(grp.size)]).cuda()
+        z = ops.segment_mm(a, b, seg) if by == "segment" else ops.gather_mm(a, b, idx_b=group)
+        db, = torch.autograd.grad(z, (b,), G)
+        ref, bound = gradient_of_b(a, G, group, len(seg))
+        within(db, ref, bound, int(seg.max()), torch.float32)
+
+
+@pytest.mark.parametrize("dtype,k,n,r", [(torch.float32, 12, 20, 3), (torch.float32, 128, 128, 5),
+                                         (torch.float32, 40, 72, 200), (torch.float64, 32, 64, 3),
+                                         (torch.float64, 48, 33, 7)])
+@pytest.mark.parametrize("by", ["segment", "gather"])
+def test_gradient_over_longer_chunks(dtype, k, n, r, by):
+    """More than 524,288 rows: a workgroup sums 512 rows or more."""
+    rows = 600011
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    a = torch.randn(rows, k, device="cuda", generator=gen, dtype=dtype)
+    G = torch.randn(rows, n, device="cuda", generator=gen, dtype=dtype)
+    b = torch.randn(r, k, n, device="cuda", generator=gen, dtype=dtype).requires_grad_(True)
+    group = torch.randint(0, r, (rows,), device="cuda", generator=gen)
+    if by == "segment":
+        group = group.sort()[0]
+        z = ops.segment_mm(a, b, torch.bincount(group, minlength=r).cpu())
+    else:
+        z = ops.gather_mm(a, b, idx_b=group)
+    db, = torch.autograd.grad(z, (b,), G)
+    ref, bound = gradient_of_b(a, G, group, r)
+    # a chunk's chain, the streams, then the group's chunks
+    within(db, ref, bound, 4096 + rows // 512, dtype)
+
+
 @pytest.mark.parametrize("k,n", [(4, 5), (7, 17), (18, 33), (47, 64), (100, 47), (61, 20),
                                  (130, 40), (255, 100)])
 def test_inf_and_nan_stay_in_their_rows(k, n):
