@@ -1710,6 +1710,162 @@ __global__ __launch_bounds__(BLOCK, MB * NBK * (int)sizeof(T) > 64 ? 2 : 3) void
   }
 }
 
+// The same partials for float32 widths that fill 128 x 128 tiles
+// (launch_grouped_grad has the line). The register tiles above take two wavefronts
+// of 8 x 4 blocks for 128 columns and read every row of a twice, 4 bytes a lane;
+// here the four wavefronts (2 x 2, each 64 x 64 of the tile as 4 x 4 blocks) share
+// one read of 16 bytes a lane. Rows are walked BK at a time through row-major LDS
+// tiles, double buffered; lane l feeds a[row k0 + l / 16][m0 + l % 16] as A^T and
+// grad[row k0 + l / 16][n0 + l % 16] as B; a row stride of 144 elements puts the
+// four rows one 64-lane read touches in distinct banks. Alternate groups of four
+// rows go to two accumulators, so that a chain of additions is as long as in the
+// register tiles, whose wavefronts share a chunk's rows.
+//
+// Bound by the float32 MFMAs and, gathered, by the rows' latency. us, register tiles
+// and these, in segments and gathered, over 64 groups:
+//   128 x 128, 300,000 rows   183   161    226   217
+//   128 x 128, 2.5M rows      951   878  1,045 1,043
+//   128 x 128, 10M rows     3,462 2,995  3,643 3,357
+//   256 x 128, 2.5M rows    1,833 1,546  1,979 1,735
+//   256 x 256, 2.5M rows    3,998 3,086  3,873 3,335
+// Gathered rows 16 at a time, with three workgroups per CU instead of two: 1,020
+// over 2.5M rows, 3,990 over 10M (two registers spilled).
+template <bool GATHER>
+__global__ __launch_bounds__(BLOCK, 2) void grouped_tn_tile_kernel(TnArgs<float> p) {
+  constexpr int BK = Mfma<float>::BK;
+  using M = Mfma<float>;
+  using acc_t = typename M::acc_t;
+  constexpr int LD = GBM + 16;
+  constexpr int EV = 4;            // elements per 16-byte load
+  constexpr int CPR = GBM / EV;    // 16-byte pieces per 128-wide tile row
+  constexpr int RPP = BLOCK / CPR; // tile rows per pass of the block
+  constexpr int PASSES = BK / RPP;
+  __shared__ __align__(16) float As[2][BK][LD];
+  __shared__ __align__(16) float Bs[2][BK][LD];
+
+  const int64_t c = blockIdx.x;
+  if (c >= p.chunk_ptr[p.R]) return;  // uniform per workgroup
+  int64_t lo = 0, hi = p.R - 1;       // last group whose first chunk is <= c
+  while (lo < hi) {
+    const int64_t mid = (lo + hi + 1) / 2;
+    if (p.chunk_ptr[mid] <= c) lo = mid; else hi = mid - 1;
+  }
+  // (32-bit positions and widths, for fewer registers: there are fewer than 2**31
+  // rows of fewer than 2**31 elements)
+  const int grp = (int)lo;
+  const int r0 = p.group_off[grp] + (int)((c - p.chunk_ptr[grp]) * p.ch);
+  const int g_end = p.group_off[grp + 1];
+  const int rows = g_end - r0 < p.ch ? g_end - r0 : (int)p.ch;  // at least one
+  const int D1 = (int)p.D1, D2 = (int)p.D2;
+  const int m0 = (int)(blockIdx.y / p.tiles_n) * GBM;
+  const int n0 = (int)(blockIdx.y % p.tiles_n) * GBN;
+  const int t = threadIdx.x;
+  const int lane = t & 63, w = t >> 6, wm = w >> 1, wn = w & 1;
+  const int li = lane & 15, h = lane >> 4;
+  const int tr = t / CPR, col = (t % CPR) * EV;
+  // Each lane's 16-byte pieces of a stage: rows past the chunk and pieces past the
+  // width (multiples of EV) load row 0 / column 0 and are zeroed when the stage is
+  // written to LDS, at its end (a test right after a load would wait for it there).
+  const bool in_a = m0 + col < D1, in_b = n0 + col < D2;
+  const int ca = in_a ? m0 + col : 0, cb = in_b ? n0 + col : 0;
+
+  // gather_mm's rows of a stage come through the permutation: they are requested
+  // one stage ahead (an unconditional load of a clamped index; the row test is
+  // applied where they are used), so no stage waits for them
+  int32_t rid[PASSES];
+  auto stage_rows = [&](int k0) {
+#pragma unroll
+    for (int q = 0; q < PASSES; ++q) {
+      const int k = k0 + q * RPP + tr;
+      if constexpr (GATHER) rid[q] = p.perm[r0 + (k < rows ? k : rows - 1)];
+    }
+  };
+  float ra[PASSES][EV], rb[PASSES][EV];
+  auto load_stage = [&](int k0) {
+#pragma unroll
+    for (int q = 0; q < PASSES; ++q) {
+      const int k = k0 + q * RPP + tr;
+      const int row = GATHER ? rid[q] : r0 + (k < rows ? k : rows - 1);
+      load_vec<float>(p.a + (int64_t)row * D1 + ca, ra[q]);
+      load_vec<float>(p.g + (int64_t)row * D2 + cb, rb[q]);
+    }
+  };
+  auto store_stage = [&](int buf, int k0) {
+#pragma unroll
+    for (int q = 0; q < PASSES; ++q) {
+      const int r = q * RPP + tr;
+      const bool ok = k0 + r < rows;
+      float xa[EV], xb[EV];
+#pragma unroll
+      for (int v = 0; v < EV; ++v) {
+        xa[v] = ok && in_a ? ra[q][v] : 0.f;
+        xb[v] = ok && in_b ? rb[q][v] : 0.f;
+      }
+      store_vec<float>(&As[buf][r][col], xa);
+      store_vec<float>(&Bs[buf][r][col], xb);
+    }
+  };
+
+  acc_t acc[2][4][4];  // of alternate groups of four rows
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[k][i][j][r] = 0.f;
+
+  stage_rows(0);
+  load_stage(0);
+  stage_rows(BK);  // the next stage's rows
+  store_stage(0, 0);
+  __syncthreads();
+  for (int k0 = 0, buf = 0; k0 < rows; k0 += BK, buf ^= 1) {
+    const bool more = k0 + BK < rows;
+    if (more) load_stage(k0 + BK);
+    stage_rows(k0 + 2 * BK);
+    __builtin_amdgcn_s_setprio(1);  // MFMA issue first (as in the forward kernel)
+#pragma unroll
+    for (int k8 = 0; k8 < BK; k8 += 8) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int kk = k8 + 4 * k + h;
+        float af[4], bf[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          af[i] = As[buf][kk][wm * 64 + i * 16 + li];
+          bf[i] = Bs[buf][kk][wn * 64 + i * 16 + li];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[k][i][j] = M::step(af[i], bf[j], acc[k][i][j]);
+      }
+    }
+    __builtin_amdgcn_s_setprio(0);
+    if (more) {
+      store_stage(buf ^ 1, k0 + BK);
+      __syncthreads();
+    }
+  }
+
+  float* const out = p.part + c * p.D1 * p.D2;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int d1 = m0 + wm * 64 + i * 16 + M::row(h, r);
+      if (d1 >= D1) continue;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int d2 = n0 + wn * 64 + j * 16 + li;
+        if (d2 < D2) out[(int64_t)d1 * D2 + d2] = acc[0][i][j][r] + acc[1][i][j][r];
+      }
+    }
+  }
+}
+
 // db[g][e] = sum of part[c][e] over g's chunks in order (0 for an empty group),
 // eight partials requested at a time.
 template <class T>
@@ -1836,18 +1992,38 @@ hipError_t launch_grouped_grad(const GemmGradLaunch& L, bool gather) {
     a.tw = a.tiles > 2 ? 4 : a.tiles;
     return max_chunks * ((a.tiles + a.tw - 1) / a.tw);
   };
+  const int64_t wgs = cut();
+  bool tiled = false;
+  if constexpr (sizeof(T) == 4) {
+    // the 128 x 128 tiles through LDS where at least 7/8 of them are columns (us over
+    // 2.5M rows, register tiles and LDS: 120 x 120 945 and 872, 112 x 112 856 and 868,
+    // 96 x 128 774 and 866, 192 x 192 2,125 and 2,886; gathered 1,058 and 1,066, 964
+    // and 1,041, 873 and 1,021, 2,225 and 3,266, over 10M rows 120 x 120 3,741 and
+    // 3,436)
+    const int64_t lds = ((L.D1 + GBM - 1) / GBM) * ((L.D2 + GBN - 1) / GBN);
+    tiled = L.D1 % 4 == 0 && L.D2 % 4 == 0 && aligned16(L.a) && aligned16(L.grad) &&
+            8 * L.D1 * L.D2 >= 7 * lds * GBM * GBN;
+    if (tiled) {
+      a.tiles_n = (int)((L.D2 + GBN - 1) / GBN);
+      const dim3 grid((unsigned)max_chunks, (unsigned)lds);
+      if (perm)
+        hipLaunchKernelGGL((grouped_tn_tile_kernel<true>), grid, dim3(BLOCK), 0, L.stream, a);
+      else
+        hipLaunchKernelGGL((grouped_tn_tile_kernel<false>), grid, dim3(BLOCK), 0, L.stream, a);
+    }
+  }
   // several tiles and fewer workgroups than two per CU: tiles of 2, 4 or 8
   // blocks, which are more of them (208 x 130 over 32K rows of 105 groups, us:
   // 7-block tiles 63, 2-block ones 55; 152 x 246 over 771K rows the other way
   // round, 3,305 with 2-block tiles for the step and 2,890 with 5-block ones)
   static constexpr int MS4_FEW[] = {8, 4, 2};
-  if (cut() < 512 && sizeof(T) == 4 && b1 > 8) {
+  if (!tiled && wgs < 512 && sizeof(T) == 4 && b1 > 8) {
     mb = best(b1, MS4_FEW, 3);
     cut();
   }
   const dim3 grid((unsigned)max_chunks, (unsigned)((a.tiles + a.tw - 1) / a.tw));
 #define MDGL_TN_CASE(M, N)                                                                    \
-  if (mb == M && nb == N) {                                                                   \
+  if (!tiled && mb == M && nb == N) {                                                         \
     if (perm)                                                                                 \
       hipLaunchKernelGGL((grouped_tn_kernel<T, M, N, true>), grid, dim3(BLOCK), 0, L.stream, a); \
     else                                                                                      \
