@@ -352,11 +352,12 @@ __device__ __forceinline__ int64_t k_of(int64_t kv, int64_t K) {
 
 // Wavefronts per SIMD that the registers of an instance allow.
 constexpr int any_waves(int nb, int km) {
-  return nb == 4 || nb * km > 256 ? 2 : (nb == 2 || km == 256 ? 3 : 5);
+  return nb == 4 || nb * km > 256 ? 2 : (nb == 2 || km == 256 ? 3 : 4);
 }
 
-// Chunks in flight: with one narrow column block two, for a fifth wavefront
-// per SIMD (four chunks would spill there).
+// Chunks in flight: with one narrow column block two, for a fourth wavefront per
+// SIMD (for a fifth three to five registers went to memory: 16 x 16 over 10M rows
+// 303 us, with four wavefronts 300).
 constexpr int any_depth(int nb, int km) { return nb == 1 && km < 256 ? 2 : 4; }
 
 // bt3[g][q][n][k] (bf16 bit patterns): part q of b[g][k_of(k)][n] (of

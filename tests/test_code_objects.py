@@ -79,10 +79,11 @@ def test_edge_rows_stream_past_the_caches(kernels, pattern):
             assert (hinted >= 8) if hints else (rows and hinted == 0), name
 
 
-def test_gradient_of_b_keeps_its_registers(kernels):
-    """No instance of the gradient of b spills: three steps of a 64 x 64 tile of
-    doubles did, two groups of four rows each."""
-    for name, (mangled, path) in _named(kernels, r"grouped_tn_(tile_)?kernel<").items():
+@pytest.mark.parametrize("pattern", [r"grouped_tn_(tile_)?kernel<", r"grouped_gemm_any_kernel<"])
+def test_grouped_products_keep_their_registers(kernels, pattern):
+    """No instance spills: three steps of a 64 x 64 tile of doubles did, two
+    groups of four rows each, and one column block at five wavefronts per SIMD."""
+    for name, (mangled, path) in _named(kernels, pattern).items():
         notes = _run(LLVM + "/llvm-readelf", "--notes", path)
         entry = next(e for e in notes.split("- .agpr_count")
                      if re.search(r"\.name: +" + re.escape(mangled) + r"\s", e))
