@@ -629,7 +629,12 @@ __global__ __launch_bounds__(SB_THREADS, 1) void grouped_gemm_split_kernel(
 // The products of the split kernel (three bf16 parts per operand, the same six
 // part products, the same float32 fallback) for the shapes it does not take: K
 // of 4 to 256 at any alignment, and 64 columns or fewer, where its four column
-// blocks of 32 would multiply zeros.
+// blocks of 32 would multiply zeros. The three part products left out are at most
+// 2^-24 of |a b| together, 2^-27 on average; sixteen products are added with one
+// rounding where float32 MFMAs, which these shapes took before, round every two.
+// Relative error against 64 bits, float32 MFMAs, these six and all nine, 1e-8:
+// 16 x 16 7.39 3.35 3.30, 47 x 100 12.4 9.24 9.23, 100 x 47 18.0 14.8 14.8, 250 x 250
+// 28.4 23.9 23.9; the three would cost 1% (16 x 16) to 13% (130 x 200) of the time.
 //
 // What bounds it is memory: a row is read and written once, and 100 x 47
 // products of 2.5M rows take 85 us of MFMA against 0.3 ms of traffic. The

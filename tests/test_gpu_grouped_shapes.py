@@ -81,6 +81,36 @@ def test_products_and_gradients(dtype, k, n):
         within(db, ref, bound, int(seg.max()), dtype)
 
 
+@pytest.mark.parametrize("by", ["segment", "gather"])
+@pytest.mark.parametrize("k,n", [(16, 16), (17, 32), (20, 250), (33, 129), (47, 100), (64, 64),
+                                 (100, 47), (100, 20), (128, 33), (130, 200), (199, 61), (250, 250),
+                                 (256, 32)])
+def test_split_products_are_no_further_off_than_float32_ones(k, n, by):
+    """The part products left out cost less than the roundings saved: the result
+    is no further from 64 bits than that of float32 MFMAs, which a value of b out
+    of the split's range (times a zero of a, so that the sums are the same) sends
+    the same call to."""
+    rows, r = 40000, 5
+    gen = torch.Generator(device="cuda").manual_seed(k * n)
+    a = torch.randn(rows, k, device="cuda", generator=gen)
+    a[:, 0] = 0
+    b = torch.randn(r, k, n, device="cuda", generator=gen)
+    group = torch.randint(0, r, (rows,), device="cuda", generator=gen).sort()[0]
+    seg = torch.bincount(group, minlength=r).cpu()
+    ref = torch.empty(rows, n, device="cuda", dtype=torch.float64)
+    for i in range(r):
+        at = (group == i).nonzero().view(-1)
+        ref[at] = a[at].double() @ b[i].double()
+
+    def off(b):
+        z = ops.segment_mm(a, b, seg) if by == "segment" else ops.gather_mm(a, b, idx_b=group)
+        return float((z.double() - ref).norm() / ref.norm())
+
+    plain = b.clone()
+    plain[:, 0] = 1e30
+    assert 0 < off(b) <= off(plain)
+
+
 def gradient_of_b(a, G, group, r):
     """a^T G per group in float64, and the sum of the products' magnitudes."""
     ref = torch.zeros(r, a.shape[1], G.shape[1], dtype=torch.float64, device="cuda")
