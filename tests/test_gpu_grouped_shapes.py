@@ -81,6 +81,48 @@ def test_products_and_gradients(dtype, k, n):
         within(db, ref, bound, int(seg.max()), dtype)
 
 
+# Every instance of the forward kernels with more tiles than workgroups: column
+# blocks by LDS depth by the number of 16-deep chunks of a row, which leaves every
+# remainder in the ring of chunks in flight; float64 in two, four and eight blocks.
+MANY = ([(torch.float32, k, n) for k, n in (
+    (12, 20), (20, 30), (40, 17), (60, 32), (70, 9), (90, 31), (100, 20), (120, 5), (140, 24),
+    (250, 16), (10, 47), (30, 64), (44, 33), (64, 50), (72, 40), (92, 64), (100, 47), (127, 60),
+    (130, 40), (160, 70), (250, 100), (9, 100), (25, 66), (47, 100), (63, 128), (66, 100),
+    (85, 129), (103, 70), (121, 90))]
+    + [(torch.float64, k, n) for k, n in ((16, 32), (48, 20), (128, 17), (32, 64), (112, 40),
+                                          (64, 100))])
+
+
+@pytest.mark.parametrize("dtype,k,n", MANY)
+def test_several_tiles_per_workgroup(dtype, k, n):
+    """2,600 groups of 0 to 260 rows: a workgroup goes from tile to tile within a
+    group and over group ends (its block of b kept, or loaded again), in segments
+    and gathered, forward and both gradients."""
+    rng = np.random.default_rng(k * n)
+    seg = rng.choice([0, 1, 5, 31, 32, 33, 127, 128, 129, 260], 2600)
+    ids = np.repeat(np.arange(seg.size), seg)
+    a, b, G = inputs(k, n, dtype, k + n, seg)
+    a.requires_grad_(True)
+    b.requires_grad_(True)
+    for by in ("segment", "gather"):
+        group = torch.from_numpy(ids if by == "segment" else rng.permutation(ids)).cuda()
+        z = ops.segment_mm(a, b, seg) if by == "segment" else ops.gather_mm(a, b, idx_b=group)
+        da, db = torch.autograd.grad(z, (a, b), G)
+        B = b.detach().double()
+        bt = B.transpose(1, 2).contiguous()
+        ref, bound = torch.zeros_like(B), torch.zeros_like(B)
+        step = max(1, (1 << 25) // (k * n))
+        for lo in range(0, group.numel(), step):
+            at = slice(lo, lo + step)
+            g, x, y = group[at], a.detach()[at].double(), G[at].double()
+            within(z.detach()[at], product(x, B, g), product(x.abs(), B.abs(), g), k, dtype)
+            within(da[at], product(y, bt, g), product(y.abs(), bt.abs(), g), n, dtype)
+            pairs = x.unsqueeze(2) * y.unsqueeze(1)
+            ref.index_add_(0, g, pairs)
+            bound.index_add_(0, g, pairs.abs())
+        within(db, ref, bound, int(seg.max()), dtype)
+
+
 @pytest.mark.parametrize("by", ["segment", "gather"])
 @pytest.mark.parametrize("k,n", [(16, 16), (17, 32), (20, 250), (33, 129), (47, 100), (64, 64),
                                  (100, 47), (100, 20), (128, 33), (130, 200), (199, 61), (250, 250),
