@@ -8,7 +8,7 @@ these follow the calculus of the forward ops and run on the same kernels:
     max(deg v, 1) for mean: ``mdgl_rows_by_degree`` on G first); for mul
     with an edge operand constant over x's last axis (attention weights),
     dX and dY come from one pass over the out-CSR
-    (``mdgl_gspmm_mul_sum_dot``: G[v] gathered once per edge, dY in CSR slot
+    (``mdgl_gspmm_mul_sum_dot_any``: G[v] gathered once per edge, dY in CSR slot
     order, then gathered to edge order);
     dX[u] = sum over u's out-edges of that gradient times d msg / dX, a
     gspmm over the out-CSR (copy for copy_lhs / add / sub, mul / div by Y for
@@ -201,7 +201,7 @@ class GSpMM(torch.autograd.Function):
                 # operand is constant over trailing groups of x (attention)
                 from .spmm import _mul_sum_dot
 
-                fused = _mul_sum_dot(g, G, y, x, min_run=1) if _trailing_groups(x, y) else None
+                fused = _mul_sum_dot(g, G, y, x) if _trailing_groups(x, y) else None
                 if fused is not None:
                     return None, None, None, _back(fused[0], x0), _back(fused[1], y0), None
             if need_x:

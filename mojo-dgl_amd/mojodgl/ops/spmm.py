@@ -373,15 +373,14 @@ def _run_rows(csr, rows, code, reduce_op, lhs, rhs, out, arg_u, arg_e, dl, dr, d
     return out, arg_u, arg_e, as_torch, dev
 
 
-def _mul_sum_dot(g, grad, y, x, kind="out", min_run=7):
+def _mul_sum_dot(g, grad, y, x, kind="out"):
     """Both gradients of a u_mul_e_sum whose edge operand `y` is constant
     over trailing groups of the node operand `x`, in one pass over the `kind`
-    CSR (mdgl_gspmm_mul_sum_dot): returns (dx, dy) as GPU tensors shaped like
-    x and y, or None when the shapes do not fit the fused kernel (the caller
-    then runs gspmm and gsddmm). `min_run`: other runs (columns per value of
-    `y`) than 2 and 4 of fewer columns are left to those too; the backward
-    passes take every run the kernel does (on 6M edges, 4 heads of 5, 9 or 12
-    columns: 448, 461, 470 us against 1,078, 1,971, 775 us separately)."""
+    CSR (mdgl_gspmm_mul_sum_dot_any): returns (dx, dy) as GPU tensors shaped like
+    x and y, or None when the shapes do not fit the fused kernel: runs (columns
+    per value of `y`) under 16 bytes or over 64 lanes of them (the caller then
+    runs gspmm and gsddmm; on 6M edges, 4 heads of 5, 9 or 12 columns: 448, 461,
+    470 us against 1,078, 1,971, 775 separately)."""
     G = grad.contiguous()
     X = x.contiguous()
     # y as (E, *x's leading feature axes, 1): the same rank as the node rows
@@ -399,8 +398,6 @@ def _mul_sum_dot(g, grad, y, x, kind="out", min_run=7):
         return None
     if E == 0:  # no messages: both gradients are zero
         return torch.zeros_like(x), torch.zeros_like(y)
-    if dout // dr < min_run and dout // dr not in (2, 4):
-        return None
     csr = g._device_csr(kind)
     sched = csr.chunks
     gdev = _lib.device()

@@ -114,7 +114,7 @@ def test_gspmm_backward(op, red, yshape):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("xshape,yshape", [((8, 32), (8, 1)), ((4, 16), (4, 1)), ((64,), (1,)),
                                            ((2, 6), (2, 1)), ((3, 128), (3, 1))],
-                         ids=["wide-8heads", "packed-4heads", "one-group", "unfusable-6",
+                         ids=["wide-8heads", "packed-4heads", "one-group", "cut-lanes-6",
                               "slabs-3x128"])
 @pytest.mark.parametrize("red", ["sum", "mean"])
 def test_gspmm_mul_backward_fused_pass(dtype, xshape, yshape, red):
@@ -122,7 +122,7 @@ def test_gspmm_mul_backward_fused_pass(dtype, xshape, yshape, red):
     both gradients come from one pass over the out-CSR (hubs split into
     chunks included). dX equals the separate gspmm bit for bit, dY the
     separate per-head dot to rounding; both against torch autograd in float64
-    (shapes the fused kernel does not take fall back to the separate ops)."""
+    (6 columns a run: lanes that end with the run)."""
     from mojodgl.ops import spmm
 
     n, e = 300, 5000
@@ -154,13 +154,12 @@ def test_gspmm_mul_backward_fused_pass(dtype, xshape, yshape, red):
         G = torch.randn(out.shape, generator=torch.Generator(device=DEV).manual_seed(63),
                         device=DEV, dtype=torch.float64).to(dtype)
         fused = spmm._mul_sum_dot(g, G, y.detach(), x.detach())
-        if xshape[-1] == 6:
-            assert fused is None  # 6 columns per group: not a power-of-two lane count
-        else:
-            dx, dy = fused
-            sep = ops.spmm._run(g, "mul", "sum", G, y.detach(), kind="out")[0]
-            assert torch.equal(dx, sep.reshape(dx.shape))
-            within(dy, ry, by)
+        # runs of at least one 16-byte lane, 6 columns among them (two lanes in
+        # float32, the second sharing columns with the first)
+        dx, dy = fused
+        sep = ops.spmm._run(g, "mul", "sum", G, y.detach(), kind="out")[0]
+        assert torch.equal(dx, sep.reshape(dx.shape))
+        within(dy, ry, by)
 
 
 def test_gspmm_gradcheck():
