@@ -113,6 +113,64 @@ static void gspmm_arguments() {
                             nullptr) == MDGL_EWORKSPACE);
 }
 
+static void newer_entry_points() {
+  int32_t ids[8] = {0};
+  int64_t wide[8] = {0};
+  uint16_t pick[8] = {0};
+  alignas(256) float x[64] = {0};
+  // endpoints and planned permutations
+  EXPECT(mdgl_coo_ingest(wide, wide, ids, ids, -1, wide, nullptr) == MDGL_EINVAL);
+  EXPECT(mdgl_coo_ingest(wide, wide, ids, ids, 5, nullptr, nullptr) == MDGL_EINVAL);
+  EXPECT(mdgl_coo_ingest(nullptr, wide, ids, ids, 5, wide, nullptr) == MDGL_EINVAL);
+  EXPECT(mdgl_permute_values(x, pick, ids, pick, x, x, 5, 4, nullptr) == MDGL_EINVAL);
+  EXPECT(mdgl_permute_values(x, pick, ids, pick, x, x, -1, MDGL_FLOAT32, nullptr) == MDGL_EINVAL);
+  EXPECT(mdgl_permute_values(x, pick, nullptr, pick, x, x, 5, MDGL_FLOAT32, nullptr) ==
+         MDGL_EINVAL);
+  // lane layouts of every width, flag and type: whole lanes that cover the row
+  for (int64_t d = 1; d <= 700; d += d < 80 ? 1 : 37) {
+    for (int flags : {0, MDGL_ANY_ALIGNMENT, MDGL_ANY_ALIGNMENT | MDGL_NARROW_SLABS,
+                      MDGL_ANY_ALIGNMENT | MDGL_ROW_LANES_2, MDGL_ANY_ALIGNMENT | MDGL_ROW_LANES_4,
+                      MDGL_ANY_ALIGNMENT | MDGL_LHS_LINE_ROWS}) {
+      for (int dt = 0; dt < 2; ++dt) {
+        int64_t vec = 0, group = 0, lanes = 0;
+        EXPECT(mdgl_gspmm_layout(5, d, d, d, 0, nullptr, nullptr, x, x, flags, dt, &vec, &group,
+                                 &lanes) == MDGL_OK);
+        EXPECT(vec >= 1 && vec * lanes >= d && (lanes - 1) * vec < d);
+        EXPECT(group >= 2 && group <= 64 && (group & (group - 1)) == 0);
+        const int64_t ls[2] = {3, d}, rs[2] = {3, 1};
+        EXPECT(mdgl_gspmm_layout(2, 3 * d, 3, 3 * d, 2, ls, rs, x, x,
+                                 flags & ~MDGL_LHS_LINE_ROWS, dt, &vec, &group,
+                                 &lanes) == MDGL_OK);
+        EXPECT(vec >= 1 && vec * lanes >= 3 * d);
+      }
+    }
+  }
+  // row dots, selected sums and the fused dot
+  EXPECT(mdgl_gspmm_row_dot(ids, ids, x, x, nullptr, 5, 8, 1, nullptr, nullptr, 0, 0,
+                            MDGL_ANY_ALIGNMENT, MDGL_FLOAT32, nullptr) == MDGL_EINVAL);
+  EXPECT(mdgl_gspmm_row_dot(ids, ids, x, x, x, 5, 8, 1, nullptr, nullptr, 0, 0, 0, MDGL_FLOAT32,
+                            nullptr) == MDGL_EINVAL);
+  for (int64_t d : {1, 3, 257, 1000})
+    EXPECT(mdgl_gspmm_row_dot(ids, ids, x, x, x, 5, d, 1, nullptr, nullptr, 0, 0,
+                              MDGL_ANY_ALIGNMENT, MDGL_FLOAT32, nullptr) == MDGL_ENOTSUP);
+  EXPECT(mdgl_gspmm_selected_sum(ids, ids, ids, x, nullptr, x, 5, 4, nullptr, nullptr, 0, 0,
+                                 nullptr, nullptr, 0, nullptr, 0, MDGL_ANY_ALIGNMENT, MDGL_FLOAT32,
+                                 nullptr) == MDGL_EINVAL);
+  EXPECT(mdgl_gspmm_selected_sum(ids, ids, ids, x, ids, x, 5, 4, ids, ids, 3, 4, ids, ids, 1,
+                                 nullptr, 0, MDGL_ANY_ALIGNMENT, MDGL_FLOAT32,
+                                 nullptr) == MDGL_EWORKSPACE);
+  EXPECT(mdgl_gspmm_selected_sum(ids, ids, ids, x, ids, x, 5, 4, nullptr, nullptr, 0, 0, nullptr,
+                                 nullptr, 0, nullptr, 0, MDGL_REPLACE_INF, MDGL_FLOAT32,
+                                 nullptr) == MDGL_EINVAL);
+  const int64_t ls[2] = {4, 3}, rs[2] = {4, 1};
+  EXPECT(mdgl_gspmm_mul_sum_dot_any(ids, ids, ids, x, x, x, x, nullptr, 5, 12, 4, 12, 2, ls, rs,
+                                    nullptr, nullptr, 0, 0, nullptr, nullptr, 0, nullptr, 0,
+                                    MDGL_ANY_ALIGNMENT, MDGL_FLOAT64, nullptr) == MDGL_EINVAL);
+  EXPECT(mdgl_gspmm_mul_sum_dot_any(ids, ids, ids, x, x, x, x, x, 5, 12, 4, 12, 2, ls, rs, nullptr,
+                                    nullptr, 0, 0, nullptr, nullptr, 0, nullptr, 0,
+                                    MDGL_ANY_ALIGNMENT, MDGL_FLOAT32, nullptr) == MDGL_ENOTSUP);
+}
+
 static void sizes_and_geometry() {
   for (int64_t n : {0, 1, 4095, 4096, 4097, 1 << 20}) {
     EXPECT(mdgl_segment_offsets_workspace_bytes(n) >= 0);
@@ -173,6 +231,7 @@ static void other_entry_points() {
 int main() {
   gsddmm_shapes();
   gspmm_arguments();
+  newer_entry_points();
   sizes_and_geometry();
   other_entry_points();
   if (failures) {

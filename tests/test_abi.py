@@ -255,6 +255,126 @@ def test_backward_helper_arguments(lib):
     assert rc in (-1, -3)
 
 
+def test_layout_query_with_any_alignment(lib):
+    """mdgl_gspmm_layout's lanes per row, by which a caller counts slabs: odd
+    widths and heads end with a lane of their own, and rows of few lanes take as
+    many as the ROW_LANES flags say at least."""
+    import numpy as np
+    from mojodgl import _lib
+
+    buf = np.zeros(64, dtype=np.float64)
+    base = (buf.ctypes.data + 127) // 128 * 128
+    mul, cl, any_ = _lib.BINARY_OPS["mul"], _lib.OP_COPY_LHS, _lib.ANY_ALIGNMENT
+
+    def layout(op, dl, dr, dout, lshape=None, rshape=None, flags=any_, dt=0, at=base):
+        got = [ctypes.c_int64(-1) for _ in range(3)]
+        nd = 0 if lshape is None else len(lshape)
+        ls = None if lshape is None else (ctypes.c_int64 * nd)(*lshape)
+        rs = None if rshape is None else (ctypes.c_int64 * nd)(*rshape)
+        rc = lib.mdgl_gspmm_layout(op, dl, dr, dout, nd, ls, rs, at, at, flags, dt,
+                                   *map(ctypes.byref, got))
+        assert rc == 0, err(lib)
+        return tuple(x.value for x in got)
+
+    assert layout(cl, 47, 47, 47) == (4, 16, 12)
+    assert layout(cl, 47, 47, 47, at=base + 4) == (4, 16, 12)
+    assert layout(mul, 200, 8, 200, (8, 25), (8, 1)) == (4, 64, 56)      # 7 lanes a head
+    assert layout(mul, 12, 4, 12, (4, 3), (4, 1)) == (2, 16, 8)
+    assert layout(cl, 602, 602, 602) == (4, 64, 151)
+    assert layout(cl, 602, 602, 602, flags=any_ | _lib.NARROW_SLABS) == (4, 32, 151)
+    assert layout(cl, 3, 3, 3, dt=1) == (2, 16, 2)
+    two, four = any_ | _lib.ROW_LANES_2, any_ | _lib.ROW_LANES_4
+    assert [layout(cl, d, d, d, flags=two)[1] for d in (1, 8, 9, 20, 33, 65)] == [2, 2, 4, 8, 16, 32]
+    assert [layout(cl, d, d, d, flags=four)[1] for d in (1, 8, 17, 33, 64, 300)] == [4, 4, 8, 16, 16,
+                                                                                  64]
+    assert lib.mdgl_gspmm_layout(_lib.BINARY_OPS["dot"], 4, 4, 4, 0, None, None, base, base, 0, 0,
+                                 ctypes.byref(ctypes.c_int64()), None, None) == -1
+    assert lib.mdgl_gspmm_layout(cl, 4, 4, 4, 0, None, None, base, base, 0, 0, None, None, None) == -1
+
+
+def test_graph_and_order_helper_arguments(lib):
+    assert lib.mdgl_coo_ingest(1, 1, 1, 1, -1, 1, None) == -1
+    rc = lib.mdgl_coo_ingest(1, 1, 1, 1, 5, None, None)
+    assert rc == -1 and "null" in err(lib)
+    for null in range(4):
+        at = [None if i == null else 1 for i in range(4)]
+        assert lib.mdgl_coo_ingest(*at, 5, 1, None) == -1 and "null" in err(lib)
+    assert lib.mdgl_permute_values(1, 1, 1, 1, 1, 1, 5, 9, None) == -1
+    assert lib.mdgl_permute_values(1, 1, 1, 1, 1, 1, -1, 0, None) == -1
+    assert lib.mdgl_permute_values(1, 1, 1, 1, 1, 1, 1 << 31, 0, None) == -1
+    for null in range(6):
+        at = [None if i == null else 1 for i in range(6)]
+        assert lib.mdgl_permute_values(*at, 5, 0, None) == -1 and "null" in err(lib)
+    assert lib.mdgl_permute_values(None, None, None, None, None, None, 0, 0, None) == 0
+
+
+def test_row_dot_and_selected_sum_arguments(lib):
+    from mojodgl import _lib
+
+    any_ = _lib.ANY_ALIGNMENT
+
+    def row_dot(dot=1, lhs=1, rowop=1, rows=10, d=64, groups=1, chunks=(None, None, 0, 0),
+                flags=any_, dt=0):
+        return lib.mdgl_gspmm_row_dot(1, 1, lhs, rowop, dot, rows, d, groups, *chunks, flags, dt,
+                                      None)
+
+    assert row_dot(rows=0) == 0                              # no rows: nothing launched
+    assert row_dot(dot=None) == -1 and "null" in err(lib)
+    assert row_dot(rowop=None) == -1 and "null" in err(lib)
+    assert row_dot(lhs=None) == -1 and "null" in err(lib)
+    assert row_dot(flags=0) == -1 and "flags" in err(lib)
+    assert row_dot(dt=3) == -1 and "dtype" in err(lib)
+    assert row_dot(rows=-1) == -1 and row_dot(rows=1 << 31) == -1
+    assert row_dot(d=64, groups=3) == -1 and "multiple" in err(lib)
+    assert row_dot(chunks=(None, None, 3, 8)) == -1 and "schedule" in err(lib)
+    # a run under one 16-byte lane, or over 64 of them
+    assert row_dot(d=3) == -3 and row_dot(d=257) == -3
+    assert row_dot(d=1, dt=1) == -3 and row_dot(d=129, dt=1) == -3
+    assert row_dot(d=12, groups=4) == -3
+
+    def selected(sel=1, eid=1, lhs=1, dst=1, rows=10, d=4, chunks=(None, None, 0, 0, None, None, 0),
+                 ws=(None, 0), flags=any_, dt=0):
+        return lib.mdgl_gspmm_selected_sum(1, 1, eid, lhs, sel, dst, rows, d, *chunks, *ws, flags,
+                                           dt, None)
+
+    assert selected(rows=0) == 0 and selected(d=0) == 0
+    assert selected(sel=None) == -1 and "selection" in err(lib)
+    assert selected(eid=None) == -1 and "eid" in err(lib)
+    assert selected(lhs=None) == -1 and selected(dst=None) == -1
+    assert selected(flags=any_ | _lib.RHS_CSR_ORDER) == -1 and "flags" in err(lib)
+    assert selected(dt=2) == -1 and selected(rows=-1) == -1 and selected(d=-1) == -1
+    assert selected(chunks=(1, 1, 3, 8, 1, 1, 1)) == -2 and "workspace" in err(lib)
+    assert selected(chunks=(1, 1, 3, 8, 1, 1, 1), ws=(4096 + 8, 1 << 20)) == -1
+
+
+def test_fused_dot_arguments(lib):
+    from mojodgl import _lib
+
+    ls, rs = (ctypes.c_int64 * 2)(2, 6), (ctypes.c_int64 * 2)(2, 1)
+
+    def fused(rowop=16, dot=16, dl=12, dr=2, dout=12, lshape=ls, rshape=rs,
+              flags=_lib.ANY_ALIGNMENT, dt=0, rows=10, lhs=16):
+        return lib.mdgl_gspmm_mul_sum_dot_any(16, 16, 16, lhs, 16, rowop, 16, dot, rows, dl, dr, dout,
+                                              2, lshape, rshape, None, None, 0, 0, None, None, 0,
+                                              None, 0, flags, dt, None)
+
+    assert fused(rows=0) == 0
+    assert fused(dot=None) == -1 and "dot" in err(lib)
+    assert fused(rowop=None) == -1 and "row operand" in err(lib)
+    assert fused(lhs=None) == -1 and "null" in err(lib)
+    assert fused(dt=7) == -1
+    # without ANY_ALIGNMENT the runs are whole aligned lanes
+    assert fused(flags=0) == -3
+    # heads of 3 columns are under a 16-byte lane of float32; of 300 over 64 of them
+    short = (ctypes.c_int64 * 2)(4, 3), (ctypes.c_int64 * 2)(4, 1)
+    assert fused(dl=12, dr=4, lshape=short[0], rshape=short[1]) == -3
+    wide = (ctypes.c_int64 * 2)(2, 300), (ctypes.c_int64 * 2)(2, 1)
+    assert fused(dl=600, dr=2, dout=600, lshape=wide[0], rshape=wide[1]) == -3
+    # an edge operand that is not one value per run
+    flat = (ctypes.c_int64 * 2)(1, 6)
+    assert fused(dl=12, dr=6, lshape=ls, rshape=flat) == -3
+
+
 def test_workspace_sizes(lib):
     assert lib.mdgl_gspmm_workspace_bytes(0, 64, 0, 0) == 0
     assert lib.mdgl_gspmm_workspace_bytes(10, 64, 0, 0) >= 10 * 64 * 4
