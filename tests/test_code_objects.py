@@ -79,12 +79,22 @@ def test_edge_rows_stream_past_the_caches(kernels, pattern):
             assert (hinted >= 8) if hints else (rows and hinted == 0), name
 
 
+def _notes(kernel):
+    """The kernel's entry in its code object's metadata."""
+    notes = _run(LLVM + "/llvm-readelf", "--notes", kernel[1])
+    return next(e for e in notes.split("- .agpr_count")
+                if re.search(r"\.name: +" + re.escape(kernel[0]) + r"\s", e))
+
+
+def test_dots_of_whole_vectors_keep_eight_wavefronts(kernels):
+    """64 registers at most: eight wavefronts per SIMD wait for their rows."""
+    (kernel,) = _named(kernels, r"gsddmm_dot_kernel<float, 4, 0>").values()
+    assert int(re.search(r"\.vgpr_count: +(\d+)", _notes(kernel)).group(1)) <= 64
+
+
 @pytest.mark.parametrize("pattern", [r"grouped_tn_(tile_)?kernel<", r"grouped_gemm_any_kernel<"])
 def test_grouped_products_keep_their_registers(kernels, pattern):
     """No instance spills: three steps of a 64 x 64 tile of doubles did, two
     groups of four rows each, and one column block at five wavefronts per SIMD."""
-    for name, (mangled, path) in _named(kernels, pattern).items():
-        notes = _run(LLVM + "/llvm-readelf", "--notes", path)
-        entry = next(e for e in notes.split("- .agpr_count")
-                     if re.search(r"\.name: +" + re.escape(mangled) + r"\s", e))
-        assert re.search(r"\.private_segment_fixed_size: 0\b", entry), name
+    for name, kernel in _named(kernels, pattern).items():
+        assert re.search(r"\.private_segment_fixed_size: 0\b", _notes(kernel)), name
