@@ -307,6 +307,11 @@ class _DeviceCSR:
         """int64 row pointers on the host."""
         return self._raw.host_indptr()
 
+    @property
+    def longest(self):
+        """Slots of the longest row."""
+        return self._raw.longest
+
     def chunks_for(self, chunk_len):
         """The heavy-row schedule for another chunk length (cached)."""
         if int(chunk_len) == self.chunks.chunk_len:

@@ -184,10 +184,13 @@ def gsddmm(g, op, lhs_data, rhs_data, lhs_target="u", rhs_target="v"):
     lhs = _lib.on_device(L, dtype) if L is not None else None
     rhs = _lib.on_device(R, dtype) if R is not None else None
     if op == "dot" and num_edges >= DOT_SLOT_MIN_EDGES and L.shape[1:] == R.shape[1:] \
-            and DOT_SLOT_MIN_ROW * dout <= dtype.itemsize * dl <= DOT_SLOT_MAX_ROW * dout \
-            and {lhs_target, rhs_target} == {"u", "v"}:
+            and {lhs_target, rhs_target} == {"u", "v"} \
+            and _slot_row(dtype.itemsize * dl // dout, num_edges, num_nodes):
         try:
             csr = g._dot_csr()
+            if csr is not None and dtype.itemsize * dl <= DOT_SLOT_MIN_ROW * dout \
+                    and csr.longest * num_nodes > DOT_SLOT_EVEN * num_edges:
+                csr = None
             out = None if csr is None else _slot_dot(
                 csr, *((lhs, rhs) if lhs_target == "u" else (rhs, lhs)), num_edges, num_nodes, dl,
                 dout, tuple(fshape), dtype)
@@ -210,24 +213,43 @@ def gsddmm(g, op, lhs_data, rhs_data, lhs_target="u", rhs_target="v"):
 
 
 # an edge-wise dot between the endpoints runs in CSR slot order from this many
-# edges on, when a dot's rows have this many bytes or more: a destination's row
+# edges on, when a dot's rows have more than this many bytes: a destination's row
 # then stays in registers, one gathered row per edge less, for the results'
-# move into edge-id order (128 columns, 20M edges: 3,187 us edge by edge, 1,484
+# move into edge-id order (128 columns, 20M edges: 3,119 us edge by edge, 1,484
 # slot by slot and 107 for the planned move, 370 until that is planned
 # (_ValueOrder); 2,658 us with the destinations' rows read again from cache for
 # every slot). The most is what 64 lanes of 16 bytes hold: wider rows go edge by
-# edge, which is decided before the in-CSR would be built for them
+# edge, which is decided before the in-CSR would be built for them.
+# Rows of a single 128-byte line gain on graphs of many edges a row and even
+# degrees only. us edge by edge and slot by slot, rows of 128 and of 256 bytes,
+# random destinations: 2 edges a row 365 565, 713 663; 8 a row 599 620, 1,322
+# 792; 16 a row 590 453, 1,141 671; power law: 4 a row 264 500, 555 590; 20 a row
+# 163 214, 330 286; 24 a row (60M edges) 2,002 2,316, 4,278 3,249
 DOT_SLOT_MIN_EDGES = 1 << 20
 DOT_SLOT_MIN_ROW = 128
 DOT_SLOT_MAX_ROW = 1024
+DOT_SLOT_MEAN = 16  # edges a row on average, for rows of DOT_SLOT_MIN_ROW bytes
+DOT_SLOT_EVEN = 4   # times that average: the longest row, for the same
+
+
+def _slot_row(row, num_edges, num_nodes):
+    """Whether dots over rows of `row` bytes may run in slot order."""
+    return DOT_SLOT_MIN_ROW < row <= DOT_SLOT_MAX_ROW or (
+        row == DOT_SLOT_MIN_ROW and num_edges >= DOT_SLOT_MEAN * num_nodes)
 
 
 def _slot_dot(csr, x, y, num_edges, num_nodes, d, dout, fshape, dtype):
     """The dot of every edge between its source's row of `x` and its
     destination's of `y` (mdgl_gspmm_row_dot: the same sums, and so the same
-    bits, as edge by edge) in edge-id order."""
+    bits, as edge by edge) in edge-id order. Rows are split as short as the
+    backward passes' (a slot's dot is its own: nothing to fold), so that the rows
+    of a wavefront end together (20 edges a row, power law, 64 columns: 366 us
+    with 512 slots a unit, 286 with 64)."""
     lib, code, st = _lib.lib(), _lib.dtype_code(dtype), _lib.stream()
-    tdt, gdev, sched = _lib.torch_dtype(dtype), _lib.device(), csr.chunks
+    tdt, gdev = _lib.torch_dtype(dtype), _lib.device()
+    sched = csr.chunks
+    if _autograd.NARROW_SPLIT < sched.chunk_len:
+        sched = csr.chunks_for(_autograd.NARROW_SPLIT)
     tmp = torch.empty((num_edges, dout), dtype=tdt, device=gdev)
     _lib.check(lib.mdgl_gspmm_row_dot(
         csr.indptr.data_ptr(), csr.indices.data_ptr(), x.data_ptr(), y.data_ptr(), tmp.data_ptr(),

@@ -161,3 +161,32 @@ def test_dots_too_wide_for_the_slot_kernel_build_no_csr(dtype, d, slots, monkeyp
         got = ops.u_dot_v(g, x, y)
         assert torch.equal(got, (x[u] * y[v]).sum(-1, keepdim=True))
     assert (g._current_csr("in") is not None) == slots
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,d", [(torch.float32, 32), (torch.float64, 16)])
+def test_dots_of_one_line_go_slot_by_slot_on_even_graphs_only(dtype, d, monkeypatch):
+    """Rows of 128 bytes: slot by slot from 16 edges a row on when no row has more
+    than four times that; one column more takes the slot order in any case. The
+    results are the same bits either way."""
+    from mojodgl.ops import sddmm
+
+    monkeypatch.setattr(sddmm, "DOT_SLOT_MIN_EDGES", 1)
+    calls = []
+    real = sddmm._slot_dot
+    monkeypatch.setattr(sddmm, "_slot_dot", lambda *a: calls.append(1) or real(*a))
+    rng = np.random.default_rng(d)
+    n = 60
+    even = np.repeat(np.arange(n), 20)
+    hub = np.concatenate([even, np.full(400, 7)])
+    few = np.repeat(np.arange(n), 15)
+    for v, slots in ((even, True), (hub, False), (few, False)):
+        u = rng.integers(0, n, v.size)
+        for width in (d, d + 1):
+            g = dgl.graph((u, v), num_nodes=n)
+            x, y = (torch.randn(n, width, device="cuda", dtype=dtype) for _ in range(2))
+            want = ops.u_dot_v(g, x, y)  # the first dot of a graph: edge by edge
+            del calls[:]
+            for _ in range(2):
+                assert torch.equal(ops.u_dot_v(g, x, y), want)
+            assert bool(calls) == (slots or width > d)
