@@ -388,7 +388,10 @@ __device__ __forceinline__ void gspmm_body(const GspmmArgs<T>& a, bool chunk, in
         auto ro_of = [&](auto iu) MDGL_INLINE { return row_bcast<F + decltype(iu)::value>(my_ro); };
         auto w_of = [&](auto iu) MDGL_INLINE { return row_bcast<F + decltype(iu)::value>(my_w); };
         auto e_of = [&](auto iu) MDGL_INLINE { return row_bcast<F + decltype(iu)::value>(cur_e); };
-        if (rem >= U)
+        // a divide is a dozen instructions: one body for all rows of the wavefront
+        // (elsewhere the rows with a whole batch save its tests)
+        const bool whole = OP == OP_DIV ? __builtin_amdgcn_ballot_w64(rem < U) == 0 : rem >= U;
+        if (whole)
           batch(std::true_type{}, start + base + F, U, lo_of, ro_of, w_of, e_of);
         else
           batch(std::false_type{}, start + base + F, rem, lo_of, ro_of, w_of, e_of);

@@ -34,7 +34,7 @@ _OPS = frozenset(BINARY_OPS) | {"copy_lhs", "copy_rhs"}
 _LANES = {}
 
 
-def _row_lanes(num_edges, num_rows):
+def _row_lanes(num_edges, num_rows, divides=False):
     """The least lanes a row of a gspmm takes, as a flag, by the edges a row has
     on average (the kernel's description has the layouts). With few, rows of few
     columns packed closely keep more rows in flight, and most end within the
@@ -50,10 +50,14 @@ def _row_lanes(num_edges, num_rows):
       16, random           136 289 325    108 306 249    113 311 253
       20, power law         80 121 224     84 139 196    133 190 287
     16 columns likewise (4, random: 466 589 1,277 with 16 lanes, 341 414 715
-    with 4; 16, random: 293 432 660 and 308 388 630)."""
+    with 4; 16, random: 293 432 660 and 308 388 630). A quotient costs more
+    than its bytes, also in lanes past the row: rows of more than one column
+    take only the lanes they need at any mean (u_div_e_sum of 16 columns, 20
+    edges a row, power law: 620 us with 16 lanes, 452; 24 a row, 8 columns:
+    5,396 and 3,280)."""
     if num_edges < 6 * num_rows:
         return _lib.ROW_LANES_2
-    return _lib.ROW_LANES_4 if num_edges < 12 * num_rows else 0
+    return _lib.ROW_LANES_4 if num_edges < 12 * num_rows or divides else 0
 
 
 
@@ -273,7 +277,7 @@ def _run(g, op, reduce_op, lhs_data, rhs_data, replace_inf=False, want_arg=False
         rhs = _lib.on_device(R, dtype) if R is not None else None
         csr = g._device_csr(kind)
         flags = _lib.ANY_ALIGNMENT | (_lib.REPLACE_INF if replace_inf else 0) \
-            | _row_lanes(num_edges, num_dst)
+            | _row_lanes(num_edges, num_dst, code == BINARY_OPS["div"] and dout > 1)
         replay = key is not None
         if rows is not None:
             # the layout choices pay over whole graphs, not a few rows

@@ -265,7 +265,7 @@ def test_rows_of_few_lanes(dtype, d, lanes, monkeypatch):
         return None if a is None else torch.from_numpy(a).cuda()
 
     with monkeypatch.context() as m:
-        m.setattr(ops.spmm, "_row_lanes", lambda num_edges, num_rows: lanes)
+        m.setattr(ops.spmm, "_row_lanes", lambda *counts: lanes)
         m.setattr(heterograph, "CHUNK_LEN", 1 << 20)
         g = dgl.graph((u, v), num_nodes=n)
         for op, a, b in operands:
@@ -285,7 +285,7 @@ def test_rows_of_few_lanes(dtype, d, lanes, monkeypatch):
 
     def backward(fewest):
         with monkeypatch.context() as m:
-            m.setattr(ops.spmm, "_row_lanes", lambda num_edges, num_rows: fewest)
+            m.setattr(ops.spmm, "_row_lanes", lambda *counts: fewest)
             g = dgl.graph((u, v), num_nodes=n)
             out = []
             for op, a, b in operands:
