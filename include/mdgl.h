@@ -66,8 +66,9 @@ extern "C" {
 #define MDGL_ANY_ALIGNMENT 64
 /* mdgl_gspmm, _selected_sum, _mul_sum_dot_any: a row of fewer than 16 lanes takes
  * the power of two covering them, at least 2 (4), instead of 16 -- for graphs of
- * few edges a row (about 6, 12 on average). Results are the same bit for bit; only
- * the lane layout changes. At most one of the two. */
+ * few edges a row (under about 6, 12 on average), and _4 for quotients of several
+ * columns at any number of them (lanes past the row would divide too). Results
+ * are the same bit for bit; only the lane layout changes. At most one of the two. */
 #define MDGL_ROW_LANES_2 128
 #define MDGL_ROW_LANES_4 256
 /* mdgl_segment_reduce(_arg): the caller knows that no segment has more than
@@ -187,12 +188,12 @@ int mdgl_gspmm_rows(const int32_t* indptr, const int32_t* indices, const int32_t
                     int32_t* arg_e, const int32_t* rows, int64_t num_rows, int flags, int dtype,
                     void* stream);
 
-/* The lane width (values per lane: 1, 2 or 4 in float32, 1 or 2 in
- * float64) and, when `group` is not null, the lanes per row slab (a power
- * of two up to 64) that mdgl_gspmm picks for these operands, shapes,
- * alignments and flags, so a caller can tell how many rows share a
- * wavefront (64 / group) and how many column slabs a row is cut into
- * (ceil(ceil(dout / vec) / group)). No counterpart in the
+/* The lane width (values per lane: 1, 2 or 4 in either type) and, when `group`
+ * is not null, the lanes per row slab (a power of two, 2 to 64) that mdgl_gspmm
+ * picks for these operands, shapes, alignments and flags, so a caller can tell
+ * how many rows share a wavefront (64 / group). A row takes ceil(dout / vec) lanes without
+ * MDGL_ANY_ALIGNMENT; with it each run of columns has lanes of its own, and
+ * mdgl_gspmm_layout gives their number. No counterpart in the
  * reference (its kernel is a CPU loop, src/ported.mojo:352-423); it is the
  * planning query behind the host's scheduling choices for a gspmm call. */
 int mdgl_gspmm_lanes(int op, int64_t dl, int64_t dr, int64_t dout, int nd,

@@ -16,6 +16,8 @@
 //  * grouped_gemm_f64_kernel: float64, K a multiple of 16 up to 128, in two,
 //    four or eight blocks of 16 columns;
 //  * grouped_gemm_kernel: what is left.
+// Gradient of b: grouped_tn_kernel on register tiles, grouped_tn_tile_kernel on
+// 128 x 128 tiles through LDS for float32 widths that fill them, tn_fold_kernel.
 //
 // grouped_gemm_kernel:
 //
@@ -646,7 +648,7 @@ __global__ __launch_bounds__(SB_THREADS, 1) void grouped_gemm_split_kernel(
 // Work mapping. A workgroup of NW wavefronts holds the group's b block (NB
 // blocks of 32 columns x KMAX) in LDS as three bf16 planes and walks a
 // contiguous range of 32 NW-row tiles; wavefront w owns 32 rows of a tile and
-// all NB blocks. The block is small (14 to 104 KB), so up to eight workgroups
+// all NB blocks. The block is small (14 to 104 KB), so up to four workgroups
 // share a CU and their wavefronts cover each other's waits: the loads of a row
 // run four 16-deep chunks ahead (two with one narrow block), without the split
 // kernel's exact wait counts. Two chunks requested at a time instead of one:
@@ -1902,7 +1904,7 @@ constexpr int64_t TN_CHUNKS = 2048;                // chunks, about, when rows a
 constexpr int64_t TN_PART_BYTES = 256ll << 20;     // partials kept below this when rows allow
 
 // Rows per chunk: TN_CH, doubled to TN_CH_MOST while there are more than
-// TN_CHUNKS chunks (at most n / ch + R of them; eight workgroups a CU) and
+// TN_CHUNKS chunks (at most n / ch + R of them; eight workgroups for each CU) and
 // further while their partials pass TN_PART_BYTES, and at most n (n < 2**31).
 inline int64_t tn_chunk_rows(int64_t n, int64_t D1, int64_t D2, int64_t R, int64_t es) {
   int64_t ch = TN_CH;

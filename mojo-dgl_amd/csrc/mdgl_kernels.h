@@ -38,7 +38,7 @@ struct GspmmParams {
   int vec;      // elements per lane (1 or 16 / sizeof(T))
   int64_t run_len;  // columns per run of consecutive operand columns (>= vec)
   int lpg;      // lanes per run
-  int group;    // lanes per row slab (16, 32 or 64)
+  int group;    // lanes per row slab (a power of two, 2 to 64)
   int64_t num_chunks;
   const int32_t* chunk_row;
   const int32_t* chunk_start;
